@@ -86,8 +86,8 @@ typedef struct lisa_stats {
   int32_t num_nodes;  /* internal BVH nodes (64 B each) */
   int32_t num_emitters; /* triangles whose material emits (the NEE light BVH) */
   uint64_t device_bytes; /* device memory held by the context */
-  int32_t wide_tree;  /* 1: the scene's tree also has its 4-wide form, which the uncounted path
-                         kernels walk (lisa_set_wide_threshold) */
+  int32_t wide_tree;  /* 1: the scene's Morton tree also has its 4-wide form, which
+                         lisa_trace_rays walks (lisa_set_wide_threshold) */
   int32_t reserved;
 } lisa_stats;
 
@@ -115,7 +115,8 @@ lisa_status lisa_set_scene(lisa_ctx* ctx, const float* verts, const float* norma
  * in the build's Morton order and both LBVHs are refit bottom-up, keeping
  * topology and Morton codes (animated / re-posed geometry; cheaper than a
  * rebuild, box quality degrades with large motion); a 4-wide form of the
- * tree is rebuilt from the refitted one.  No counterpart in the
+ * tree is rebuilt from the refitted one, and the tree that renders walk is
+ * clustered anew from the moved triangles.  No counterpart in the
  * reference, whose GAS is built once (optix_wrapper.cc:104-106). */
 lisa_status lisa_update_vertices(lisa_ctx* ctx, const float* verts, const float* normals);
 
@@ -174,13 +175,15 @@ lisa_status lisa_synchronize(lisa_ctx* ctx);
  * (render.cc:146-147). */
 lisa_status lisa_get_stats(const lisa_ctx* ctx, lisa_stats* out);
 /* Scenes set from now on with at least min_triangles triangles (default
- * 2^20) also get the 4-wide form of their tree (128 bytes per inner node: each
- * node's children, inner children replaced by their own two), and the path
- * kernels that count nothing walk it: fewer, wider visits, which pay where
- * the tree streams from HBM.  The hits are the same (closest hit, equal t to
- * the lower triangle id); node-visit counters (LISA_FLAG_COUNT) stay those of
- * the binary tree.  0 gives every scene the wide form.  No counterpart in
- * the reference (OptiX chooses its acceleration structure). */
+ * 2^20) also get the 4-wide form of their Morton tree (128 bytes per inner
+ * node: each node's children, inner children replaced by their own two), and
+ * lisa_trace_rays takes its hits from it: fewer, wider visits, which pay where
+ * the tree streams from HBM.  (The path kernels that count nothing walk an
+ * agglomerated 4-wide tree that every scene has.)  The hits are the same
+ * (closest hit, equal t to the lower triangle id); node-visit counters
+ * (LISA_FLAG_COUNT) stay those of the binary tree.  0 gives every scene the
+ * wide form.  No counterpart in the reference (OptiX chooses its acceleration
+ * structure). */
 lisa_status lisa_set_wide_threshold(lisa_ctx* ctx, int64_t min_triangles);
 /* Counters of the last call made with LISA_FLAG_COUNT (or lisa_trace_rays). */
 lisa_status lisa_get_counters(const lisa_ctx* ctx, uint64_t* counters /* LISA_NCOUNTERS */);

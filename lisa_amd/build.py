@@ -37,8 +37,8 @@ def _run(cmd):
 
 def build(verbose_resources=False, defines=(), out_dir=OUT, cli=True):
     """Compile liblisa.so (and the CLI) into out_dir; `defines` are extra
-    -D tuning macros (LISA_STACK_LDS, LISA_PATH_MIN_BLOCKS, LISA_WIDE_WAVES, LISA_MODE_WAVES,
-    LISA_EMIT_WAVES, LISA_TILE_WAVES; LISA_PATH_BLOCK must stay 64: a workgroup is one wave)."""
+    -D tuning macros (LISA_STACK_LDS, LISA_WALK_STACK, LISA_PATH_MIN_BLOCKS,
+    LISA_MODE_WAVES, LISA_EMIT_WAVES, LISA_TILE_WAVES; LISA_PATH_BLOCK must stay 64: a workgroup is one wave)."""
     os.makedirs(out_dir, exist_ok=True)
     dev_o = os.path.join(out_dir, "lisa_device.o")
     cache_o = os.path.join(out_dir, "lisa_cache.o")
@@ -63,14 +63,15 @@ def build(verbose_resources=False, defines=(), out_dir=OUT, cli=True):
 
 
 # Variant of the library with a 2-entry LDS traversal stack: every deeper
-# entry goes to the per-lane private overflow array, so a parity test run
-# against it exercises that path (the default 20-entry stack never
+# entry goes to the per-lane private overflow array, and a walk of the
+# agglomerated tree past 9 entries is left to the Morton tree, so a parity test
+# run against it exercises both paths (the default 20-entry stack never
 # overflows on the benchmark scenes).
 SMALL_STACK = os.path.join(OUT, "stack2")
 
 
 def build_small_stack():
-    return build(defines=("LISA_STACK_LDS=2",), out_dir=SMALL_STACK, cli=False)
+    return build(defines=("LISA_STACK_LDS=2", "LISA_WALK_STACK=9"), out_dir=SMALL_STACK, cli=False)
 
 
 if __name__ == "__main__":

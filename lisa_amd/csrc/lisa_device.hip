@@ -8,7 +8,9 @@
 //                           (child boxes live in the parent; ref bit 31 = leaf,
 //                           low bits = sorted triangle / node index)
 //   wide   float4[8 * nI]   scenes of >= 2^20 triangles: the 4-wide form (k_wide),
-//                           one 128-byte line per internal node
+//                           one 128-byte line per internal node (lisa_trace_rays)
+//   walk   float4[8 * cap]  the agglomerated 4-wide tree that the path kernels walk
+//                           (k_agg, k_walk_nodes), cap ~ 1.07 T
 //   tris   float4[3 * T]    48 bytes per triangle in Morton order:
 //                           v0.xyz|prim id, v1.xyz|material id, v2.xyz|0
 //   nrm    float4[3 * T]    vertex normals in the same order (shading gather)
@@ -55,27 +57,22 @@ constexpr int kNeeTries = 30;   // shader.cu:199
 #ifndef LISA_PATH_BLOCK
 #define LISA_PATH_BLOCK 64
 #endif
-// Waves per SIMD the plain path kernel k_path is compiled for: 6 with a
-// 20-entry LDS stack (24 LDS words per lane with the lane state: 6 KB per
-// 64-lane workgroup) at 80 VGPRs and no spills.  The cache-mode paths run at
-// 5, except the tiled prefix-emission mode (6: its spills sit around the
-// walks and the island's frames ran 2 % faster than at 5; its persistent
-// form would spill far more at 6 and stays at 5), the counting and recording
-// builds at 4, and the batched forms keep the registers they need.
+// Waves per SIMD the path kernels are compiled for: 5 (96 VGPRs).  The walk of
+// the 4-wide tree holds a node's 28 words at once; at 6 waves (80 VGPRs) k_path
+// spills 29 registers around it and C2 (32 spp) takes 55.4 ms against 44.5, at 4
+// (101 VGPRs, no spill) 49.2.  The counting and recording builds run at 4, and
+// the batched lane-queue form keeps the registers it needs.
 #ifndef LISA_PATH_MIN_BLOCKS
-#define LISA_PATH_MIN_BLOCKS 6
-#endif
-#ifndef LISA_WIDE_WAVES
-#define LISA_WIDE_WAVES 6  // k_path over the 4-wide tree (5 measured 8 % slower on C3)
+#define LISA_PATH_MIN_BLOCKS 5
 #endif
 #ifndef LISA_MODE_WAVES
 #define LISA_MODE_WAVES 5  // the cache-mode path kernels
 #endif
 #ifndef LISA_EMIT_WAVES
-#define LISA_EMIT_WAVES 6  // the query kernel with the prefix-emission light samples
+#define LISA_EMIT_WAVES 5  // the query kernel with the prefix-emission light samples
 #endif
 #ifndef LISA_TILE_WAVES
-#define LISA_TILE_WAVES 6  // the batched wave-tile form
+#define LISA_TILE_WAVES 5  // the batched wave-tile form
 #endif
 // The BSDF of opaque materials, chosen at compile time as the reference
 // chooses it with an #include (shader.cu:4): a type with
@@ -86,6 +83,12 @@ constexpr int kNeeTries = 30;   // shader.cu:199
 #endif
 constexpr int kStackLds = LISA_STACK_LDS;
 constexpr int kStackMax = 64;
+// Entries closest_walk may hold (at most kStackMax) before it leaves a query
+// to closest().
+#ifndef LISA_WALK_STACK
+#define LISA_WALK_STACK 64
+#endif
+constexpr int kWalkStack = LISA_WALK_STACK;
 // LDS words per lane of a path kernel: the traversal stack, then the pixel's
 // running sum of sample radiance (3 floats, touched once per sample) and the
 // NEE light material (written when a NEE ray finds a light) -- in LDS so
@@ -102,6 +105,7 @@ constexpr int kTileW = kPathBlock >= 128 ? 16 : 8;
 constexpr int kTileH = kPathBlock / kTileW;
 constexpr int kRayBlock = 256;
 static_assert(kStackLds >= 1 && kStackLds <= kStackMax, "LDS stack depth");
+static_assert(kWalkStack >= 3 && kWalkStack <= kStackMax, "walk stack depth");
 static_assert(kPathBlock == 64 || kPathBlock == 128 || kPathBlock == 256, "path block size");
 
 struct DevMat {
@@ -116,6 +120,8 @@ struct BvhView {
   const float4* __restrict__ tris;
   int32_t T;
   const float4* __restrict__ wide;  // the 4-wide form of `nodes` (null: none)
+  const char* __restrict__ walk;    // the walk tree (k_agg, k_walk_nodes; null: none)
+  float span;                       // largest |coordinate| of the boxes (closest_walk's margin)
 };
 
 struct SceneView {
@@ -272,17 +278,17 @@ struct TravCount {
 // resolves equal t to the lower triangle id; the any-hit query answers "is
 // any triangle strictly before (tlim, lim_prim)" and stops at the first.
 // `stk` points at this lane's first LDS stack slot; consecutive entries are
-// kStride words apart, so a wave's 64 lanes hit 64 distinct banks.
+// kStride words apart, so a wave's 64 lanes hit 64 distinct banks.  `spill`:
+// kStackMax - kStackLds private words for the entries past the LDS part.
+// volatile: the compiler keeps the pop's LDS read and private read apart
+// instead of merging them into one generic (flat) load through a selected
+// pointer.  (An empty asm with a memory clobber does the same but makes the
+// batched kernels re-read their scene views, which live in global memory,
+// after every pop.)
 template <bool kCount, int kStride>
 __device__ __forceinline__ int32_t closest(const BvhView& bv, const RayT& r, float tmin,
                                            float tlim, uint32_t lim_prim, bool any, float& t_out,
-                                           uint32_t* stk, TravCount& cnt) {
-  // Entries past the LDS part of the stack.  volatile: the compiler keeps
-  // the pop's LDS read and private read apart instead of merging them into
-  // one generic (flat) load through a selected pointer.  (An empty asm with
-  // a memory clobber does the same but makes the batched kernels re-read
-  // their scene views, which live in global memory, after every pop.)
-  volatile uint32_t spill[kStackMax - kStackLds];
+                                           uint32_t* stk, volatile uint32_t* spill, TravCount& cnt) {
   float best_t = tlim;
   float cull_t = tlim * kWiden;
   uint32_t best_prim = lim_prim;
@@ -459,6 +465,159 @@ __device__ __forceinline__ int32_t closest_wide(const BvhView& bv, const RayT& r
   return best_k;
 }
 
+// The same query over the walk tree (k_agg, k_walk_nodes): the scene's
+// triangles under an agglomerated 4-wide tree.  The accepted triangle is
+// closest()'s: the acceptance rule does not depend on the order of the tests,
+// the leaf boxes are the same, and every box test here accepts whatever
+// closest()'s slab test accepts.
+//
+// Box tests: t = l / D - O / D as one fused multiply-add per plane with the
+// near and far planes picked by the sign of D (the node's float4s are loaded
+// in that order).  Its error is below 5u (|O| + span) / |D| (u = 2^-24), so
+// the near planes are moved by e = 2^-20 (|O| + span) / |D| towards the
+// origin and the far planes away from it, which covers that error and the
+// slack of slab()'s own rounding and kRobust (12u of t).  An axis whose
+// arithmetic overflows gives NaN and is left out of the test.  A direction
+// component of zero takes 1 / D = 2^100: a plane on the wrong side of the
+// origin is then at t < -2^60 or > 2^60.
+//
+// An iteration visits an inner node and then tests a triangle if the lane
+// holds one, so the wave runs one copy of the triangle test per iteration
+// whatever its lanes found (the four slots' tests in closest_wide() each ran
+// whenever one lane of the wave needed them).  A stack that would pass
+// kWalkStack entries (never seen on a benchmark scene; the tree's depth is not
+// bounded by the construction) leaves the query to closest() over the Morton
+// tree, as does a scene without a walk tree.
+//
+// Bound by instruction issue of the wave's longest walk.  Visits per ray and
+// per wave of 64 (the longest): Cornell box of 65k triangles 23.4 / 60.5 in
+// the binary Morton tree, 11.4 / 29.7 in its 4-wide form, 4.2 / 17.0 here;
+// icosphere of 328k 21.0 / 63.6, 11.1 / 32.7, 5.4 / 23.2.  k_path at 32 spp,
+// 1024^2: C2 67.5 -> 44.5 ms; icosphere of 1.3M triangles, 1080p, 16 spp:
+// 85.6 -> 53.8 ms (before: its 4-wide Morton walk).
+template <int kStride>
+__device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r, float tmin,
+                                                float tlim, uint32_t lim_prim, bool any, float& t_out,
+                                                uint32_t* stk, volatile uint32_t* spill) {
+  bool done = false;
+  int32_t best_k = -1;
+  if (bv.walk) {
+    const float big = 0x1p100f;
+    const F3 inv = mk(fabsf(r.inv.x) <= big ? r.inv.x : copysignf(big, r.inv.x),
+                      fabsf(r.inv.y) <= big ? r.inv.y : copysignf(big, r.inv.y),
+                      fabsf(r.inv.z) <= big ? r.inv.z : copysignf(big, r.inv.z));
+    const float ux = r.O.x * inv.x, uy = r.O.y * inv.y, uz = r.O.z * inv.z;
+    const float ex = (fabsf(r.O.x) + bv.span) * fabsf(inv.x) * 0x1p-20f;
+    const float ey = (fabsf(r.O.y) + bv.span) * fabsf(inv.y) * 0x1p-20f;
+    const float ez = (fabsf(r.O.z) + bv.span) * fabsf(inv.z) * 0x1p-20f;
+    const F3 on = mk(-ux - ex, -uy - ey, -uz - ez), of = mk(ex - ux, ey - uy, ez - uz);
+    // byte offsets of the near planes in a node: lo at 0, hi at 16
+    const uint32_t sx = inv.x < 0.0f ? 16u : 0u, sy = inv.y < 0.0f ? 16u : 0u, sz = inv.z < 0.0f ? 16u : 0u;
+    const char* __restrict__ base = bv.walk;
+    float best_t = tlim, cull_t = tlim * kWiden;
+    uint32_t best_prim = lim_prim, cur = 0;
+    int sp = 0;
+    done = true;
+    for (;;) {
+      bool pop = false;
+      if (!(cur & kLeaf)) {
+        const uint32_t ox = (cur << 7) | sx, oy = (cur << 7) | sy, oz = (cur << 7) | sz;
+        const float4 nx = *reinterpret_cast<const float4*>(base + ox);
+        const float4 fx = *reinterpret_cast<const float4*>(base + (ox ^ 16u));
+        const float4 ny = *reinterpret_cast<const float4*>(base + oy + 32u);
+        const float4 fy = *reinterpret_cast<const float4*>(base + (oy ^ 16u) + 32u);
+        const float4 nz = *reinterpret_cast<const float4*>(base + oz + 64u);
+        const float4 fz = *reinterpret_cast<const float4*>(base + (oz ^ 16u) + 64u);
+        const uint4 rf = *reinterpret_cast<const uint4*>(base + (cur << 7) + 96u);
+        float key[4];
+        uint32_t ref[4] = {rf.x, rf.y, rf.z, rf.w};
+        auto box = [&](float lx, float ly, float lz, float hx, float hy, float hz) {
+          const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(lx, inv.x, on.x), __builtin_fmaf(ly, inv.y, on.y)),
+                                       __builtin_fmaf(lz, inv.z, on.z)), tmin);
+          const float tf = fminf(fminf(fminf(__builtin_fmaf(hx, inv.x, of.x), __builtin_fmaf(hy, inv.y, of.y)),
+                                       __builtin_fmaf(hz, inv.z, of.z)), cull_t);
+          return tn <= tf ? tn : INFINITY;
+        };
+        key[0] = box(nx.x, ny.x, nz.x, fx.x, fy.x, fz.x);
+        key[1] = box(nx.y, ny.y, nz.y, fx.y, fy.y, fz.y);
+        key[2] = box(nx.z, ny.z, nz.z, fx.z, fy.z, fz.z);
+        key[3] = box(nx.w, ny.w, nz.w, fx.w, fy.w, fz.w);
+        // sorting network on (key, ref): (0,1) (2,3) (0,2) (1,3) (1,2)
+        auto cswap = [&](int i, int j) {
+          const bool sw = key[j] < key[i];
+          const float ki = key[i], kj = key[j];
+          const uint32_t ri = ref[i], rj = ref[j];
+          key[i] = sw ? kj : ki;
+          key[j] = sw ? ki : kj;
+          ref[i] = sw ? rj : ri;
+          ref[j] = sw ? ri : rj;
+        };
+        cswap(0, 1);
+        cswap(2, 3);
+        cswap(0, 2);
+        cswap(1, 3);
+        cswap(1, 2);
+        if (sp <= kStackLds - 3) {
+          // far to near; an entry that is not there is overwritten by the next
+          stk[sp * kStride] = ref[3];
+          sp += key[3] < INFINITY ? 1 : 0;
+          stk[sp * kStride] = ref[2];
+          sp += key[2] < INFINITY ? 1 : 0;
+          stk[sp * kStride] = ref[1];
+          sp += key[1] < INFINITY ? 1 : 0;
+        } else {
+          if (sp > kWalkStack - 3) {
+            done = false;
+            break;
+          }
+#pragma unroll
+          for (int q = 3; q >= 1; --q) {
+            if (key[q] < INFINITY) {
+              if (sp < kStackLds)
+                stk[sp * kStride] = ref[q];
+              else
+                spill[sp - kStackLds] = ref[q];
+              ++sp;
+            }
+          }
+        }
+        cur = ref[0];
+        pop = !(key[0] < INFINITY);
+      }
+      if (!pop && (cur & kLeaf)) {
+        const uint32_t k = cur & ~kLeaf;
+        const float4* tp = bv.tris + 3 * (size_t)k;
+        const float4 t0 = tp[0], t1 = tp[1], t2 = tp[2];
+        const uint32_t prim = __float_as_uint(t0.w);
+        float t;
+        if (watertight(r, xyz(t0), xyz(t1), xyz(t2), t) && t > tmin &&
+            (t < best_t || (t == best_t && prim < best_prim))) {
+          best_t = t;
+          cull_t = t * kWiden;
+          best_prim = prim;
+          best_k = (int32_t)k;
+          if (any) break;
+        }
+        pop = true;
+      }
+      if (pop) {
+        if (sp == 0) break;
+        --sp;
+        if (sp < kStackLds)
+          cur = stk[sp * kStride];
+        else
+          cur = spill[sp - kStackLds];
+      }
+    }
+    t_out = best_t;
+  }
+  if (!done) {
+    TravCount tc;
+    best_k = closest<false, kStride>(bv, r, tmin, tlim, lim_prim, any, t_out, stk, spill, tc);
+  }
+  return best_k;
+}
+
 // ---------------------------------------------------------------------------
 // Ray batch kernel (hit-id parity, lisa_trace_rays).
 // ---------------------------------------------------------------------------
@@ -479,11 +638,15 @@ __global__ __launch_bounds__(kRayBlock) void k_trace_rays(SceneView sc, const fl
   float t = 0.0f;
   if (sc.all.T > 0 && ray_valid(d)) {
     const RayT r = make_ray(o, d);
+    volatile uint32_t spill[kStackMax - kStackLds];
     int32_t k = closest<kCount, kRayBlock>(sc.all, r, tmin, tmax, 0xFFFFFFFFu, false, t,
-                                           stk + threadIdx.x, cnt);
-    // with a 4-wide tree, the hit of its walk (which the path kernels use;
-    // the counts stay the binary walk's)
-    if (sc.all.wide) k = closest_wide<kRayBlock>(sc.all, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x);
+                                           stk + threadIdx.x, spill, cnt);
+    // the hit is the walk tree's (which the path kernels use), or with a
+    // 4-wide form of the Morton tree that one's; the counts are the binary walk's
+    if (!sc.all.wide)
+      k = closest_walk<kRayBlock>(sc.all, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x, spill);
+    else
+      k = closest_wide<kRayBlock>(sc.all, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x);
     if (k >= 0) prim = (int32_t)__float_as_uint(sc.all.tris[3 * (size_t)k].w);
   }
   prim_out[i] = prim;
@@ -602,8 +765,7 @@ struct Job {
 // suffix radiance (final - so far) / throughput of each vertex becomes a
 // training row at the sample's row slots.  Without accum_prev the launch writes its own mean (no
 // running mean over subframes; the subframe then only picks the RNG stream).
-template <bool kRecord, bool kCount, class Src, int kMode = 0, bool kF64 = false, bool kWide = false,
-          class Bsdf = LISA_BSDF>
+template <bool kRecord, bool kCount, class Src, int kMode = 0, bool kF64 = false, class Bsdf = LISA_BSDF>
 __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   Job job;
   if (!src.next(job)) return;
@@ -616,6 +778,15 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
 
   uint64_t c_rad = 0, c_occ = 0, c_rhit = 0, c_inv = 0, c_smp = 0, c_px = 0;
   TravCount tc;
+  volatile uint32_t spill[kStackMax - kStackLds];
+  // A query over one of the scene's trees: the counting builds walk the
+  // Morton tree, whose visits the counters define, the others the walk tree.
+  auto query = [&](const BvhView& bv, const RayT& r, float tlim, uint32_t lim, bool any, float& t) -> int32_t {
+    if constexpr (kCount)
+      return closest<true, kPathBlock>(bv, r, kTmin, tlim, lim, any, t, my_stk, spill, tc);
+    else
+      return closest_walk<kPathBlock>(bv, r, kTmin, tlim, lim, any, t, my_stk, spill);
+  };
 
   // the pixel's sum of sample radiance, in LDS after the lane's stack
   float* const acc = reinterpret_cast<float*>(my_stk + kStackLds * kPathBlock);
@@ -829,7 +1000,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
       float t = 0.0f;
       if (valid && scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
         const RayT r = make_ray(O, D);
-        k = closest<kCount, kPathBlock>(scp->emit, r, kTmin, kTmax, 0xFFFFFFFFu, false, t, my_stk, tc);
+        k = query(scp->emit, r, kTmax, 0xFFFFFFFFu, false, t);
       }
       if (!valid) {  // counts as a ray, misses without traversal
         const int32_t code = hitf ? -1 : -5;
@@ -927,8 +1098,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
       // kMode 3's light sample: is the sampled triangle the closest emitter
       // along the line?  Then its any-hit test (qstage 3), else its bounce.
       float t = 0.0f;
-      const int32_t k = closest<kCount, kPathBlock>(scp->emit, make_ray(O, D), kTmin, kTmax, 0xFFFFFFFFu,
-                                                    false, t, my_stk, tc);
+      const int32_t k = query(scp->emit, make_ray(O, D), kTmax, 0xFFFFFFFFu, false, t);
       if (k == ls_k) {
         const float4 e0 = scp->emit.tris[3 * (size_t)k], e1 = scp->emit.tris[3 * (size_t)k + 1];
         tE = t;
@@ -951,12 +1121,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     if (valid && scp->all.T > 0) {
       const RayT r = make_ray(O, D);
       const bool any = qstage >= 2;
-      if constexpr (kWide && !kCount)
-        k = closest_wide<kPathBlock>(scp->all, r, kTmin, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu,
-                                     any, t, my_stk);
-      else
-        k = closest<kCount, kPathBlock>(scp->all, r, kTmin, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu,
-                                        any, t, my_stk, tc);
+      k = query(scp->all, r, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu, any, t);
     }
 
     if (qstage == 0) {
@@ -1123,21 +1288,21 @@ struct OnePixel {
   }
 };
 
-template <bool kRecord, bool kCount, bool kF64 = false, bool kWide = false>
-__global__ __launch_bounds__(kPathBlock, (kRecord || kCount) ? 4 : (kWide ? LISA_WIDE_WAVES : LISA_PATH_MIN_BLOCKS)) void k_path(SceneView sc, PathArgs p) {
+template <bool kRecord, bool kCount, bool kF64 = false>
+__global__ __launch_bounds__(kPathBlock, (kRecord || kCount) ? 4 : LISA_PATH_MIN_BLOCKS) void k_path(SceneView sc, PathArgs p) {
   __shared__ uint32_t stk[kLaneLds * kPathBlock];
   OnePixel src{sc, p, false};
-  path_lane<kRecord, kCount, OnePixel, 0, kF64, kWide>(src, stk + threadIdx.x);
+  path_lane<kRecord, kCount, OnePixel, 0, kF64>(src, stk + threadIdx.x);
 }
 
 // Path loop in a cache mode (1: cached render of the full image in tiles,
 // 2: training paths on a pixel list).
-template <int kMode, bool kWide = false>
+template <int kMode>
 __global__ __launch_bounds__(kPathBlock, kMode == 3 ? LISA_EMIT_WAVES : LISA_MODE_WAVES) void k_path_mode(
     SceneView sc, PathArgs p) {
   __shared__ uint32_t stk[kLaneLds * kPathBlock];
   OnePixel src{sc, p, false};
-  path_lane<false, false, OnePixel, kMode, false, kWide>(src, stk + threadIdx.x);
+  path_lane<false, false, OnePixel, kMode>(src, stk + threadIdx.x);
 }
 
 // One scene's pixels from a device counter, for persistent launches: the
@@ -1189,12 +1354,12 @@ struct PixelQueue {
 // Persistent form of the path loop (kMode as in k_path_mode, 0 = plain):
 // `total` work indices (pixels of the list, or 64 per 8x8 tile) handed out
 // by `counter`, which must be zero at launch.
-template <int kMode, bool kWide = false>
+template <int kMode>
 __global__ __launch_bounds__(kPathBlock, kMode == 3 ? LISA_MODE_WAVES : 1) void k_path_pq(
     SceneView sc, PathArgs p, uint32_t* counter, uint32_t total, uint32_t chunk) {
   __shared__ uint32_t stk[kLaneLds * kPathBlock];
   PixelQueue src{sc, p, counter, total, chunk, 0u, 0u};
-  path_lane<false, false, PixelQueue, kMode, false, kWide>(src, stk + threadIdx.x);
+  path_lane<false, false, PixelQueue, kMode>(src, stk + threadIdx.x);
 }
 
 // frame[item] += throughput * max(network output, 0) / spp for every query.
@@ -1617,7 +1782,7 @@ __device__ __forceinline__ bool wf_advance(const BatchScene* __restrict__ scenes
   const BatchScene* bs = scenes + scene;
   const SceneView* scp = &bs->sc;
   const PathArgs* pp = &bs->p;
-  TravCount tc;
+  volatile uint32_t spill[kStackMax - kStackLds];
 
   auto finish_sample = [&]() {
     acc = acc + color;
@@ -1783,7 +1948,7 @@ __device__ __forceinline__ bool wf_advance(const BatchScene* __restrict__ scenes
       float t = 0.0f;
       if (valid && scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
         const RayT r = make_ray(O, D);
-        k = closest<false, kWfBlock>(scp->emit, r, kTmin, kTmax, 0xFFFFFFFFu, false, t, my_stk, tc);
+        k = closest_walk<kWfBlock>(scp->emit, r, kTmin, kTmax, 0xFFFFFFFFu, false, t, my_stk, spill);
       }
       if (!valid) {  // counts as a ray, misses without traversal
         hitf = false;
@@ -2461,6 +2626,235 @@ __global__ __launch_bounds__(kBuildBlock) void k_wide(const float4* __restrict__
   w[7] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
+// ---------------------------------------------------------------------------
+// The walk tree: the Morton-ordered triangles of a scene under an
+// agglomerated binary tree (parallel locally-ordered clustering, Meister &
+// Bittner, TVCG 2018), collapsed to 4-wide nodes.  Morton order puts a large
+// triangle (a wall, a floor) among the small ones near its centroid, and
+// every box above it then spans the room; clustering by the surface area of
+// the union leaves such triangles for last.
+//
+// k_agg: one workgroup clusters 1024 consecutive clusters in LDS until 64 are
+// left (the last pass: until the root is left), so a scene takes
+// 1 + log16(T / 1024) launches and no global compaction.  Every cluster finds
+// its nearest neighbour (smallest area of the union) within kAggRadius places;
+// pairs that chose each other merge, and the list is compacted in order.  A
+// tie goes to the neighbour at index ^ 1, then to the lower index pair: the
+// pair that is smallest in this order always merges, so every round shrinks
+// the list, and equal boxes halve it.  After kAggRounds rounds every cluster
+// merges with index ^ 1.
+// ---------------------------------------------------------------------------
+constexpr int kAggChunk = 1024, kAggOut = 64, kAggRadius = 8, kAggRounds = 96;
+constexpr int kAggGroups = kAggChunk / kAggOut;  // outputs of one pass that a workgroup of the next takes
+
+// in (null: the triangles themselves) / out: kAggOut clusters per workgroup,
+// 2 float4 each (lo.xyz | ref, hi.xyz | 0), their counts in in_cnt / out_cnt.
+// nodes: binary nodes in the layout of the Morton tree (64 bytes), this
+// workgroup's from index base + blockIdx.x * (kAggChunk - 1); the root is
+// node 0.
+__global__ __launch_bounds__(kAggChunk) void k_agg(const float4* __restrict__ tris, int32_t T,
+                                                   const float4* __restrict__ in,
+                                                   const uint32_t* __restrict__ in_cnt, int32_t n_in,
+                                                   uint32_t base, float4* __restrict__ nodes,
+                                                   float4* __restrict__ out, uint32_t* __restrict__ out_cnt) {
+  __shared__ float sb[6][kAggChunk];
+  __shared__ uint32_t sref[kAggChunk], snn[kAggChunk];
+  __shared__ uint32_t wsum[kAggChunk / 64];
+  const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool last = gridDim.x == 1;
+  int32_t n;
+  float b[6] = {};
+  uint32_t ref = kEmpty;
+  if (!in) {
+    const int32_t first = (int32_t)blockIdx.x * kAggChunk;
+    n = min(T - first, kAggChunk);
+    if (tid < n) {
+      leaf_box(tris, first + tid, b);
+      ref = kLeaf | (uint32_t)(first + tid);
+      for (int c = 0; c < 6; ++c) sb[c][tid] = b[c];
+      sref[tid] = ref;
+    }
+  } else {
+    // the workgroup's kAggGroups lists, closed up in order
+    const int32_t g0 = (int32_t)blockIdx.x * kAggGroups, g = g0 + tid / kAggOut, r = tid % kAggOut;
+    n = 0;
+    int32_t off = 0, mine = 0;
+    for (int32_t q = g0; q < min(g0 + kAggGroups, n_in); ++q) {
+      const int32_t c = (int32_t)in_cnt[q];
+      if (q < g) off += c;
+      if (q == g) mine = c;
+      n += c;
+    }
+    if (r < mine) {
+      const float4 lo = in[2 * ((size_t)g * kAggOut + r)], hi = in[2 * ((size_t)g * kAggOut + r) + 1];
+      const int32_t at = off + r;
+      sb[0][at] = lo.x, sb[1][at] = lo.y, sb[2][at] = lo.z;
+      sb[3][at] = hi.x, sb[4][at] = hi.y, sb[5][at] = hi.z;
+      sref[at] = __float_as_uint(lo.w);
+    }
+  }
+  __syncthreads();
+  const int32_t target = last ? 1 : max(1, (n + kAggGroups - 1) / kAggGroups);
+  base += blockIdx.x * (uint32_t)(kAggChunk - 1);
+  uint32_t created = 0;
+  for (int32_t it = 0; n > target; ++it) {
+    int32_t best = -1;
+    if (tid < n) {
+      for (int c = 0; c < 6; ++c) b[c] = sb[c][tid];
+      ref = sref[tid];
+      const int32_t pair = tid ^ 1;
+      if (it < kAggRounds) {
+        // area of the union; boxes of non-finite triangles count as the largest
+        auto area = [&](int32_t j) {
+          const float dx = fmaxf(b[3], sb[3][j]) - fminf(b[0], sb[0][j]);
+          const float dy = fmaxf(b[4], sb[4][j]) - fminf(b[1], sb[1][j]);
+          const float dz = fmaxf(b[5], sb[5][j]) - fminf(b[2], sb[2][j]);
+          const float s = dx * dy + dy * dz + dz * dx;
+          return s < 3e38f ? s : 3e38f;
+        };
+        float bs = INFINITY;
+        const int32_t j1 = min(tid + kAggRadius, n - 1);
+        for (int32_t j = max(tid - kAggRadius, 0); j <= j1; ++j) {
+          const float s = area(j);
+          if (j != tid && s < bs) {
+            bs = s;
+            best = j;
+          }
+        }
+        if (pair < n && area(pair) == bs) best = pair;
+      } else if (pair < n) {
+        best = pair;
+      }
+      snn[tid] = (uint32_t)best;
+    }
+    __syncthreads();
+    const bool mate = tid < n && best >= 0 && (int32_t)snn[best] == tid;
+    const bool owner = mate && tid < best, keep = tid < n && !(mate && tid > best);
+    float o[6] = {};
+    uint32_t oref = 0;
+    if (owner) {
+      for (int c = 0; c < 6; ++c) o[c] = sb[c][best];
+      oref = sref[best];
+    }
+    const uint64_t km = __ballot(keep), om = __ballot(owner), below = (1ull << lane) - 1ull;
+    if (lane == 0) wsum[wave] = (uint32_t)__popcll(km) | ((uint32_t)__popcll(om) << 16);
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+    for (int w = 0; w < kAggChunk / 64; ++w) {
+      const uint32_t v = wsum[w];
+      if (w < wave) before += v;
+      all += v;
+    }
+    if (owner) {
+      const uint32_t rank = (before >> 16) + (uint32_t)__popcll(om & below);
+      const uint32_t idx = last && (all & 0xFFFFu) == 1u ? 0u : base + created + rank;
+      float4* np = nodes + 4 * (size_t)idx;
+      np[0] = make_float4(b[0], b[1], b[2], b[3]);
+      np[1] = make_float4(b[4], b[5], o[0], o[1]);
+      np[2] = make_float4(o[2], o[3], o[4], o[5]);
+      np[3] = make_float4(__uint_as_float(ref), __uint_as_float(oref), 0.0f, 0.0f);
+      for (int c = 0; c < 3; ++c) {
+        b[c] = fminf(b[c], o[c]);
+        b[3 + c] = fmaxf(b[3 + c], o[3 + c]);
+      }
+      ref = idx;
+    }
+    if (keep) {
+      const uint32_t at = (before & 0xFFFFu) + (uint32_t)__popcll(km & below);
+      for (int c = 0; c < 6; ++c) sb[c][at] = b[c];
+      sref[at] = ref;
+    }
+    n = (int32_t)(all & 0xFFFFu);
+    created += all >> 16;
+    __syncthreads();
+  }
+  if (last) {
+    if (T == 1 && tid == 0) {  // a root with the single leaf
+      nodes[0] = make_float4(sb[0][0], sb[1][0], sb[2][0], sb[3][0]);
+      nodes[1] = make_float4(sb[4][0], sb[5][0], 0.0f, 0.0f);
+      nodes[2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      nodes[3] = make_float4(__uint_as_float(sref[0]), __uint_as_float(kEmpty), 0.0f, 0.0f);
+    }
+    return;
+  }
+  if (tid < n) {
+    float4* op = out + 2 * ((size_t)blockIdx.x * kAggOut + tid);
+    op[0] = make_float4(sb[0][tid], sb[1][tid], sb[2][tid], __uint_as_float(sref[tid]));
+    op[1] = make_float4(sb[3][tid], sb[4][tid], sb[5][tid], 0.0f);
+  }
+  if (tid == 0) out_cnt[blockIdx.x] = (uint32_t)n;
+}
+
+// Binary nodes that k_agg may write for T triangles: node 0 and kAggChunk - 1
+// per workgroup of every pass.
+inline size_t agg_capacity(int64_t T) {
+  size_t n = 1;
+  for (int64_t c = (T + kAggChunk - 1) / kAggChunk;; c = (c + kAggGroups - 1) / kAggGroups) {
+    n += (size_t)c * (kAggChunk - 1);
+    if (c <= 1) return n;
+  }
+}
+
+// The 4-wide node of every binary node n (those that a walk reaches and the
+// rest): n's children, and twice the inner slot of the largest area replaced
+// by its own two.  128 bytes: lo.x hi.x lo.y hi.y lo.z hi.z of the four slots
+// (a float4 each), the four refs, 16 bytes unused.  An empty slot has an
+// inverted box and the ref of the dummy triangle after the last one, which is
+// never hit.
+__global__ __launch_bounds__(kBuildBlock) void k_walk_nodes(const float4* __restrict__ nodes, uint32_t n_nodes,
+                                                            int32_t T, float4* __restrict__ walk) {
+  const uint32_t n = blockIdx.x * kBuildBlock + threadIdx.x;
+  if (n >= n_nodes) return;
+  const float4* np = nodes + 4 * (size_t)n;
+  float lo[4][3], hi[4][3];
+  uint32_t ref[4];
+  ref[0] = node_child(np, 0, lo[0], hi[0]);
+  ref[1] = node_child(np, 1, lo[1], hi[1]);
+  if (ref[0] == kEmpty) return;  // an index that k_agg left out
+  int m = ref[1] == kEmpty ? 1 : 2;
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+    if (s >= m) {
+      for (int a = 0; a < 3; ++a) lo[s][a] = INFINITY, hi[s][a] = -INFINITY;
+      ref[s] = kLeaf | (uint32_t)T;
+    }
+#pragma unroll
+  for (int step = 2; step < 4; ++step) {
+    int open = -1;
+    float best = -1.0f;
+    uint32_t r = 0;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float dx = hi[s][0] - lo[s][0], dy = hi[s][1] - lo[s][1], dz = hi[s][2] - lo[s][2];
+      const float area = dx * dy + dy * dz + dz * dx;
+      if (!(ref[s] & kLeaf) && (open < 0 || area > best)) {
+        best = area;
+        open = s;
+        r = ref[s];
+      }
+    }
+    if (open < 0) break;
+    float l0[3], h0[3], l1[3], h1[3];
+    const float4* cp = nodes + 4 * (size_t)r;
+    const uint32_t c0 = node_child(cp, 0, l0, h0), c1 = node_child(cp, 1, l1, h1);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (s == open) {
+        for (int a = 0; a < 3; ++a) lo[s][a] = l0[a], hi[s][a] = h0[a];
+        ref[s] = c0;
+      }
+    for (int a = 0; a < 3; ++a) lo[step][a] = l1[a], hi[step][a] = h1[a];
+    ref[step] = c1;
+  }
+  float4* w = walk + 8 * (size_t)n;
+  for (int a = 0; a < 3; ++a) {
+    w[2 * a] = make_float4(lo[0][a], lo[1][a], lo[2][a], lo[3][a]);
+    w[2 * a + 1] = make_float4(hi[0][a], hi[1][a], hi[2][a], hi[3][a]);
+  }
+  w[6] = make_float4(__uint_as_float(ref[0]), __uint_as_float(ref[1]), __uint_as_float(ref[2]),
+                     __uint_as_float(ref[3]));
+}
+
 }  // namespace
 
 // ===========================================================================
@@ -2477,6 +2871,12 @@ struct DevBvh {
   int32_t* parent = nullptr;      // parent of each internal node (kept for refits)
   int32_t* leaf_parent = nullptr; // parent of each leaf
   uint2* range = nullptr;         // sorted leaves [lo, hi] of each internal node (kept for refits)
+  // the walk tree (null: none): 4-wide nodes, the binary nodes they come
+  // from, and k_agg's cluster lists and counts (kept for vertex updates)
+  float4* walk = nullptr;
+  float4* agg = nullptr;
+  float4* lists = nullptr;
+  uint32_t* counts = nullptr;
   uint64_t bytes = 0;
 };
 
@@ -2599,16 +2999,19 @@ hipError_t wf_pending(hipStream_t st, const WfState& ws, uint32_t* pending) {
   return e;
 }
 
+// Triangle count from which a scene's Morton tree also gets its 4-wide form
+// (closest_wide, walked by lisa_trace_rays): 2^20 triangles (64 MB of nodes and
+// 48 MB of triangle records) no longer stay in the caches, and the fewer, wider
+// visits pay; below it the binary walk is the faster one.
+constexpr int64_t kWideMinTris = 1 << 20;
+// closest_walk addresses a node by a 32-bit byte offset: 2^25 nodes of 128
+// bytes, scenes of up to 31 million triangles; larger ones keep the Morton tree.
+constexpr size_t kWalkMaxNodes = size_t{1} << 25;
+
 // lisa_render_progressive: n launches of the plain megakernel, one per
 // subframe, chained in one instantiated hipGraph; before each launch the
 // nodes' arguments (subframe index, buffers) are set on the executable graph,
 // so one graph serves every run of n subframes at one image size.
-// Triangle count from which a scene's tree also gets its 4-wide form
-// (closest_wide): 2^20 triangles (64 MB of nodes and 48 MB of triangle
-// records) no longer stay in the caches, and the fewer, wider visits pay;
-// below it the binary walk is the faster one.
-constexpr int64_t kWideMinTris = 1 << 20;
-
 struct ProgGraph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -2646,6 +3049,7 @@ struct lisa_ctx {
   float render_ms = 0.0f, bvh_ms = 0.0f;
   uint64_t scene_bytes = 0, accum_bytes = 0;
   float bmin[3] = {0, 0, 0}, bmax[3] = {1, 1, 1};  // scene box (cache features)
+  float span = 0.0f;                               // its largest |coordinate|
   float ecull_c[3] = {0, 0, 0}, ecull_h[3] = {INFINITY, INFINITY, INFINITY};  // never culls
   // radiance-cache frame scratch (lisa_render_cached), grown on demand
   DevBuf<float4> c_frame, c_tacc;
@@ -2681,8 +3085,8 @@ struct lisa_ctx {
   DevBuf<float> c_jrgb;
   WfBuffers wf;  // the wavefront form of lisa_render (LISA_FLAG_WAVEFRONT)
   ProgGraph pg;  // lisa_render_progressive's chain of subframe launches
-  // scenes of at least this many triangles get the 4-wide form of their tree
-  // and the path kernels walk it (lisa_set_wide_threshold)
+  // scenes of at least this many triangles get the 4-wide form of their
+  // Morton tree (lisa_set_wide_threshold)
   int64_t wide_min_tris = kWideMinTris;
   // FP64 progressive sums (LISA_FLAG_FP64_ACCUM full renders): r, g, b sums
   // and the sample count per pixel; valid while they belong to the accum
@@ -2739,6 +3143,10 @@ void free_bvh(DevBvh& b) {
   (void)hipFree(b.parent);
   (void)hipFree(b.leaf_parent);
   (void)hipFree(b.range);
+  (void)hipFree(b.walk);
+  (void)hipFree(b.agg);
+  (void)hipFree(b.lists);
+  (void)hipFree(b.counts);
   b = DevBvh();
 }
 
@@ -2757,8 +3165,12 @@ void free_scene(lisa_ctx* c) {
 }
 
 SceneView view(const lisa_ctx* c) {
-  return SceneView{BvhView{c->all.nodes, c->all.tris, c->all.T, c->all.wide},
-                   BvhView{c->emit.nodes, c->emit.tris, c->emit.T, nullptr},
+  // boxes that reach infinity leave closest_walk's margin infinite: such a
+  // scene keeps the Morton tree
+  const bool finite = std::isfinite(c->span);
+  auto walk = [&](const DevBvh& b) { return finite ? reinterpret_cast<const char*>(b.walk) : nullptr; };
+  return SceneView{BvhView{c->all.nodes, c->all.tris, c->all.T, c->all.wide, walk(c->all), c->span},
+                   BvhView{c->emit.nodes, c->emit.tris, c->emit.T, nullptr, walk(c->emit), c->span},
                    c->d_nrm,
                    c->d_mats,
                    make_float4(c->ecull_c[0], c->ecull_c[1], c->ecull_c[2], 0.0f),
@@ -2865,6 +3277,34 @@ lisa_status wide_nodes(lisa_ctx* ctx, DevBvh& b, hipStream_t st) {
   return LISA_OK;
 }
 
+// The walk tree of b (whose triangle records are in place), enqueued on st: no
+// allocation, no wait.
+lisa_status build_walk(lisa_ctx* ctx, DevBvh& b, hipStream_t st) {
+  if (!b.walk || b.T == 0) return LISA_OK;
+  int32_t chunks = (b.T + kAggChunk - 1) / kAggChunk;
+  // two sets of lists in turn
+  const size_t half = (size_t)chunks * kAggOut * 2;
+  const float4* in = nullptr;
+  const uint32_t* in_cnt = nullptr;
+  int32_t n_in = 0;
+  uint32_t base = 1;
+  for (int pass = 0;; ++pass) {
+    float4* out = b.lists + (pass & 1 ? half : 0);
+    uint32_t* out_cnt = b.counts + (pass & 1 ? (b.T + kAggChunk - 1) / kAggChunk : 0);
+    k_agg<<<chunks, kAggChunk, 0, st>>>(b.tris, b.T, in, in_cnt, n_in, base, b.agg, out, out_cnt);
+    if (chunks == 1) break;
+    base += (uint32_t)chunks * (kAggChunk - 1);
+    in = out;
+    in_cnt = out_cnt;
+    n_in = chunks;
+    chunks = (chunks + kAggGroups - 1) / kAggGroups;
+  }
+  const uint32_t cap = (uint32_t)agg_capacity(b.T);
+  k_walk_nodes<<<grid_for(cap, kBuildBlock), kBuildBlock, 0, st>>>(b.agg, cap, b.T, b.walk);
+  HIP_TRY(ctx, hipGetLastError());
+  return LISA_OK;
+}
+
 // LBVH over the n triangles gid[0..n) (all T when gid is null) of the soup
 // already on the device: centroid bounds -> 30-bit Morton codes -> 4-pass LDS
 // radix sort -> Morton-ordered triangle records -> Karras hierarchy -> refit.
@@ -2875,7 +3315,7 @@ lisa_status build_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
   hipStream_t st = ctx->stream;
   b.T = n;
   b.nI = n > 1 ? n - 1 : 1;
-  const size_t nodes_b = 64 * (size_t)b.nI, tris_b = 48 * (size_t)std::max(n, 1);
+  const size_t nodes_b = 64 * (size_t)b.nI, tris_b = 48 * ((size_t)std::max(n, 1) + 1);
   HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.nodes), nodes_b));
   if (wide) {
     HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.wide), 2 * nodes_b));
@@ -2890,6 +3330,16 @@ lisa_status build_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
   b.bytes += nodes_b + tris_b + 16 * (size_t)std::max(n, 1);
   HIP_TRY(ctx, hipMemsetAsync(b.nodes, 0, nodes_b, st));
   if (n == 0) return LISA_OK;
+  if (agg_capacity(n) <= kWalkMaxNodes) {
+    const size_t cap = agg_capacity(n), chunks = ((size_t)n + kAggChunk - 1) / kAggChunk;
+    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.walk), 128 * cap));
+    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.agg), 64 * cap));
+    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.lists), 64 * chunks * kAggOut));
+    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.counts), 8 * chunks));
+    b.bytes += 192 * cap + 64 * chunks * kAggOut + 8 * chunks;
+    HIP_TRY(ctx, hipMemsetAsync(b.agg, 0xFF, 64 * cap, st));  // refs kEmpty: indexes that k_agg leaves out
+    HIP_TRY(ctx, hipMemsetAsync(b.tris + 3 * (size_t)n, 0, 48, st));  // the dummy triangle of empty slots
+  }
   Scratch S;
   float *d_part = nullptr, *d_bounds = nullptr;
   int32_t *d_parent = b.parent, *d_leafp = b.leaf_parent;
@@ -2928,6 +3378,7 @@ lisa_status build_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
     if (rc != LISA_OK) return rc;
   }
   lisa_status rw = wide_nodes(ctx, b, st);
+  if (rw == LISA_OK) rw = build_walk(ctx, b, st);
   if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipGetLastError());
   // scratch is freed on return: wait for the kernels that use it
@@ -2948,6 +3399,7 @@ lisa_status refit_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
     if (rc != LISA_OK) return rc;
   }
   lisa_status rw = wide_nodes(ctx, b, st);
+  if (rw == LISA_OK) rw = build_walk(ctx, b, st);
   if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipStreamSynchronize(st));
   HIP_TRY(ctx, hipGetLastError());
@@ -2974,10 +3426,7 @@ lisa_status launch_persistent(lisa_ctx* ctx, PathArgs a, int slot) {
     total = a.tiles_x * ((a.height + 7) / 8) * 64u;
   }
   const unsigned blocks = (unsigned)(ctx->cus * kPersistentBlocksPerCu);
-  if (ctx->all.wide)
-    k_path_pq<kMode, true><<<blocks, kPathBlock, 0, st>>>(view(ctx), a, counter, total, 1u);
-  else
-    k_path_pq<kMode><<<blocks, kPathBlock, 0, st>>>(view(ctx), a, counter, total, 1u);
+  k_path_pq<kMode><<<blocks, kPathBlock, 0, st>>>(view(ctx), a, counter, total, 1u);
   HIP_TRY(ctx, hipGetLastError());
   return LISA_OK;
 }
@@ -3077,10 +3526,11 @@ lisa_status read_scene_box(lisa_ctx* ctx, bool may_alloc = true) {
   float rb[16];
   HIP_TRY(ctx, hipMemcpy(rb, ctx->all.nodes, 64, hipMemcpyDeviceToHost));
   root_box(rb, ctx->bmin, ctx->bmax);
-  ctx->emit_area = 0.0f;  // no light samples unless the emitters below have area
-  if (ctx->emit.T <= 0) return LISA_OK;
   float S = 0.0f;
   for (int a = 0; a < 3; ++a) S = std::max(S, std::max(std::fabs(ctx->bmin[a]), std::fabs(ctx->bmax[a])));
+  ctx->span = S;
+  ctx->emit_area = 0.0f;  // no light samples unless the emitters below have area
+  if (ctx->emit.T <= 0) return LISA_OK;
   const float m2 = S * 0x1p-11f;
   float lo[3], hi[3];
   HIP_TRY(ctx, hipMemcpy(rb, ctx->emit.nodes, 64, hipMemcpyDeviceToHost));
@@ -3163,10 +3613,7 @@ lisa_status trace_train_rows(lisa_ctx* ctx, PathArgs a, const int32_t* d_pix, si
   a.t_row = ctx->c_trow.p;
   a.t_n = ctx->c_tn.p;
   a.t_depth = depth;
-  if (ctx->all.wide)
-    k_path_mode<2, true><<<grid_for((int64_t)n, kPathBlock), kPathBlock, 0, st>>>(view(ctx), a);
-  else
-    k_path_mode<2><<<grid_for((int64_t)n, kPathBlock), kPathBlock, 0, st>>>(view(ctx), a);
+  k_path_mode<2><<<grid_for((int64_t)n, kPathBlock), kPathBlock, 0, st>>>(view(ctx), a);
   HIP_TRY(ctx, hipGetLastError());
   lisa_status rc = scan_counts(ctx, ctx->c_tn.p, paths, ctx->c_tscan, ctx->c_qcount.p + 1, st);
   if (rc != LISA_OK) return rc;
@@ -3220,13 +3667,8 @@ lisa_status trace_queries_launch(lisa_ctx* ctx, PathArgs& a, const int32_t* d_pi
       a.tiles_x = (a.width + kTileW - 1) / kTileW;
       blocks = a.tiles_x * ((a.height + kTileH - 1) / kTileH);
     }
-    const bool wide = ctx->all.wide != nullptr;
-    if (a.emit_expect && wide)
-      k_path_mode<3, true><<<blocks, kPathBlock, 0, st>>>(view(ctx), a);
-    else if (a.emit_expect)
+    if (a.emit_expect)
       k_path_mode<3><<<blocks, kPathBlock, 0, st>>>(view(ctx), a);
-    else if (wide)
-      k_path_mode<1, true><<<blocks, kPathBlock, 0, st>>>(view(ctx), a);
     else
       k_path_mode<1><<<blocks, kPathBlock, 0, st>>>(view(ctx), a);
     HIP_TRY(ctx, hipGetLastError());
@@ -3319,6 +3761,7 @@ lisa_status lisa_update_vertices_noalloc(lisa_ctx* ctx, const float* d_verts, co
       if (rc != LISA_OK) return rc;
     }
     lisa_status rw = wide_nodes(ctx, *b, st);
+    if (rw == LISA_OK) rw = build_walk(ctx, *b, st);
     if (rw != LISA_OK) return rw;
   }
   HIP_TRY(ctx, hipGetLastError());
@@ -3522,12 +3965,8 @@ lisa_status lisa_render(lisa_ctx* ctx, const lisa_render_params* p, float* accum
     k_path<false, true, true><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
   else if (count)
     k_path<false, true><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
-  else if (a.fp64 && ctx->all.wide)
-    k_path<false, false, true, true><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
   else if (a.fp64)
     k_path<false, false, true><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
-  else if (ctx->all.wide)
-    k_path<false, false, false, true><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
   else
     k_path<false, false><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
   HIP_TRY(ctx, hipGetLastError());
@@ -3590,11 +4029,8 @@ lisa_status lisa_render_progressive(lisa_ctx* ctx, const lisa_render_params* p, 
   a.counters = ctx->d_counters;
   a.sum64 = f64 ? ctx->c_sum64.p : nullptr;
   SceneView sv = view(ctx);
-  const bool wide = ctx->all.wide != nullptr;
-  void* const fn = f64 ? (wide ? reinterpret_cast<void*>(&k_path<false, false, true, true>)
-                               : reinterpret_cast<void*>(&k_path<false, false, true>))
-                       : (wide ? reinterpret_cast<void*>(&k_path<false, false, false, true>)
-                               : reinterpret_cast<void*>(&k_path<false, false, false>));
+  void* const fn = f64 ? reinterpret_cast<void*>(&k_path<false, false, true>)
+                       : reinterpret_cast<void*>(&k_path<false, false>);
   auto node_params = [&](PathArgs& pa, void** args) {
     hipKernelNodeParams kp;
     std::memset(&kp, 0, sizeof(kp));
@@ -4229,10 +4665,7 @@ lisa_status lisa_render_cached(lisa_ctx* ctx, lisa_cache* cache, const lisa_rend
       if (rc != LISA_OK) return rc;
     } else {
       const unsigned tiles = ((p->width + kTileW - 1) / kTileW) * ((p->height + kTileH - 1) / kTileH);
-      if (ctx->all.wide)
-        k_path<false, false, false, true><<<tiles, kPathBlock, 0, st>>>(view(ctx), a);
-      else
-        k_path<false, false><<<tiles, kPathBlock, 0, st>>>(view(ctx), a);
+      k_path<false, false><<<tiles, kPathBlock, 0, st>>>(view(ctx), a);
       HIP_TRY(ctx, hipGetLastError());
     }
     HIP_TRY(ctx, hipStreamSynchronize(st));
