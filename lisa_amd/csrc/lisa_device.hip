@@ -267,6 +267,19 @@ __device__ __forceinline__ bool light_sample_bounded(float4 c, float4 H, F3 O, f
   return 0.9f * A <= d2;
 }
 
+// Triangle bounds widened outward by one ulp: an origin exactly on a face
+// plane of the tight box with a zero direction component would make the
+// slab test evaluate 0 * inf = NaN; inside the widened box it cannot.
+__device__ __forceinline__ void leaf_box(const float4* __restrict__ tris, int32_t k, float* b) {
+  const float4 a = tris[3 * (size_t)k], c = tris[3 * (size_t)k + 1], e = tris[3 * (size_t)k + 2];
+  b[0] = nextafterf(fminf(fminf(a.x, c.x), e.x), -INFINITY);
+  b[1] = nextafterf(fminf(fminf(a.y, c.y), e.y), -INFINITY);
+  b[2] = nextafterf(fminf(fminf(a.z, c.z), e.z), -INFINITY);
+  b[3] = nextafterf(fmaxf(fmaxf(a.x, c.x), e.x), INFINITY);
+  b[4] = nextafterf(fmaxf(fmaxf(a.y, c.y), e.y), INFINITY);
+  b[5] = nextafterf(fmaxf(fmaxf(a.z, c.z), e.z), INFINITY);
+}
+
 struct TravCount {
   uint64_t visits = 0, tests = 0;
 };
@@ -610,6 +623,15 @@ __device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r
       }
     }
     t_out = best_t;
+    // closest() tests a triangle only when slab() passes its leaf box, and the
+    // wider test above may let one more through: a hit whose rounded t is past
+    // tmin though the ray leaves the box before it, an edge just outside the
+    // box.  The hit stands if its own box passes; otherwise closest() answers.
+    if (best_k >= 0) {
+      float b[6], tn;
+      leaf_box(bv.tris, best_k, b);
+      done = done && slab(b[0], b[1], b[2], b[3], b[4], b[5], r, tmin, tlim * kWiden, tn);
+    }
   }
   if (!done) {
     TravCount tc;
@@ -2458,19 +2480,6 @@ __global__ __launch_bounds__(kBuildBlock) void k_karras(const uint32_t* __restri
     leaf_parent[g + 1] = (int32_t)i;
   else
     parent[g + 1] = (int32_t)i;
-}
-
-// Triangle bounds widened outward by one ulp: an origin exactly on a face
-// plane of the tight box with a zero direction component would make the
-// slab test evaluate 0 * inf = NaN; inside the widened box it cannot.
-__device__ __forceinline__ void leaf_box(const float4* __restrict__ tris, int32_t k, float* b) {
-  const float4 a = tris[3 * (size_t)k], c = tris[3 * (size_t)k + 1], e = tris[3 * (size_t)k + 2];
-  b[0] = nextafterf(fminf(fminf(a.x, c.x), e.x), -INFINITY);
-  b[1] = nextafterf(fminf(fminf(a.y, c.y), e.y), -INFINITY);
-  b[2] = nextafterf(fminf(fminf(a.z, c.z), e.z), -INFINITY);
-  b[3] = nextafterf(fmaxf(fmaxf(a.x, c.x), e.x), INFINITY);
-  b[4] = nextafterf(fmaxf(fmaxf(a.y, c.y), e.y), INFINITY);
-  b[5] = nextafterf(fmaxf(fmaxf(a.z, c.z), e.z), INFINITY);
 }
 
 __device__ __forceinline__ void store_slot(float4* nodes, int32_t node, int slot, const float* b) {

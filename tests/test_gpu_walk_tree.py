@@ -153,3 +153,37 @@ def test_follows_vertex_updates(capi, oracle_mod, T):
             rp, rt, _ = o.closest_hit(O, D, brute=True)
             assert np.array_equal(gp, rp) and _same(gt, rt)
             assert _same(*_both(capi, ctx))
+
+
+def test_hits_at_the_edge_of_the_leaf_box(capi, oracle_mod):
+    """Rays whose rounded hit lies just past tmin, or just inside a triangle's
+    edge, while the Morton walk's test of the leaf's own box fails (or just
+    passes): the Morton walk's answer.  Large flat quads among small ones give t
+    a relative error near 1e-3."""
+    rs = np.random.default_rng(7)
+    q = np.float32([[-1.6, 0, -1.6, -1.6, 0, 1.6, 1.6, 0, 1.6], [-1.6, 0, -1.6, 1.6, 0, 1.6, 1.6, 0, -1.6]])
+    small, n, _ = _soup(400, 7)
+    v = np.concatenate([q, small * 0.1 + np.float32([0.0, -1.5, 0.0] * 3)])
+    n, m = np.tile(np.float32([0, 1, 0]), (len(v), 3)), np.zeros(len(v), np.int32)
+    k = 1 << 20
+    D = rs.normal(size=(k, 3))
+    D /= np.linalg.norm(D, axis=1, keepdims=True)
+    D[:, 1] = np.abs(D[:, 1]) + 0.01
+    O = rs.uniform(-1.5, 1.5, (k, 3))
+    O[:, 1] = -D[:, 1] * 1e-4 * (1.0 + rs.uniform(-2e-3, 2e-3, k))  # t near tmin
+    h = k // 2  # the quads' outer edges, from a distance
+    P = rs.uniform(-1.6, 1.6, (h, 3))
+    P[:, 0] = np.where(rs.random(h) < 0.5, 1.0, -1.0) * np.float64(np.float32(1.6)) * (1 + rs.uniform(-2e-7, 2e-7, h))
+    P[:, 1] = 0.0
+    O[:h] = P - D[:h] * rs.uniform(0.5, 3.0, (h, 1))
+    O, D = O.astype(np.float32), D.astype(np.float32)
+    o = oracle_mod.Scene(v, n, m, MATS)
+    with capi.Context(0) as ctx:
+        ctx.set_scene(v, n, m, MATS)
+        gp, gt = ctx.trace_rays(O, D)
+        rp, rt, _ = o.closest_hit(O, D, threads=16)
+        near = (rt > 0) & (rt < 1.1e-4)
+        assert near.any() and (~near[h:]).any() and (rp[:h] < 0).any()
+        bp, _, _ = o.closest_hit(O[h:h + 8192], D[h:h + 8192], brute=True)
+        assert (bp != rp[h:h + 8192]).any()  # the box does decide some of these
+        assert np.array_equal(gp, rp) and _same(gt, rt)
