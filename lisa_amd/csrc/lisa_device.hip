@@ -242,6 +242,40 @@ __device__ __forceinline__ bool line_culled(float4 c, float4 H, F3 O, F3 d) {
   if (fabsf(vx * d.y - vy * d.x) > H.x * ay + H.y * ax) return true;
   return false;
 }
+// The next try of an NEE loop whose line is not culled: draws tries (three
+// LCG steps each) until line_culled() lets one through or kNeeTries are made.
+// True: `raw` holds its draws, as hemisphere_raw gives them.  False: all are
+// made.  The draws stay integers k - 2^23 (raw times 2^23, exact): the state
+// with bit 23 flipped is (k - 2^23) mod 2^24 and steps by the same recurrence,
+// so a draw is a multiply-add, a sign extension and a conversion.  The products
+// of a test are fused (one rounding each instead of two, within the margin), and
+// its three axes run without branches: nearly every vertex makes all of its
+// tries, and a wave makes them together (C2 at 32 spp 44.5 -> 40.4 ms, Cornell box
+// of 1k triangles at 256^2, 16 spp 5.4 -> 4.6 ms, with lcg24).
+__device__ __forceinline__ bool next_try(float4 c, float4 H, F3 O, uint32_t& seed, int32_t& tries, F3& raw) {
+  const float vx = c.x - O.x, vy = c.y - O.y, vz = c.z - O.z;
+  uint32_t t = seed ^ 0x800000u;
+  float x, y, z;
+  bool culled;
+  auto draw = [&]() {
+    t = lcg24(t);
+    return (float)((int32_t)(t << 8) >> 8);
+  };
+  do {
+    x = draw();
+    y = draw();
+    z = draw();
+    const float ax = fabsf(x), ay = fabsf(y), az = fabsf(z);
+    const float px = __builtin_fmaf(vy, z, -(vz * y)), py = __builtin_fmaf(vz, x, -(vx * z)),
+                pz = __builtin_fmaf(vx, y, -(vy * x));
+    const float qx = __builtin_fmaf(H.y, az, H.z * ay), qy = __builtin_fmaf(H.z, ax, H.x * az),
+                qz = __builtin_fmaf(H.x, ay, H.y * ax);
+    culled = ((fabsf(px) > qx) | (fabsf(py) > qy) | (fabsf(pz) > qz)) & (fminf(fminf(ax, ay), az) != 0.0f);
+  } while (culled && ++tries < kNeeTries);
+  seed = t ^ 0x800000u;
+  raw = mk(x, y, z) * 0x1p-23f;
+  return !culled;
+}
 // emit_culled: the ray misses the box -- the box lies behind the origin along
 // an axis the ray moves away on, or the ray's line misses it.
 __device__ __forceinline__ bool emit_culled(float4 c, float4 H, F3 O, F3 D) {
@@ -835,8 +869,10 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   int32_t occl_cnt = 0;
   size_t rec_base = (size_t)item * pp->spp;
 
+  constexpr bool kScan = !kCount && !kRecord;  // culled NEE tries by next_try, none seen one by one
   constexpr bool kQuery = kMode == 1 || kMode == 3;  // ends at the cache query
   constexpr bool kEmit = kMode == 3;                 // prefix emission in expectation
+  static_assert(kScan || !kEmit, "kMode 3 leaves the draws of a try to the NEE loop");
   uint32_t t_used = 0;  // kMode 2: vertex slots recorded in this sample
   // kMode 3: the current radiance ray is a bounce drawn on
   // the condition that it hits no emitter (redrawn when it does); lw is the
@@ -942,7 +978,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     if (kRecord) hash = (hash ^ ((uint32_t)code ^ 0x5bd1e995u)) * 16777619u;
     if (hitf) return end_nee(xyz(scp->mats[*light_mat].emission_emit) * Bsdf::eval(N, D));
     if (++tries == kNeeTries) return end_nee(mk(0.0f, 0.0f, 0.0f));
-    D = hemisphere_raw(seed);  // finished in the emitter-query loop
+    if (!kScan) D = hemisphere_raw(seed);  // finished in the emitter-query loop
     qstage = 1;
     return true;
   };
@@ -1005,15 +1041,26 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     // false (shader.cu:172-184), so with the flag false a ray that hits no
     // emitter is resolved here; these cheap tries loop without waiting for
     // the wave's full traversals.
-    // D holds hemisphere()'s raw draws; with the flag false a try whose line
-    // misses every emitter ends here without normalising them.
+    // With the flag false a try whose line misses every emitter ends here
+    // without normalising its draws (kScan: in next_try; else D holds the draws
+    // of the try).
     while (qstage == 1) {
-      if (kCount) c_occ++;
-      if (kRecord) occl_cnt++;
-      if (!hitf && line_culled(scp->ecull_c, scp->ecull_h, O, D)) {
-        alive = nee_after(-5);
-        if (!alive) break;
-        continue;
+      if constexpr (kScan) {
+        if (hitf) {
+          D = hemisphere_raw(seed);
+        } else if (!next_try(scp->ecull_c, scp->ecull_h, O, seed, tries, D)) {
+          alive = end_nee(mk(0.0f, 0.0f, 0.0f));
+          if (!alive) break;
+          continue;
+        }
+      } else {
+        if (kCount) c_occ++;
+        if (kRecord) occl_cnt++;
+        if (!hitf && line_culled(scp->ecull_c, scp->ecull_h, O, D)) {
+          alive = nee_after(-5);
+          if (!alive) break;
+          continue;
+        }
       }
       D = hemisphere_dir(D, N);
       const bool valid = ray_valid(D);
@@ -1053,7 +1100,6 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
         hitf = (ent & 1) != 0;
         *light_mat = ent >> 1;
         tries = 0;
-        D = hemisphere_raw(seed);
         qstage = 1;
         continue;
       }
@@ -1231,7 +1277,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
               ent = (*light_mat << 1) | (hitf ? 1 : 0);
               nl = 0;
             }
-            D = hemisphere_raw(seed);
+            if (!kScan) D = hemisphere_raw(seed);
           }
         }
       }

@@ -50,15 +50,20 @@ __device__ __forceinline__ uint32_t tea16(uint32_t v0, uint32_t v1) {
   }
   return v0;
 }
+// One step of the LCG (random.h:49-55).  Only the low 24 bits of the state are
+// ever drawn from, and the low 24 bits of a step depend on no others, so a
+// 24-bit multiply-add (full rate; a 32-bit multiply is a quarter of it) gives
+// every draw; the bits above are not the LCG's.
+__device__ __forceinline__ uint32_t lcg24(uint32_t s) { return __umul24(s, 1664525u) + 1013904223u; }
 __device__ __forceinline__ float rnd(uint32_t& s) {
-  s = 1664525u * s + 1013904223u;
+  s = lcg24(s);
   return (float)(s & 0x00FFFFFFu) / (float)0x01000000;
 }
 // rnd(s) * 2 - 1 (maths.cu:6-8) as one fused multiply-add: k * 2^-24 * 2 - 1
 // is exact for every 24-bit k (a multiple of 2^-23 in [-1, 1)), so the fused
 // form gives the same bits with two instructions fewer.
 __device__ __forceinline__ float rng(uint32_t& s) {
-  s = 1664525u * s + 1013904223u;
+  s = lcg24(s);
   return __builtin_fmaf((float)(s & 0x00FFFFFFu), 0x1p-23f, -1.0f);
 }
 
