@@ -64,14 +64,14 @@ def build(verbose_resources=False, defines=(), out_dir=OUT, cli=True):
 
 # Variant of the library with a 2-entry LDS traversal stack: every deeper
 # entry goes to the per-lane private overflow array, and a walk of the
-# agglomerated tree past 9 entries is left to the Morton tree, so a parity test
+# agglomerated tree past 8 entries is left to the Morton tree, so a parity test
 # run against it exercises both paths (the default 20-entry stack never
 # overflows on the benchmark scenes).
 SMALL_STACK = os.path.join(OUT, "stack2")
 
 
 def build_small_stack():
-    return build(defines=("LISA_STACK_LDS=2", "LISA_WALK_STACK=9"), out_dir=SMALL_STACK, cli=False)
+    return build(defines=("LISA_STACK_LDS=2", "LISA_WALK_STACK=8"), out_dir=SMALL_STACK, cli=False)
 
 
 if __name__ == "__main__":

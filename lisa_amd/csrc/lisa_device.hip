@@ -52,15 +52,16 @@ constexpr int kNeeTries = 30;   // shader.cu:199
 // a private spill array.  The depth of a Karras tree over index-augmented
 // 30-bit keys is below 64, so kStackMax entries always suffice.
 #ifndef LISA_STACK_LDS
-#define LISA_STACK_LDS 20
+#define LISA_STACK_LDS 26
 #endif
 #ifndef LISA_PATH_BLOCK
 #define LISA_PATH_BLOCK 64
 #endif
 // Waves per SIMD the path kernels are compiled for: 5 (96 VGPRs).  The walk of
 // the 4-wide tree holds a node's 28 words at once; at 6 waves (80 VGPRs) k_path
-// spills 29 registers around it and C2 (32 spp) takes 55.4 ms against 44.5, at 4
-// (101 VGPRs, no spill) 49.2.  The counting and recording builds run at 4, and
+// spills 23 registers around it and C2 (32 spp) takes 38.4 ms against 37.2, at 4
+// (101 VGPRs, no spill) 40.3.  The query kernel with the light samples carries
+// more state: 4 (at 5 it spills 95 registers).  The counting and recording builds run at 4, and
 // the batched lane-queue form keeps the registers it needs.
 #ifndef LISA_PATH_MIN_BLOCKS
 #define LISA_PATH_MIN_BLOCKS 5
@@ -69,7 +70,7 @@ constexpr int kNeeTries = 30;   // shader.cu:199
 #define LISA_MODE_WAVES 5  // the cache-mode path kernels
 #endif
 #ifndef LISA_EMIT_WAVES
-#define LISA_EMIT_WAVES 5  // the query kernel with the prefix-emission light samples
+#define LISA_EMIT_WAVES 4  // the query kernel with the prefix-emission light samples
 #endif
 #ifndef LISA_TILE_WAVES
 #define LISA_TILE_WAVES 5  // the batched wave-tile form
@@ -83,20 +84,21 @@ constexpr int kNeeTries = 30;   // shader.cu:199
 #endif
 constexpr int kStackLds = LISA_STACK_LDS;
 constexpr int kStackMax = 64;
-// Entries closest_walk may hold (at most kStackMax) before it leaves a query
-// to closest().
+// LDS stack entries closest_walk may hold before it leaves a query to
+// closest().
 #ifndef LISA_WALK_STACK
-#define LISA_WALK_STACK 64
+#define LISA_WALK_STACK LISA_STACK_LDS
 #endif
 constexpr int kWalkStack = LISA_WALK_STACK;
+constexpr int kStackRows = kStackLds > kWalkStack ? kStackLds : kWalkStack;  // LDS words per lane of a walk
 // LDS words per lane of a path kernel: the traversal stack, then the pixel's
 // running sum of sample radiance (3 floats, touched once per sample) and the
 // NEE light material (written when a NEE ray finds a light) -- in LDS so
-// that they hold no register through the path loop.  At 20 + 4 words a
-// 64-lane workgroup takes 6 KB, 24 of them (6 waves per SIMD) 144 KB
-// (6.5 KB per workgroup measured 7 % slower: fewer workgroups fit).  The
-// benchmark scenes' traversals need at most 18 stack entries.
-constexpr int kLaneLds = kStackLds + 4;
+// that they hold no register through the path loop.  At 26 + 4 words a
+// 64-lane workgroup takes 7.5 KB, 20 of them (5 waves per SIMD) 150 KB of the
+// CU's 160 (28 + 4 words: fewer workgroups fit, C2 5 % slower; 20 + 4: walks of
+// the batch scenes pass the stack, 25 % slower there).
+constexpr int kLaneLds = kStackRows + 4;
 // Path workgroup: kPathBlock work-items on a kTileW x kTileH pixel tile
 // (64: 8x8, 128: 16x8, 256: 16x16), so a wave covers a compact 8-row or
 // 4-row block of pixels whose camera rays start coherent.
@@ -105,7 +107,7 @@ constexpr int kTileW = kPathBlock >= 128 ? 16 : 8;
 constexpr int kTileH = kPathBlock / kTileW;
 constexpr int kRayBlock = 256;
 static_assert(kStackLds >= 1 && kStackLds <= kStackMax, "LDS stack depth");
-static_assert(kWalkStack >= 3 && kWalkStack <= kStackMax, "walk stack depth");
+static_assert(kWalkStack >= 4, "walk stack depth");
 static_assert(kPathBlock == 64 || kPathBlock == 128 || kPathBlock == 256, "path block size");
 
 struct DevMat {
@@ -531,10 +533,15 @@ __device__ __forceinline__ int32_t closest_wide(const BvhView& bv, const RayT& r
 // An iteration visits an inner node and then tests a triangle if the lane
 // holds one, so the wave runs one copy of the triangle test per iteration
 // whatever its lanes found (the four slots' tests in closest_wide() each ran
-// whenever one lane of the wave needed them).  A stack that would pass
-// kWalkStack entries (never seen on a benchmark scene; the tree's depth is not
-// bounded by the construction) leaves the query to closest() over the Morton
-// tree, as does a scene without a walk tree.
+// whenever one lane of the wave needed them).  The empty asm statements keep
+// the compiler from threading the jumps of lanes that hold an inner node after
+// an inner node, or a triangle after a triangle, into loops of their own, where
+// the rest of the wave would wait for them (C2 at 32 spp 45.9 ms against
+// 37.3).  The stack is LDS only and ends
+// in a sentinel; a walk that would pass kWalkStack entries leaves the query to
+// closest() over the Morton tree (the tree's depth is not bounded by its
+// construction; 20 entries are passed by 1e-5 of a batch scene's walks, 28 by
+// none seen), as does a scene without a walk tree.
 //
 // Bound by instruction issue of the wave's longest walk.  Visits per ray and
 // per wave of 64 (the longest): Cornell box of 65k triangles 23.4 / 60.5 in
@@ -563,10 +570,11 @@ __device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r
     const char* __restrict__ base = bv.walk;
     float best_t = tlim, cull_t = tlim * kWiden;
     uint32_t best_prim = lim_prim, cur = 0;
-    int sp = 0;
+    int sp = 1;
+    stk[0] = kEmpty;  // popped last: the end of the walk
     done = true;
     for (;;) {
-      bool pop = false;
+      asm volatile("" : "+v"(cur));
       if (!(cur & kLeaf)) {
         const uint32_t ox = (cur << 7) | sx, oy = (cur << 7) | sy, oz = (cur << 7) | sz;
         const float4 nx = *reinterpret_cast<const float4*>(base + ox);
@@ -604,38 +612,28 @@ __device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r
         cswap(0, 2);
         cswap(1, 3);
         cswap(1, 2);
-        if (sp <= kStackLds - 3) {
-          // far to near; an entry that is not there is overwritten by the next
-          stk[sp * kStride] = ref[3];
-          sp += key[3] < INFINITY ? 1 : 0;
-          stk[sp * kStride] = ref[2];
-          sp += key[2] < INFINITY ? 1 : 0;
-          stk[sp * kStride] = ref[1];
-          sp += key[1] < INFINITY ? 1 : 0;
-        } else {
-          if (sp > kWalkStack - 3) {
-            done = false;
-            break;
-          }
-#pragma unroll
-          for (int q = 3; q >= 1; --q) {
-            if (key[q] < INFINITY) {
-              if (sp < kStackLds)
-                stk[sp * kStride] = ref[q];
-              else
-                spill[sp - kStackLds] = ref[q];
-              ++sp;
-            }
-          }
-        }
+        // far to near; an entry that is not there is overwritten by the next
+        stk[sp * kStride] = ref[3];
+        sp += key[3] < INFINITY ? 1 : 0;
+        stk[sp * kStride] = ref[2];
+        sp += key[2] < INFINITY ? 1 : 0;
+        stk[sp * kStride] = ref[1];
+        sp += key[1] < INFINITY ? 1 : 0;
         cur = ref[0];
-        pop = !(key[0] < INFINITY);
+        if (!(key[0] < INFINITY)) cur = stk[--sp * kStride];
+        if (sp > kWalkStack - 3) {
+          done = false;
+          cur = kEmpty;
+        }
       }
-      if (!pop && (cur & kLeaf)) {
+      asm volatile("" : "+v"(cur));
+      if (cur == kEmpty) break;
+      if (cur & kLeaf) {
         const uint32_t k = cur & ~kLeaf;
         const float4* tp = bv.tris + 3 * (size_t)k;
         const float4 t0 = tp[0], t1 = tp[1], t2 = tp[2];
         const uint32_t prim = __float_as_uint(t0.w);
+        cur = stk[--sp * kStride];
         float t;
         if (watertight(r, xyz(t0), xyz(t1), xyz(t2), t) && t > tmin &&
             (t < best_t || (t == best_t && prim < best_prim))) {
@@ -643,17 +641,8 @@ __device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r
           cull_t = t * kWiden;
           best_prim = prim;
           best_k = (int32_t)k;
-          if (any) break;
+          if (any) cur = kEmpty;
         }
-        pop = true;
-      }
-      if (pop) {
-        if (sp == 0) break;
-        --sp;
-        if (sp < kStackLds)
-          cur = stk[sp * kStride];
-        else
-          cur = spill[sp - kStackLds];
       }
     }
     t_out = best_t;
@@ -684,7 +673,7 @@ __global__ __launch_bounds__(kRayBlock) void k_trace_rays(SceneView sc, const fl
                                                           int32_t* __restrict__ prim_out,
                                                           float* __restrict__ t_out,
                                                           unsigned long long* counters) {
-  __shared__ uint32_t stk[kStackLds * kRayBlock];
+  __shared__ uint32_t stk[kStackRows * kRayBlock];
   const int32_t i = blockIdx.x * kRayBlock + threadIdx.x;
   if (i >= n) return;
   const F3 o = mk(O[3 * i], O[3 * i + 1], O[3 * i + 2]);
@@ -845,7 +834,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   };
 
   // the pixel's sum of sample radiance, in LDS after the lane's stack
-  float* const acc = reinterpret_cast<float*>(my_stk + kStackLds * kPathBlock);
+  float* const acc = reinterpret_cast<float*>(my_stk + kStackRows * kPathBlock);
   acc[0] = 0.0f;
   acc[kPathBlock] = 0.0f;
   acc[2 * kPathBlock] = 0.0f;
@@ -859,7 +848,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   int32_t qstage = 0;  // 0 radiance ray, 1 NEE emitter query, 2 NEE any-hit query
   int32_t tries = 0, matE = -1;
   // RayState::material of the NEE's light (shader.cu:38), in LDS after acc
-  int32_t* const light_mat = reinterpret_cast<int32_t*>(my_stk + (kStackLds + 3) * kPathBlock);
+  int32_t* const light_mat = reinterpret_cast<int32_t*>(my_stk + (kStackRows + 3) * kPathBlock);
   *light_mat = 0;
   uint32_t primE = 0xFFFFFFFFu;
   float tE = kTmax;
@@ -2072,8 +2061,8 @@ __device__ __forceinline__ void wf_enqueue(const WfState& ws, uint32_t nxt, bool
 
 __global__ __launch_bounds__(kWfBlock, 4) void k_wf_shade(const BatchScene* __restrict__ scenes, int32_t n_scenes,
                                                           uint32_t total, WfState ws, uint32_t cur) {
-  __shared__ uint32_t stk[(kStackLds + 1) * kWfBlock];
-  uint32_t* row = stk + kStackLds * kWfBlock;
+  __shared__ uint32_t stk[(kStackRows + 1) * kWfBlock];
+  uint32_t* row = stk + kStackRows * kWfBlock;
   const uint32_t n = ws.cnt[cur];
   for (uint32_t base = blockIdx.x * kWfBlock; base < n; base += gridDim.x * kWfBlock) {
     const uint32_t i = base + threadIdx.x;
@@ -2086,8 +2075,8 @@ __global__ __launch_bounds__(kWfBlock, 4) void k_wf_shade(const BatchScene* __re
 
 __global__ __launch_bounds__(kWfBlock, 4) void k_wf_start(const BatchScene* __restrict__ scenes, int32_t n_scenes,
                                                           uint32_t total, WfState ws) {
-  __shared__ uint32_t stk[(kStackLds + 1) * kWfBlock];
-  uint32_t* row = stk + kStackLds * kWfBlock;
+  __shared__ uint32_t stk[(kStackRows + 1) * kWfBlock];
+  uint32_t* row = stk + kStackRows * kWfBlock;
   const uint32_t i = blockIdx.x * kWfBlock + threadIdx.x;
   uint32_t req = 0;
   bool need = false;
