@@ -132,6 +132,7 @@ struct SceneView {
   const float4* __restrict__ nrm;  // vertex normals, Morton order of `all`
   const DevMat* __restrict__ mats;
   float4 ecull_c, ecull_h;  // emitter cull box: centre, inflated half extents (emit_culled)
+  uint32_t emit_root;       // root of the emitters' walk tree, in `all`'s walk nodes
 };
 
 // ---------------------------------------------------------------------------
@@ -549,10 +550,19 @@ __device__ __forceinline__ int32_t closest_wide(const BvhView& bv, const RayT& r
 // icosphere of 328k 21.0 / 63.6, 11.1 / 32.7, 5.4 / 23.2.  k_path at 32 spp,
 // 1024^2: C2 67.5 -> 44.5 ms; icosphere of 1.3M triangles, 1080p, 16 spp:
 // 85.6 -> 53.8 ms (before: its 4-wide Morton walk).
-template <int kStride>
-__device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r, float tmin,
+//
+// Pausing (kPause): once no more than a quarter of the lanes that entered are
+// left walking, each of these puts its walk on its stack and leaves with
+// paused != 0; the same query called again (paused as left) goes on from there.
+// The caller gives the finished lanes their next rays in between.  Without it 76 %
+// of the walk's iterations on C2 ran for 16 lanes or fewer (14 of 64 walking on
+// average, 38 with it), for 1.6 times as many rounds of the path loop (C2 at
+// 32 spp 38.4 -> 29.1 ms).  An eighth of the lanes 29.8, a half 29.7 ms.
+template <int kStride, bool kPause = false>
+__device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitters, const RayT& r, float tmin,
                                                 float tlim, uint32_t lim_prim, bool any, float& t_out,
-                                                uint32_t* stk, volatile uint32_t* spill) {
+                                                uint32_t* stk, volatile uint32_t* spill, int32_t& paused) {
+  const BvhView& bv = sc.all;
   bool done = false;
   int32_t best_k = -1;
   if (bv.walk) {
@@ -569,11 +579,31 @@ __device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r
     const uint32_t sx = inv.x < 0.0f ? 16u : 0u, sy = inv.y < 0.0f ? 16u : 0u, sz = inv.z < 0.0f ? 16u : 0u;
     const char* __restrict__ base = bv.walk;
     float best_t = tlim, cull_t = tlim * kWiden;
-    uint32_t best_prim = lim_prim, cur = 0;
+    uint32_t best_prim = lim_prim, cur = emitters ? sc.emit_root : 0u;
     int sp = 1;
-    stk[0] = kEmpty;  // popped last: the end of the walk
+    int quorum = 0;
+    if (kPause && paused) {
+      sp = paused;
+      cur = stk[sp * kStride];
+      best_t = __uint_as_float(stk[(sp + 1) * kStride]);
+      best_prim = stk[(sp + 2) * kStride];
+      best_k = (int32_t)stk[(sp + 3) * kStride];
+      cull_t = best_t * kWiden;
+      paused = 0;
+    } else {
+      stk[0] = kEmpty;  // popped last: the end of the walk
+    }
+    if (kPause) quorum = __popcll(__ballot(1)) / 4;
     done = true;
     for (;;) {
+      if (kPause && __popcll(__ballot(1)) <= quorum && cur != kEmpty) {
+        stk[sp * kStride] = cur;
+        stk[(sp + 1) * kStride] = __float_as_uint(best_t);
+        stk[(sp + 2) * kStride] = best_prim;
+        stk[(sp + 3) * kStride] = (uint32_t)best_k;
+        paused = sp;
+        return -1;
+      }
       asm volatile("" : "+v"(cur));
       if (!(cur & kLeaf)) {
         const uint32_t ox = (cur << 7) | sx, oy = (cur << 7) | sy, oz = (cur << 7) | sz;
@@ -621,7 +651,7 @@ __device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r
         sp += key[1] < INFINITY ? 1 : 0;
         cur = ref[0];
         if (!(key[0] < INFINITY)) cur = stk[--sp * kStride];
-        if (sp > kWalkStack - 3) {
+        if (sp > kWalkStack - 4) {  // room for a node's entries or a paused walk
           done = false;
           cur = kEmpty;
         }
@@ -657,8 +687,12 @@ __device__ __forceinline__ int32_t closest_walk(const BvhView& bv, const RayT& r
     }
   }
   if (!done) {
+    const BvhView slow{emitters ? sc.emit.nodes : sc.all.nodes, emitters ? sc.emit.tris : sc.all.tris,
+                       emitters ? sc.emit.T : sc.all.T, nullptr, nullptr, 0.0f};
     TravCount tc;
-    best_k = closest<false, kStride>(bv, r, tmin, tlim, lim_prim, any, t_out, stk, spill, tc);
+    best_k = closest<false, kStride>(slow, r, tmin, tlim, lim_prim, any, t_out, stk, spill, tc);
+    if (emitters && best_k >= 0)  // the triangle's place in `all`
+      best_k = (int32_t)__float_as_uint(sc.emit.tris[3 * (size_t)best_k + 2].w);
   }
   return best_k;
 }
@@ -684,12 +718,13 @@ __global__ __launch_bounds__(kRayBlock) void k_trace_rays(SceneView sc, const fl
   if (sc.all.T > 0 && ray_valid(d)) {
     const RayT r = make_ray(o, d);
     volatile uint32_t spill[kStackMax - kStackLds];
+    int32_t paused = 0;
     int32_t k = closest<kCount, kRayBlock>(sc.all, r, tmin, tmax, 0xFFFFFFFFu, false, t,
                                            stk + threadIdx.x, spill, cnt);
     // the hit is the walk tree's (which the path kernels use), or with a
     // 4-wide form of the Morton tree that one's; the counts are the binary walk's
     if (!sc.all.wide)
-      k = closest_walk<kRayBlock>(sc.all, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x, spill);
+      k = closest_walk<kRayBlock>(sc, false, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x, spill, paused);
     else
       k = closest_wide<kRayBlock>(sc.all, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x);
     if (k >= 0) prim = (int32_t)__float_as_uint(sc.all.tris[3 * (size_t)k].w);
@@ -824,15 +859,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   uint64_t c_rad = 0, c_occ = 0, c_rhit = 0, c_inv = 0, c_smp = 0, c_px = 0;
   TravCount tc;
   volatile uint32_t spill[kStackMax - kStackLds];
-  // A query over one of the scene's trees: the counting builds walk the
-  // Morton tree, whose visits the counters define, the others the walk tree.
-  auto query = [&](const BvhView& bv, const RayT& r, float tlim, uint32_t lim, bool any, float& t) -> int32_t {
-    if constexpr (kCount)
-      return closest<true, kPathBlock>(bv, r, kTmin, tlim, lim, any, t, my_stk, spill, tc);
-    else
-      return closest_walk<kPathBlock>(bv, r, kTmin, tlim, lim, any, t, my_stk, spill);
-  };
-
+  int32_t paused = 0;  // the ray's walk is under way (closest_walk)
   // the pixel's sum of sample radiance, in LDS after the lane's stack
   float* const acc = reinterpret_cast<float*>(my_stk + kStackRows * kPathBlock);
   acc[0] = 0.0f;
@@ -845,7 +872,8 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   // of the NEE rays and of the next bounce).
   F3 O = mk(0.0f, 0.0f, 0.0f), D = O, color = O, att = O, N = O, Din = O;
   bool hitf = false;
-  int32_t qstage = 0;  // 0 radiance ray, 1 NEE emitter query, 2 NEE any-hit query
+  // 0 radiance ray, 1 NEE try, 6 its emitter query (kScan), 2 its any-hit query
+  int32_t qstage = 0;
   int32_t tries = 0, matE = -1;
   // RayState::material of the NEE's light (shader.cu:38), in LDS after acc
   int32_t* const light_mat = reinterpret_cast<int32_t*>(my_stk + (kStackRows + 3) * kPathBlock);
@@ -867,7 +895,8 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   // the condition that it hits no emitter (redrawn when it does); lw is the
   // pending light sample's weight
   bool cond = false;
-  int32_t rejects = 0, ls_k = 0;  // ls_k: the light sample's emitter triangle
+  int32_t rejects = 0;
+  uint32_t ls_prim = 0;  // the light sample's emitter triangle
   float lw = 0.0f;
   // kMode 3 with nee_loops > 1: the vertex's entry light and flag (light * 2
   // + flag) and the NEE runs done
@@ -1025,14 +1054,15 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
       alive = begin_sample();
       continue;
     }
-    // -- NEE occlusion rays, first query: the closest emitter (emitter BVH).
+    // -- NEE occlusion rays, first query: the closest emitter (emitter tree).
     // A miss and a non-emitting closest hit both leave a false hit flag
     // false (shader.cu:172-184), so with the flag false a ray that hits no
     // emitter is resolved here; these cheap tries loop without waiting for
     // the wave's full traversals.
     // With the flag false a try whose line misses every emitter ends here
     // without normalising its draws (kScan: in next_try; else D holds the draws
-    // of the try).
+    // of the try).  kScan: a try that needs the emitter tree leaves its query to
+    // the walk below (qstage 6), beside the other lanes' rays.
     while (qstage == 1) {
       if constexpr (kScan) {
         if (hitf) {
@@ -1042,6 +1072,21 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
           if (!alive) break;
           continue;
         }
+        D = hemisphere_dir(D, N);
+        if (!ray_valid(D)) {  // counts as a ray, misses without traversal
+          hitf = false;
+          alive = nee_after(-5);
+        } else if (scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
+          qstage = 6;
+        } else if (!hitf) {
+          alive = nee_after(-5);
+        } else {  // stale hit flag: a miss clears it, any other hit keeps it
+          tE = kTmax;
+          primE = 0xFFFFFFFFu;
+          matE = -1;
+          qstage = 2;
+        }
+        if (!alive) break;
       } else {
         if (kCount) c_occ++;
         if (kRecord) occl_cnt++;
@@ -1050,35 +1095,35 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
           if (!alive) break;
           continue;
         }
+        D = hemisphere_dir(D, N);
+        const bool valid = ray_valid(D);
+        if (kCount && !valid) c_inv++;
+        int32_t k = -1;
+        float t = 0.0f;
+        if (valid && scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
+          const RayT r = make_ray(O, D);
+          k = closest<kCount, kPathBlock>(scp->emit, r, kTmin, kTmax, 0xFFFFFFFFu, false, t, my_stk, spill, tc);
+        }
+        if (!valid) {  // counts as a ray, misses without traversal
+          const int32_t code = hitf ? -1 : -5;
+          hitf = false;
+          alive = nee_after(code);
+        } else if (k >= 0) {  // an emitter: is anything in front of it?
+          const float4 e0 = scp->emit.tris[3 * (size_t)k], e1 = scp->emit.tris[3 * (size_t)k + 1];
+          tE = t;
+          primE = __float_as_uint(e0.w);
+          matE = (int32_t)__float_as_uint(e1.w);
+          qstage = 2;
+        } else if (!hitf) {
+          alive = nee_after(-5);
+        } else {  // stale hit flag: a miss clears it, any other hit keeps it
+          tE = kTmax;
+          primE = 0xFFFFFFFFu;
+          matE = -1;
+          qstage = 2;
+        }
+        if (!alive) break;
       }
-      D = hemisphere_dir(D, N);
-      const bool valid = ray_valid(D);
-      if (kCount && !valid) c_inv++;
-      int32_t k = -1;
-      float t = 0.0f;
-      if (valid && scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
-        const RayT r = make_ray(O, D);
-        k = query(scp->emit, r, kTmax, 0xFFFFFFFFu, false, t);
-      }
-      if (!valid) {  // counts as a ray, misses without traversal
-        const int32_t code = hitf ? -1 : -5;
-        hitf = false;
-        alive = nee_after(code);
-      } else if (k >= 0) {  // an emitter: is anything in front of it?
-        const float4 e0 = scp->emit.tris[3 * (size_t)k], e1 = scp->emit.tris[3 * (size_t)k + 1];
-        tE = t;
-        primE = __float_as_uint(e0.w);
-        matE = (int32_t)__float_as_uint(e1.w);
-        qstage = 2;
-      } else if (!hitf) {
-        alive = nee_after(-5);
-      } else {  // stale hit flag: a miss clears it, any other hit keeps it
-        tE = kTmax;
-        primE = 0xFFFFFFFFu;
-        matE = -1;
-        qstage = 2;
-      }
-      if (!alive) break;
     }
     if (!alive) continue;  // the pixel is written at the top of the loop
     if (kEmit && qstage == 5) {
@@ -1132,9 +1177,9 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
           const float cy = fabsf(dot(nt, w)) / sqrtf(dot(nt, nt));
           const float q = Bsdf::pdf(Din, N, w, 1.0f);  // the bounce's density at roughness 1
           lw = q * cy * pp->emit_area / r2;
-          ls_k = lo;
+          ls_prim = __float_as_uint(p0.w);
           D = w;
-          qstage = 4;  // the emitter query below: is lo the closest emitter?
+          qstage = 4;  // the emitter query below: is it the closest emitter?
         } else {
           D = Bsdf::sample(Din, N, seed, rough);  // p^ = 0
           cond = true;
@@ -1151,35 +1196,23 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
         }
       }
     }
-    if (kEmit && qstage == 4) {
-      // kMode 3's light sample: is the sampled triangle the closest emitter
-      // along the line?  Then its any-hit test (qstage 3), else its bounce.
-      float t = 0.0f;
-      const int32_t k = query(scp->emit, make_ray(O, D), kTmax, 0xFFFFFFFFu, false, t);
-      if (k == ls_k) {
-        const float4 e0 = scp->emit.tris[3 * (size_t)k], e1 = scp->emit.tris[3 * (size_t)k + 1];
-        tE = t;
-        primE = __float_as_uint(e0.w);
-        matE = (int32_t)__float_as_uint(e1.w);
-        qstage = 3;
-      } else {  // p^ = 0
-        D = Bsdf::sample(Din, N, seed, rough);
-        cond = true;
-        rejects = 0;
-        qstage = 0;
-      }
-    }
-
-    // -- one full traversal per iteration: the closest hit of a radiance ray
-    // (qstage 0) or the any-hit query of an occlusion ray (qstage 2).
+    // -- one traversal per iteration: the closest hit of a radiance ray
+    // (qstage 0), the any-hit query of an occlusion ray (qstage 2, 3) or
+    // (kScan) the emitter query of an NEE try or a light sample (qstage 6, 4).
     const bool valid = ray_valid(D);
     int32_t k = -1;
     float t = 0.0f;
     if (valid && scp->all.T > 0) {
       const RayT r = make_ray(O, D);
-      const bool any = qstage >= 2;
-      k = query(scp->all, r, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu, any, t);
+      const bool any = qstage == 2 || (kEmit && qstage == 3);
+      if constexpr (kScan)
+        k = closest_walk<kPathBlock, true>(*scp, qstage >= 4, r, kTmin, any ? tE : kTmax,
+                                           any ? primE : 0xFFFFFFFFu, any, t, my_stk, spill, paused);
+      else
+        k = closest<kCount, kPathBlock>(scp->all, r, kTmin, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu, any, t,
+                                        my_stk, spill, tc);
     }
+    if (kScan && paused) continue;
 
     if (qstage == 0) {
       // radiance: miss (189-194) / closest hit (211-255)
@@ -1273,6 +1306,32 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
       if (finish) {
         finish_sample();
         alive = begin_sample();
+      }
+    } else if (kScan && qstage >= 4) {
+      // the closest emitter of an NEE try (6) or a light sample (4)
+      float4 e0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), e1 = e0;
+      if (k >= 0) {
+        e0 = scp->all.tris[3 * (size_t)k];
+        e1 = scp->all.tris[3 * (size_t)k + 1];
+      }
+      const uint32_t prim = __float_as_uint(e0.w);
+      if (k >= 0 && (qstage == 6 || (kEmit && prim == ls_prim))) {  // is anything in front of it?
+        tE = t;
+        primE = prim;
+        matE = (int32_t)__float_as_uint(e1.w);
+        qstage = qstage == 6 ? 2 : 3;
+      } else if (kEmit && qstage == 4) {  // p^ = 0
+        D = Bsdf::sample(Din, N, seed, rough);
+        cond = true;
+        rejects = 0;
+        qstage = 0;
+      } else if (!hitf) {
+        alive = nee_after(-5);
+      } else {  // stale hit flag: a miss clears it, any other hit keeps it
+        tE = kTmax;
+        primE = 0xFFFFFFFFu;
+        matE = -1;
+        qstage = 2;
       }
     } else if (kEmit && qstage == 3) {
       // the light sample of a prefix bounce: visible unless blocked before (tE, primE)
@@ -1840,6 +1899,7 @@ __device__ __forceinline__ bool wf_advance(const BatchScene* __restrict__ scenes
   const SceneView* scp = &bs->sc;
   const PathArgs* pp = &bs->p;
   volatile uint32_t spill[kStackMax - kStackLds];
+  int32_t paused = 0;
 
   auto finish_sample = [&]() {
     acc = acc + color;
@@ -2005,13 +2065,13 @@ __device__ __forceinline__ bool wf_advance(const BatchScene* __restrict__ scenes
       float t = 0.0f;
       if (valid && scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
         const RayT r = make_ray(O, D);
-        k = closest_walk<kWfBlock>(scp->emit, r, kTmin, kTmax, 0xFFFFFFFFu, false, t, my_stk, spill);
+        k = closest_walk<kWfBlock>(*scp, true, r, kTmin, kTmax, 0xFFFFFFFFu, false, t, my_stk, spill, paused);
       }
       if (!valid) {  // counts as a ray, misses without traversal
         hitf = false;
         alive = nee_after();
       } else if (k >= 0) {  // an emitter: is anything in front of it?
-        const float4 e0 = scp->emit.tris[3 * (size_t)k], e1 = scp->emit.tris[3 * (size_t)k + 1];
+        const float4 e0 = scp->all.tris[3 * (size_t)k], e1 = scp->all.tris[3 * (size_t)k + 1];
         tE = t;
         primE = __float_as_uint(e0.w);
         matE = (int32_t)__float_as_uint(e1.w);
@@ -2829,9 +2889,22 @@ __global__ __launch_bounds__(kAggChunk) void k_agg(const float4* __restrict__ tr
   if (tid == 0) out_cnt[blockIdx.x] = (uint32_t)n;
 }
 
+// The places of the scene's triangles by id, and from these the places of the
+// emitters among them, into the last word of their records.
+__global__ __launch_bounds__(kBuildBlock) void k_place(const uint32_t* __restrict__ prim, int32_t T, uint32_t* place) {
+  const int32_t k = blockIdx.x * kBuildBlock + threadIdx.x;
+  if (k < T) place[prim[k]] = (uint32_t)k;
+}
+__global__ __launch_bounds__(kBuildBlock) void k_link(const uint32_t* __restrict__ prim, int32_t T,
+                                                      const uint32_t* __restrict__ place, float4* tris) {
+  const int32_t k = blockIdx.x * kBuildBlock + threadIdx.x;
+  if (k < T) tris[3 * (size_t)k + 2].w = __uint_as_float(place[prim[k]]);
+}
+
 // Binary nodes that k_agg may write for T triangles: node 0 and kAggChunk - 1
 // per workgroup of every pass.
 inline size_t agg_capacity(int64_t T) {
+  if (T <= 0) return 0;
   size_t n = 1;
   for (int64_t c = (T + kAggChunk - 1) / kAggChunk;; c = (c + kAggGroups - 1) / kAggGroups) {
     n += (size_t)c * (kAggChunk - 1);
@@ -2845,8 +2918,14 @@ inline size_t agg_capacity(int64_t T) {
 // (a float4 each), the four refs, 16 bytes unused.  An empty slot has an
 // inverted box and the ref of the dummy triangle after the last one, which is
 // never hit.
+//
+// The emitters' tree (links: their triangle records, whose last word is the
+// triangle's place among all of the scene's) lies after the scene's in the same
+// node array, from node `first`, and refers to the scene's triangles: one walk
+// serves both by its root.
 __global__ __launch_bounds__(kBuildBlock) void k_walk_nodes(const float4* __restrict__ nodes, uint32_t n_nodes,
-                                                            int32_t T, float4* __restrict__ walk) {
+                                                            int32_t T, const float4* __restrict__ links,
+                                                            uint32_t first, float4* __restrict__ walk) {
   const uint32_t n = blockIdx.x * kBuildBlock + threadIdx.x;
   if (n >= n_nodes) return;
   const float4* np = nodes + 4 * (size_t)n;
@@ -2890,7 +2969,14 @@ __global__ __launch_bounds__(kBuildBlock) void k_walk_nodes(const float4* __rest
     for (int a = 0; a < 3; ++a) lo[step][a] = l1[a], hi[step][a] = h1[a];
     ref[step] = c1;
   }
-  float4* w = walk + 8 * (size_t)n;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    if (!(ref[s] & kLeaf))
+      ref[s] += first;
+    else if (links && ref[s] != (kLeaf | (uint32_t)T))
+      ref[s] = kLeaf | __float_as_uint(links[3 * (size_t)(ref[s] & ~kLeaf) + 2].w);
+  }
+  float4* w = walk + 8 * ((size_t)first + n);
   for (int a = 0; a < 3; ++a) {
     w[2 * a] = make_float4(lo[0][a], lo[1][a], lo[2][a], lo[3][a]);
     w[2 * a + 1] = make_float4(hi[0][a], hi[1][a], hi[2][a], hi[3][a]);
@@ -2915,8 +3001,9 @@ struct DevBvh {
   int32_t* parent = nullptr;      // parent of each internal node (kept for refits)
   int32_t* leaf_parent = nullptr; // parent of each leaf
   uint2* range = nullptr;         // sorted leaves [lo, hi] of each internal node (kept for refits)
-  // the walk tree (null: none): 4-wide nodes, the binary nodes they come
-  // from, and k_agg's cluster lists and counts (kept for vertex updates)
+  // the walk tree (null: none): 4-wide nodes (the emitters' in the scene's
+  // array), the binary nodes they come from, and k_agg's cluster lists and
+  // counts (kept for vertex updates)
   float4* walk = nullptr;
   float4* agg = nullptr;
   float4* lists = nullptr;
@@ -3214,11 +3301,12 @@ SceneView view(const lisa_ctx* c) {
   const bool finite = std::isfinite(c->span);
   auto walk = [&](const DevBvh& b) { return finite ? reinterpret_cast<const char*>(b.walk) : nullptr; };
   return SceneView{BvhView{c->all.nodes, c->all.tris, c->all.T, c->all.wide, walk(c->all), c->span},
-                   BvhView{c->emit.nodes, c->emit.tris, c->emit.T, nullptr, walk(c->emit), c->span},
+                   BvhView{c->emit.nodes, c->emit.tris, c->emit.T, nullptr, nullptr, c->span},
                    c->d_nrm,
                    c->d_mats,
                    make_float4(c->ecull_c[0], c->ecull_c[1], c->ecull_c[2], 0.0f),
-                   make_float4(c->ecull_h[0], c->ecull_h[1], c->ecull_h[2], 0.0f)};
+                   make_float4(c->ecull_h[0], c->ecull_h[1], c->ecull_h[2], 0.0f),
+                   (uint32_t)agg_capacity(c->all.T)};
 }
 
 // Device scratch freed at scope exit.
@@ -3321,30 +3409,62 @@ lisa_status wide_nodes(lisa_ctx* ctx, DevBvh& b, hipStream_t st) {
   return LISA_OK;
 }
 
-// The walk tree of b (whose triangle records are in place), enqueued on st: no
-// allocation, no wait.
-lisa_status build_walk(lisa_ctx* ctx, DevBvh& b, hipStream_t st) {
-  if (!b.walk || b.T == 0) return LISA_OK;
-  int32_t chunks = (b.T + kAggChunk - 1) / kAggChunk;
-  // two sets of lists in turn
-  const size_t half = (size_t)chunks * kAggOut * 2;
-  const float4* in = nullptr;
-  const uint32_t* in_cnt = nullptr;
-  int32_t n_in = 0;
-  uint32_t base = 1;
-  for (int pass = 0;; ++pass) {
-    float4* out = b.lists + (pass & 1 ? half : 0);
-    uint32_t* out_cnt = b.counts + (pass & 1 ? (b.T + kAggChunk - 1) / kAggChunk : 0);
-    k_agg<<<chunks, kAggChunk, 0, st>>>(b.tris, b.T, in, in_cnt, n_in, base, b.agg, out, out_cnt);
-    if (chunks == 1) break;
-    base += (uint32_t)chunks * (kAggChunk - 1);
-    in = out;
-    in_cnt = out_cnt;
-    n_in = chunks;
-    chunks = (chunks + kAggGroups - 1) / kAggGroups;
+// The walk trees of the scene and of its emitters (their triangle records are
+// in place and linked), enqueued on the context's stream: no allocation, no wait.
+lisa_status build_walk(lisa_ctx* ctx) {
+  hipStream_t st = ctx->stream;
+  DevBvh &all = ctx->all, &emit = ctx->emit;
+  if (!all.walk) return LISA_OK;
+  for (DevBvh* b : {&all, &emit}) {
+    if (b->T == 0) continue;
+    const int32_t chunks0 = (b->T + kAggChunk - 1) / kAggChunk;
+    int32_t chunks = chunks0, n_in = 0;
+    const float4* in = nullptr;
+    const uint32_t* in_cnt = nullptr;
+    uint32_t base = 1;
+    for (int pass = 0;; ++pass) {  // two sets of lists in turn
+      float4* out = b->lists + (pass & 1 ? (size_t)chunks0 * kAggOut * 2 : 0);
+      uint32_t* out_cnt = b->counts + (pass & 1 ? chunks0 : 0);
+      k_agg<<<chunks, kAggChunk, 0, st>>>(b->tris, b->T, in, in_cnt, n_in, base, b->agg, out, out_cnt);
+      if (chunks == 1) break;
+      base += (uint32_t)chunks * (kAggChunk - 1);
+      in = out;
+      in_cnt = out_cnt;
+      n_in = chunks;
+      chunks = (chunks + kAggGroups - 1) / kAggGroups;
+    }
+    const uint32_t cap = (uint32_t)agg_capacity(b->T);
+    k_walk_nodes<<<grid_for(cap, kBuildBlock), kBuildBlock, 0, st>>>(
+        b->agg, cap, all.T, b == &emit ? emit.tris : nullptr, b == &emit ? (uint32_t)agg_capacity(all.T) : 0u,
+        all.walk);
   }
-  const uint32_t cap = (uint32_t)agg_capacity(b.T);
-  k_walk_nodes<<<grid_for(cap, kBuildBlock), kBuildBlock, 0, st>>>(b.agg, cap, b.T, b.walk);
+  HIP_TRY(ctx, hipGetLastError());
+  return LISA_OK;
+}
+
+// Memory of the walk trees, and the emitters' places among the scene's
+// triangles (enqueued; `place` is T words of scratch).
+lisa_status prepare_walk(lisa_ctx* ctx, uint32_t* place) {
+  hipStream_t st = ctx->stream;
+  DevBvh &all = ctx->all, &emit = ctx->emit;
+  const size_t nodes = agg_capacity(all.T) + agg_capacity(emit.T);
+  if (all.T == 0 || nodes > kWalkMaxNodes) return LISA_OK;
+  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&all.walk), 128 * nodes));
+  all.bytes += 128 * nodes;
+  for (DevBvh* b : {&all, &emit}) {
+    if (b->T == 0) continue;
+    const size_t cap = agg_capacity(b->T), chunks = ((size_t)b->T + kAggChunk - 1) / kAggChunk;
+    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b->agg), 64 * cap));
+    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b->lists), 64 * chunks * kAggOut));
+    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b->counts), 8 * chunks));
+    b->bytes += 64 * cap + 64 * chunks * kAggOut + 8 * chunks;
+    HIP_TRY(ctx, hipMemsetAsync(b->agg, 0xFF, 64 * cap, st));  // refs kEmpty: indexes that k_agg leaves out
+  }
+  HIP_TRY(ctx, hipMemsetAsync(all.tris + 3 * (size_t)all.T, 0, 48, st));  // the dummy triangle of empty slots
+  if (emit.T > 0) {
+    k_place<<<grid_for(all.T, kBuildBlock), kBuildBlock, 0, st>>>(all.prim, all.T, place);
+    k_link<<<grid_for(emit.T, kBuildBlock), kBuildBlock, 0, st>>>(emit.prim, emit.T, place, emit.tris);
+  }
   HIP_TRY(ctx, hipGetLastError());
   return LISA_OK;
 }
@@ -3374,16 +3494,6 @@ lisa_status build_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
   b.bytes += nodes_b + tris_b + 16 * (size_t)std::max(n, 1);
   HIP_TRY(ctx, hipMemsetAsync(b.nodes, 0, nodes_b, st));
   if (n == 0) return LISA_OK;
-  if (agg_capacity(n) <= kWalkMaxNodes) {
-    const size_t cap = agg_capacity(n), chunks = ((size_t)n + kAggChunk - 1) / kAggChunk;
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.walk), 128 * cap));
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.agg), 64 * cap));
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.lists), 64 * chunks * kAggOut));
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.counts), 8 * chunks));
-    b.bytes += 192 * cap + 64 * chunks * kAggOut + 8 * chunks;
-    HIP_TRY(ctx, hipMemsetAsync(b.agg, 0xFF, 64 * cap, st));  // refs kEmpty: indexes that k_agg leaves out
-    HIP_TRY(ctx, hipMemsetAsync(b.tris + 3 * (size_t)n, 0, 48, st));  // the dummy triangle of empty slots
-  }
   Scratch S;
   float *d_part = nullptr, *d_bounds = nullptr;
   int32_t *d_parent = b.parent, *d_leafp = b.leaf_parent;
@@ -3422,7 +3532,6 @@ lisa_status build_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
     if (rc != LISA_OK) return rc;
   }
   lisa_status rw = wide_nodes(ctx, b, st);
-  if (rw == LISA_OK) rw = build_walk(ctx, b, st);
   if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipGetLastError());
   // scratch is freed on return: wait for the kernels that use it
@@ -3443,7 +3552,6 @@ lisa_status refit_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
     if (rc != LISA_OK) return rc;
   }
   lisa_status rw = wide_nodes(ctx, b, st);
-  if (rw == LISA_OK) rw = build_walk(ctx, b, st);
   if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipStreamSynchronize(st));
   HIP_TRY(ctx, hipGetLastError());
@@ -3767,6 +3875,7 @@ lisa_status lisa_update_vertices(lisa_ctx* ctx, const float* verts, const float*
   HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
   lisa_status rc = refit_bvh(ctx, ctx->all, d_v, d_n, ctx->d_nrm);
   if (rc == LISA_OK) rc = refit_bvh(ctx, ctx->emit, d_v, nullptr, nullptr);
+  if (rc == LISA_OK) rc = build_walk(ctx);
   if (rc != LISA_OK) return rc;
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
   HIP_TRY(ctx, hipStreamSynchronize(st));
@@ -3805,9 +3914,10 @@ lisa_status lisa_update_vertices_noalloc(lisa_ctx* ctx, const float* d_verts, co
       if (rc != LISA_OK) return rc;
     }
     lisa_status rw = wide_nodes(ctx, *b, st);
-    if (rw == LISA_OK) rw = build_walk(ctx, *b, st);
     if (rw != LISA_OK) return rw;
   }
+  lisa_status rw = build_walk(ctx);
+  if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipGetLastError());
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
   HIP_TRY(ctx, hipStreamSynchronize(st));
@@ -3952,6 +4062,10 @@ lisa_status lisa_set_scene(lisa_ctx* ctx, const float* verts, const float* norma
                              (int64_t)T >= ctx->wide_min_tris);
   if (rc == LISA_OK)
     rc = build_bvh(ctx, ctx->emit, d_v, d_n, d_mat, d_gid, (int32_t)emit_ids.size(), nullptr);
+  uint32_t* d_place = nullptr;
+  if (rc == LISA_OK) HIP_TRY(ctx, S.alloc(&d_place, (size_t)T));
+  if (rc == LISA_OK) rc = prepare_walk(ctx, d_place);
+  if (rc == LISA_OK) rc = build_walk(ctx);
   if (rc != LISA_OK) return rc;
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
   HIP_TRY(ctx, hipStreamSynchronize(st));
