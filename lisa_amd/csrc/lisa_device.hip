@@ -245,39 +245,106 @@ __device__ __forceinline__ bool line_culled(float4 c, float4 H, F3 O, F3 d) {
   if (fabsf(vx * d.y - vy * d.x) > H.x * ay + H.y * ax) return true;
   return false;
 }
-// The next try of an NEE loop whose line is not culled: draws tries (three
-// LCG steps each) until line_culled() lets one through or kNeeTries are made.
-// True: `raw` holds its draws, as hemisphere_raw gives them.  False: all are
-// made.  The draws stay integers k - 2^23 (raw times 2^23, exact): the state
-// with bit 23 flipped is (k - 2^23) mod 2^24 and steps by the same recurrence,
-// so a draw is a multiply-add, a sign extension and a conversion.  The products
-// of a test are fused (one rounding each instead of two, within the margin), and
-// its three axes run without branches: nearly every vertex makes all of its
-// tries, and a wave makes them together (C2 at 32 spp 44.5 -> 40.4 ms, Cornell box
-// of 1k triangles at 256^2, 16 spp 5.4 -> 4.6 ms, with lcg24).
-__device__ __forceinline__ bool next_try(float4 c, float4 H, F3 O, uint32_t& seed, int32_t& tries, F3& raw) {
-  const float vx = c.x - O.x, vy = c.y - O.y, vz = c.z - O.z;
-  uint32_t t = seed ^ 0x800000u;
-  float x, y, z;
-  bool culled;
+// Whether an NEE try is culled by its line (line_culled).  `t` is the LCG state
+// before its draws with bit 23 flipped, which is the state - 2^23 mod 2^24 and
+// steps by the same recurrence, and is left after them: the draws come as
+// integers k - 2^23 (hemisphere_raw's times 2^23, exact), a multiply-add, a sign
+// extension and a conversion each.  The products of a test are fused (one
+// rounding each instead of two, within the margin), its three axes run without
+// branches.  (vx, vy, vz): the box's centre from the vertex; H: its half extents.
+__device__ __forceinline__ bool try_culled(float vx, float vy, float vz, float4 H, uint32_t& t) {
   auto draw = [&]() {
     t = lcg24(t);
     return (float)((int32_t)(t << 8) >> 8);
   };
-  do {
-    x = draw();
-    y = draw();
-    z = draw();
-    const float ax = fabsf(x), ay = fabsf(y), az = fabsf(z);
-    const float px = __builtin_fmaf(vy, z, -(vz * y)), py = __builtin_fmaf(vz, x, -(vx * z)),
-                pz = __builtin_fmaf(vx, y, -(vy * x));
-    const float qx = __builtin_fmaf(H.y, az, H.z * ay), qy = __builtin_fmaf(H.z, ax, H.x * az),
-                qz = __builtin_fmaf(H.x, ay, H.y * ax);
-    culled = ((fabsf(px) > qx) | (fabsf(py) > qy) | (fabsf(pz) > qz)) & (fminf(fminf(ax, ay), az) != 0.0f);
-  } while (culled && ++tries < kNeeTries);
-  seed = t ^ 0x800000u;
-  raw = mk(x, y, z) * 0x1p-23f;
-  return !culled;
+  const float x = draw(), y = draw(), z = draw();
+  const float ax = fabsf(x), ay = fabsf(y), az = fabsf(z);
+  const float px = __builtin_fmaf(vy, z, -(vz * y)), py = __builtin_fmaf(vz, x, -(vx * z)),
+              pz = __builtin_fmaf(vx, y, -(vy * x));
+  const float qx = __builtin_fmaf(H.y, az, H.z * ay), qy = __builtin_fmaf(H.z, ax, H.x * az),
+              qz = __builtin_fmaf(H.x, ay, H.y * ax);
+  return ((fabsf(px) > qx) | (fabsf(py) > qy) | (fabsf(pz) > qz)) & (fminf(fminf(ax, ay), az) != 0.0f);
+}
+
+// kTryJump[j]: 3 j steps of the LCG (j tries) as one, s -> x s + y mod 2^24.
+struct TryJumps {
+  uint2 j[32];
+};
+constexpr TryJumps make_try_jumps() {
+  TryJumps t{};
+  uint32_t a = 1, c = 0;
+  for (int j = 0; j < 32; ++j) {
+    t.j[j].x = a;
+    t.j[j].y = c;
+    for (int k = 0; k < 3; ++k) {
+      a = (a * 1664525u) & 0xFFFFFFu;
+      c = (c * 1664525u + 1013904223u) & 0xFFFFFFu;
+    }
+  }
+  return t;
+}
+__device__ const TryJumps kTryJumps = make_try_jumps();
+static_assert(kNeeTries <= 31, "a half wave makes a vertex's tries at once");
+
+// The lanes with `scan` go to their next NEE try that is not culled, or past
+// their last one: tries and seed are advanced past the culled ones, and the
+// result says whether there is a try left (its draws are next in seed).  Every
+// lane of the wave calls it.
+//
+// Nearly every vertex makes all of its tries, but a wave reaches here with 10 to
+// 15 vertices: each half wave then makes all tries of one vertex at once, from
+// the LCG states 3 j steps on, and the first that is not culled is a bit scan of
+// the ballot.  A pass costs about two tries and serves two vertices (C2 at 32 spp
+// 29.1 -> 25.4 ms, Cornell box of 1k triangles 256^2, 16 spp 4.26 -> 3.66).  With more than kNeeSerial vertices every lane
+// makes its own tries in turn (`shared` false: always, where the lanes' scenes
+// may differ).
+constexpr int kNeeSerial = 30;  // 16 measured 5 % slower on C2; 64 (never in turn) the same
+template <bool shared>
+__device__ __forceinline__ bool nee_scan(bool scan, float4 c, float4 H, F3 O, uint32_t& seed, int32_t& tries) {
+  uint64_t m = __ballot(scan);
+  const float vx = c.x - O.x, vy = c.y - O.y, vz = c.z - O.z;
+  const uint32_t t = seed ^ 0x800000u;
+  bool found = false;
+  if (!shared || __popcll(m) > kNeeSerial) {
+    if (scan) {
+      uint32_t u = t, at = t;
+      while (tries < kNeeTries && try_culled(vx, vy, vz, H, u)) {
+        at = u;
+        ++tries;
+      }
+      found = tries < kNeeTries;
+      seed = at ^ 0x800000u;
+    }
+    return found;
+  }
+  if (m == 0) return false;
+  const int lane = (int)__lane_id(), j = lane & 31;
+  const uint2 jump = kTryJumps.j[j];
+  const uint32_t pack = (t & 0xFFFFFFu) | ((uint32_t)tries << 24);
+  int32_t adv = 0;
+  while (m) {
+    const int i0 = __ffsll((unsigned long long)m) - 1;
+    m &= m - 1;
+    const int i1 = m ? __ffsll((unsigned long long)m) - 1 : i0;
+    m &= m - 1;
+    const int src = lane < 32 ? i0 : i1;
+    const float sx = __shfl(vx, src), sy = __shfl(vy, src), sz = __shfl(vz, src);
+    const uint32_t w = __shfl(pack, src);
+    uint32_t u = __umul24(w, jump.x) + jump.y;
+    const bool left = !try_culled(sx, sy, sz, H, u) && j + (int)(w >> 24) < kNeeTries;
+    const uint64_t b = __ballot(left);
+    if (lane == i0 || lane == i1) {
+      const uint32_t h = lane == i0 ? (uint32_t)b : (uint32_t)(b >> 32);
+      found = h != 0;
+      adv = found ? __ffs((int)h) - 1 : kNeeTries - tries;
+    }
+  }
+  if (scan) {
+    tries += adv;
+    const uint2 g = kTryJumps.j[adv];
+    seed = (__umul24(t, g.x) + g.y) ^ 0x800000u;
+  }
+  return found;
 }
 // emit_culled: the ray misses the box -- the box lies behind the origin along
 // an axis the ray moves away on, or the ray's line misses it.
@@ -551,13 +618,14 @@ __device__ __forceinline__ int32_t closest_wide(const BvhView& bv, const RayT& r
 // 1024^2: C2 67.5 -> 44.5 ms; icosphere of 1.3M triangles, 1080p, 16 spp:
 // 85.6 -> 53.8 ms (before: its 4-wide Morton walk).
 //
-// Pausing (kPause): once no more than a quarter of the lanes that entered are
-// left walking, each of these puts its walk on its stack and leaves with
+// Pausing (kPause): once no more than half of the lanes that entered are left
+// walking, each of these puts its walk on its stack and leaves with
 // paused != 0; the same query called again (paused as left) goes on from there.
 // The caller gives the finished lanes their next rays in between.  Without it 76 %
 // of the walk's iterations on C2 ran for 16 lanes or fewer (14 of 64 walking on
 // average, 38 with it), for 1.6 times as many rounds of the path loop (C2 at
-// 32 spp 38.4 -> 29.1 ms).  An eighth of the lanes 29.8, a half 29.7 ms.
+// 32 spp 38.4 -> 29.1 ms).  The share of the lanes, with nee_scan: a quarter 25.4,
+// 3 / 8 25.1, a half 25.1 ms; icosphere of 1.3M triangles 33.5, 31.6, 30.7 ms.
 template <int kStride, bool kPause = false>
 __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitters, const RayT& r, float tmin,
                                                 float tlim, uint32_t lim_prim, bool any, float& t_out,
@@ -593,7 +661,7 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
     } else {
       stk[0] = kEmpty;  // popped last: the end of the walk
     }
-    if (kPause) quorum = __popcll(__ballot(1)) / 4;
+    if (kPause) quorum = __popcll(__ballot(1)) / 2;
     done = true;
     for (;;) {
       if (kPause && __popcll(__ballot(1)) <= quorum && cur != kEmpty) {
@@ -847,8 +915,12 @@ struct Job {
 // running mean over subframes; the subframe then only picks the RNG stream).
 template <bool kRecord, bool kCount, class Src, int kMode = 0, bool kF64 = false, class Bsdf = LISA_BSDF>
 __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
-  Job job;
-  if (!src.next(job)) return;
+  constexpr bool kScan = !kCount && !kRecord;  // culled NEE tries by nee_scan, none seen one by one
+  Job job{0, 0, 0};
+  // kScan: a lane without work stays to help with the others' tries until the
+  // whole wave is done
+  bool idle = !src.next(job);
+  if (kScan ? !__ballot(!idle) : idle) return;
   const SceneView* scp = src.view();  // the current pixel's scene and launch
   const PathArgs* pp = src.args();
   uint32_t x = job.x, y = job.y;
@@ -886,7 +958,6 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   int32_t occl_cnt = 0;
   size_t rec_base = (size_t)item * pp->spp;
 
-  constexpr bool kScan = !kCount && !kRecord;  // culled NEE tries by next_try, none seen one by one
   constexpr bool kQuery = kMode == 1 || kMode == 3;  // ends at the cache query
   constexpr bool kEmit = kMode == 3;                 // prefix emission in expectation
   static_assert(kScan || !kEmit, "kMode 3 leaves the draws of a try to the NEE loop");
@@ -1034,11 +1105,14 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     if (kCount) c_px++;
   };
 
-  bool alive = begin_sample();
+  bool alive = !idle && begin_sample();
   for (;;) {
-    if (!alive) {
+    while (!alive && !idle) {
       write_pixel();
-      if (!src.next(job)) break;
+      if (!src.next(job)) {
+        idle = true;
+        break;
+      }
       scp = src.view();
       pp = src.args();
       x = job.x;
@@ -1052,42 +1126,43 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
       s = 0;
       rec_base = (size_t)item * pp->spp;
       alive = begin_sample();
-      continue;
     }
+    if (kScan ? !__ballot(!idle) : idle) break;
     // -- NEE occlusion rays, first query: the closest emitter (emitter tree).
     // A miss and a non-emitting closest hit both leave a false hit flag
     // false (shader.cu:172-184), so with the flag false a ray that hits no
     // emitter is resolved here; these cheap tries loop without waiting for
     // the wave's full traversals.
     // With the flag false a try whose line misses every emitter ends here
-    // without normalising its draws (kScan: in next_try; else D holds the draws
+    // without normalising its draws (kScan: in nee_scan; else D holds the draws
     // of the try).  kScan: a try that needs the emitter tree leaves its query to
     // the walk below (qstage 6), beside the other lanes' rays.
-    while (qstage == 1) {
-      if constexpr (kScan) {
-        if (hitf) {
-          D = hemisphere_raw(seed);
-        } else if (!next_try(scp->ecull_c, scp->ecull_h, O, seed, tries, D)) {
+    if constexpr (kScan) {
+      for (;;) {
+        const bool want = alive && qstage == 1;
+        if (!__ballot(want)) break;
+        const bool found = nee_scan<Src::kOneScene>(want && !hitf, scp->ecull_c, scp->ecull_h, O, seed, tries);
+        if (want && !hitf && !found) {
           alive = end_nee(mk(0.0f, 0.0f, 0.0f));
-          if (!alive) break;
-          continue;
+        } else if (want) {
+          D = hemisphere_dir(hemisphere_raw(seed), N);
+          if (!ray_valid(D)) {  // counts as a ray, misses without traversal
+            hitf = false;
+            alive = nee_after(-5);
+          } else if (scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
+            qstage = 6;
+          } else if (!hitf) {
+            alive = nee_after(-5);
+          } else {  // stale hit flag: a miss clears it, any other hit keeps it
+            tE = kTmax;
+            primE = 0xFFFFFFFFu;
+            matE = -1;
+            qstage = 2;
+          }
         }
-        D = hemisphere_dir(D, N);
-        if (!ray_valid(D)) {  // counts as a ray, misses without traversal
-          hitf = false;
-          alive = nee_after(-5);
-        } else if (scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
-          qstage = 6;
-        } else if (!hitf) {
-          alive = nee_after(-5);
-        } else {  // stale hit flag: a miss clears it, any other hit keeps it
-          tE = kTmax;
-          primE = 0xFFFFFFFFu;
-          matE = -1;
-          qstage = 2;
-        }
-        if (!alive) break;
-      } else {
+      }
+    } else {
+      while (qstage == 1) {
         if (kCount) c_occ++;
         if (kRecord) occl_cnt++;
         if (!hitf && line_culled(scp->ecull_c, scp->ecull_h, O, D)) {
@@ -1379,6 +1454,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
 // One pixel per work-item: the listed pixels, or the full image in
 // kTileW x kTileH tiles.
 struct OnePixel {
+  static constexpr bool kOneScene = true;
   SceneView sc;
   PathArgs p;
   bool given;
@@ -1427,6 +1503,7 @@ __global__ __launch_bounds__(kPathBlock, kMode == 3 ? LISA_EMIT_WAVES : LISA_MOD
 // together share one atomic.  Lanes whose paths end early pull more pixels
 // instead of idling behind the wave's longest path.
 struct PixelQueue {
+  static constexpr bool kOneScene = true;
   SceneView sc;
   PathArgs p;
   uint32_t* counter;
@@ -1560,6 +1637,7 @@ struct BatchScene {
 };
 
 struct QueueSrc {
+  static constexpr bool kOneScene = false;
   const BatchScene* __restrict__ scenes;
   int32_t n_scenes;
   uint32_t* counter;
@@ -1620,6 +1698,7 @@ __global__ __launch_bounds__(kPathBlock) void k_path_queue(const BatchScene* sce
 // tile's scene is the same for the whole wave, so its pointers and launch
 // constants are scalar; lanes whose pixel is done wait for the tile.
 struct TileSrc {
+  static constexpr bool kOneScene = true;
   const BatchScene* bs;  // wave-uniform: its fields are read through scalar loads
   uint32_t tile;
   bool given;
