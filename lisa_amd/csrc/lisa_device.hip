@@ -58,11 +58,11 @@ constexpr int kNeeTries = 30;   // shader.cu:199
 #define LISA_PATH_BLOCK 64
 #endif
 // Waves per SIMD the path kernels are compiled for: 5 (96 VGPRs).  The walk of
-// the 4-wide tree holds a node's 28 words at once; at 6 waves (80 VGPRs) k_path
-// spills 23 registers around it and C2 (32 spp) takes 38.4 ms against 37.2, at 4
-// (101 VGPRs, no spill) 40.3.  The query kernel with the light samples carries
-// more state: 4 (at 5 it spills 95 registers).  The counting and recording builds run at 4, and
-// the batched lane-queue form keeps the registers it needs.
+// the 4-wide tree holds a node's 28 words at once; k_path spills 7 registers
+// around it.  At 4 (no spill) C2 (32 spp) takes 25.1 ms against 22.7, and the query
+// kernel with the light samples (22 spills at 5) 2 % longer per cached frame.
+// The counting and recording builds run at 4, and the batched lane-queue form
+// keeps the registers it needs.
 #ifndef LISA_PATH_MIN_BLOCKS
 #define LISA_PATH_MIN_BLOCKS 5
 #endif
@@ -70,7 +70,7 @@ constexpr int kNeeTries = 30;   // shader.cu:199
 #define LISA_MODE_WAVES 5  // the cache-mode path kernels
 #endif
 #ifndef LISA_EMIT_WAVES
-#define LISA_EMIT_WAVES 4  // the query kernel with the prefix-emission light samples
+#define LISA_EMIT_WAVES 5  // the query kernel with the prefix-emission light samples
 #endif
 #ifndef LISA_TILE_WAVES
 #define LISA_TILE_WAVES 5  // the batched wave-tile form
@@ -894,6 +894,21 @@ struct Job {
   int32_t item;
 };
 
+// What a lane of the path loop does next.
+enum Stage : int32_t {
+  kRay = 0,        // a radiance ray
+  kTry = 1,        // the next NEE try
+  kAny = 2,        // an NEE try's any-hit query
+  kLightAny = 3,   // kMode 3: a light sample's any-hit query
+  kLightEmit = 4,  // kMode 3: a light sample's emitter query
+  kNeeEnd = 5,     // the end of an NEE loop
+  kTryEmit = 6,    // kScan: an NEE try's emitter query
+  kBounce = 7,     // kMode 3: a bounce drawn on the condition that it hits no emitter
+  kSampleEnd = 8,  // the sample is complete
+  kNext = 9,       // the next sample, or the next pixel
+  kIdle = 10       // no work left
+};
+
 // The per-lane path loop over the pixels a source hands out.  `src.view()`
 // and `src.args()` point at the scene and launch of the current pixel (read
 // again after every `src.next(j)`, which gives the lane its next pixel;
@@ -917,10 +932,8 @@ template <bool kRecord, bool kCount, class Src, int kMode = 0, bool kF64 = false
 __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   constexpr bool kScan = !kCount && !kRecord;  // culled NEE tries by nee_scan, none seen one by one
   Job job{0, 0, 0};
-  // kScan: a lane without work stays to help with the others' tries until the
-  // whole wave is done
-  bool idle = !src.next(job);
-  if (kScan ? !__ballot(!idle) : idle) return;
+  const bool work = src.next(job);
+  if (!__ballot(work)) return;
   const SceneView* scp = src.view();  // the current pixel's scene and launch
   const PathArgs* pp = src.args();
   uint32_t x = job.x, y = job.y;
@@ -944,8 +957,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
   // of the NEE rays and of the next bounce).
   F3 O = mk(0.0f, 0.0f, 0.0f), D = O, color = O, att = O, N = O, Din = O;
   bool hitf = false;
-  // 0 radiance ray, 1 NEE try, 6 its emitter query (kScan), 2 its any-hit query
-  int32_t qstage = 0;
+  int32_t stage = kNext;
   int32_t tries = 0, matE = -1;
   // RayState::material of the NEE's light (shader.cu:38), in LDS after acc
   int32_t* const light_mat = reinterpret_cast<int32_t*>(my_stk + (kStackRows + 3) * kPathBlock);
@@ -1009,67 +1021,46 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     }
     ++s;
   };
-  // The camera ray of the next sample (shader.cu:147-152); samples with no
-  // bounce finish at once.  False when the pixel has no sample left.
-  auto begin_sample = [&]() -> bool {
-    while (s < pp->spp) {
-      const float jx = rng(seed);
-      const float jy = rng(seed);
-      const float dx = (2.0f * (float)x + jx) / (float)pp->width - 1.0f;
-      const float dy = (2.0f * (float)y + jy) / (float)pp->height - 1.0f;
-      D = normalize(dx * pp->U + dy * pp->V + pp->W);
-      O = pp->eye;
-      color = mk(0.0f, 0.0f, 0.0f);
-      att = mk(1.0f, 1.0f, 1.0f);
-      hitf = false;
-      qstage = 0;
-      b = 0;
-      if (kEmit) cond = false;
-      if (kRecord) {
-        hash = 2166136261u;
-        occl_cnt = 0;
-        if (pp->rad_hits)
-          for (int32_t q = 0; q < pp->rb; ++q) pp->rad_hits[(rec_base + s) * pp->rb + q] = -3;
-      }
-      if (pp->bounces > 0) return true;
-      finish_sample();
+  // The camera ray of the next sample (shader.cu:147-152); a sample with no
+  // bounce ends at once.
+  auto begin_sample = [&]() {
+    const float jx = rng(seed);
+    const float jy = rng(seed);
+    const float dx = (2.0f * (float)x + jx) / (float)pp->width - 1.0f;
+    const float dy = (2.0f * (float)y + jy) / (float)pp->height - 1.0f;
+    D = normalize(dx * pp->U + dy * pp->V + pp->W);
+    O = pp->eye;
+    color = mk(0.0f, 0.0f, 0.0f);
+    att = mk(1.0f, 1.0f, 1.0f);
+    hitf = false;
+    b = 0;
+    if (kEmit) cond = false;
+    if (kRecord) {
+      hash = 2166136261u;
+      occl_cnt = 0;
+      if (pp->rad_hits)
+        for (int32_t q = 0; q < pp->rb; ++q) pp->rad_hits[(rec_base + s) * pp->rb + q] = -3;
     }
-    return false;
+    stage = pp->bounces > 0 ? kRay : kSampleEnd;
   };
-  // End of one shoot_ray_to_light: add its light, sample the BSDF for the
-  // next bounce (shader.cu:251-252), end the sample after the last bounce.
-  auto end_nee = [&](F3 nee) -> bool {
-    if (kEmit) {
-      // kMode 3: the light of one NEE run (the mean of nee_loops runs at the
-      // camera ray's hit, nee_loops_deep at later vertices, each added as it
-      // ends); the rest of the vertex follows the NEE loop below
-      // (qstage 5), in one place for every way a run ends
-      const int32_t runs = b > 1 ? pp->nee_loops_deep : pp->nee_loops;
-      if (runs > 1)
-        color = color + (nee * (1.0f / (float)runs)) * att;
-      else
-        color = color + nee * att;
-      qstage = 5;
-      return true;
-    }
-    color = color + nee * att;
-    D = Bsdf::sample(Din, N, seed, rough);
-    qstage = 0;
-    if (b == pp->bounces) {
-      finish_sample();
-      return begin_sample();
-    }
-    return true;
-  };
-  // One occlusion ray resolved (record `code`): return the light, try again,
-  // or give up after kNeeTries (shader.cu:200-208).
-  auto nee_after = [&](int32_t code) -> bool {
+  // One occlusion ray resolved (record `code`): the loop's end with a light or
+  // after kNeeTries, or the next try (shader.cu:200-208).
+  auto nee_after = [&](int32_t code) {
     if (kRecord) hash = (hash ^ ((uint32_t)code ^ 0x5bd1e995u)) * 16777619u;
-    if (hitf) return end_nee(xyz(scp->mats[*light_mat].emission_emit) * Bsdf::eval(N, D));
-    if (++tries == kNeeTries) return end_nee(mk(0.0f, 0.0f, 0.0f));
-    if (!kScan) D = hemisphere_raw(seed);  // finished in the emitter-query loop
-    qstage = 1;
-    return true;
+    stage = hitf || ++tries == kNeeTries ? kNeeEnd : kTry;
+    if (!kScan && stage == kTry) D = hemisphere_raw(seed);  // finished in the emitter-query loop
+  };
+  // A try whose ray hits no emitter: with the flag false that resolves it; with
+  // a stale flag a miss clears it and any other hit keeps it.
+  auto no_emitter = [&]() {
+    if (!hitf) {
+      nee_after(-5);
+    } else {
+      tE = kTmax;
+      primE = 0xFFFFFFFFu;
+      matE = -1;
+      stage = kAny;
+    }
   };
 
   // shader.cu:156-166: the pixel's mean (and running mean over subframes).
@@ -1105,29 +1096,29 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     if (kCount) c_px++;
   };
 
-  bool alive = !idle && begin_sample();
+  auto begin_pixel = [&]() {
+    scp = src.view();
+    pp = src.args();
+    x = job.x;
+    y = job.y;
+    item = job.item;
+    seed = tea16(y * pp->width + x, pp->subframe);
+    acc[0] = 0.0f;
+    acc[kPathBlock] = 0.0f;
+    acc[2 * kPathBlock] = 0.0f;
+    ad0 = ad1 = ad2 = 0.0;
+    s = 0;
+    rec_base = (size_t)item * pp->spp;
+  };
+
+  if (!work) stage = kIdle;
+  // One round: the NEE tries, the ends of NEE loops, the next samples and pixels,
+  // one traversal, its result.  Each is written once, however a lane gets there,
+  // and every lane of the wave goes through all of it until the last is idle (the
+  // idle ones help with the others' tries).  Written out at each place where an
+  // NEE loop, a sample or a pixel can end, they cost 22 spilled registers instead
+  // of 7 and 10 % of C2 (25.1 against 22.7 ms at 32 spp).
   for (;;) {
-    while (!alive && !idle) {
-      write_pixel();
-      if (!src.next(job)) {
-        idle = true;
-        break;
-      }
-      scp = src.view();
-      pp = src.args();
-      x = job.x;
-      y = job.y;
-      item = job.item;
-      seed = tea16(y * pp->width + x, pp->subframe);
-      acc[0] = 0.0f;
-      acc[kPathBlock] = 0.0f;
-      acc[2 * kPathBlock] = 0.0f;
-      ad0 = ad1 = ad2 = 0.0;
-      s = 0;
-      rec_base = (size_t)item * pp->spp;
-      alive = begin_sample();
-    }
-    if (kScan ? !__ballot(!idle) : idle) break;
     // -- NEE occlusion rays, first query: the closest emitter (emitter tree).
     // A miss and a non-emitting closest hit both leave a false hit flag
     // false (shader.cu:172-184), so with the flag false a ray that hits no
@@ -1136,38 +1127,32 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     // With the flag false a try whose line misses every emitter ends here
     // without normalising its draws (kScan: in nee_scan; else D holds the draws
     // of the try).  kScan: a try that needs the emitter tree leaves its query to
-    // the walk below (qstage 6), beside the other lanes' rays.
+    // the walk below (kTryEmit), beside the other lanes' rays.
     if constexpr (kScan) {
       for (;;) {
-        const bool want = alive && qstage == 1;
+        const bool want = stage == kTry;
         if (!__ballot(want)) break;
         const bool found = nee_scan<Src::kOneScene>(want && !hitf, scp->ecull_c, scp->ecull_h, O, seed, tries);
         if (want && !hitf && !found) {
-          alive = end_nee(mk(0.0f, 0.0f, 0.0f));
+          stage = kNeeEnd;
         } else if (want) {
           D = hemisphere_dir(hemisphere_raw(seed), N);
           if (!ray_valid(D)) {  // counts as a ray, misses without traversal
             hitf = false;
-            alive = nee_after(-5);
+            nee_after(-5);
           } else if (scp->emit.T > 0 && !emit_culled(scp->ecull_c, scp->ecull_h, O, D)) {
-            qstage = 6;
-          } else if (!hitf) {
-            alive = nee_after(-5);
-          } else {  // stale hit flag: a miss clears it, any other hit keeps it
-            tE = kTmax;
-            primE = 0xFFFFFFFFu;
-            matE = -1;
-            qstage = 2;
+            stage = kTryEmit;
+          } else {
+            no_emitter();
           }
         }
       }
     } else {
-      while (qstage == 1) {
+      while (stage == kTry) {
         if (kCount) c_occ++;
         if (kRecord) occl_cnt++;
         if (!hitf && line_culled(scp->ecull_c, scp->ecull_h, O, D)) {
-          alive = nee_after(-5);
-          if (!alive) break;
+          nee_after(-5);
           continue;
         }
         D = hemisphere_dir(D, N);
@@ -1182,37 +1167,47 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
         if (!valid) {  // counts as a ray, misses without traversal
           const int32_t code = hitf ? -1 : -5;
           hitf = false;
-          alive = nee_after(code);
+          nee_after(code);
         } else if (k >= 0) {  // an emitter: is anything in front of it?
           const float4 e0 = scp->emit.tris[3 * (size_t)k], e1 = scp->emit.tris[3 * (size_t)k + 1];
           tE = t;
           primE = __float_as_uint(e0.w);
           matE = (int32_t)__float_as_uint(e1.w);
-          qstage = 2;
-        } else if (!hitf) {
-          alive = nee_after(-5);
-        } else {  // stale hit flag: a miss clears it, any other hit keeps it
-          tE = kTmax;
-          primE = 0xFFFFFFFFu;
-          matE = -1;
-          qstage = 2;
+          stage = kAny;
+        } else {
+          no_emitter();
         }
-        if (!alive) break;
       }
     }
-    if (!alive) continue;  // the pixel is written at the top of the loop
-    if (kEmit && qstage == 5) {
-      // kMode 3, the end of a vertex's NEE run: another run from the
-      // vertex's entry flag and light (the last run's flag and light stay),
-      // then the light sample or the bounce
-      if (++nl < (b > 1 ? pp->nee_loops_deep : pp->nee_loops)) {
-        hitf = (ent & 1) != 0;
-        *light_mat = ent >> 1;
-        tries = 0;
-        qstage = 1;
-        continue;
+
+    // -- the end of an NEE loop (shoot_ray_to_light): add its light, if it has
+    // found one, then the next bounce (shader.cu:251-252) or, after the last
+    // one, the sample's end.
+    if (stage == kNeeEnd) {
+      F3 nee = mk(0.0f, 0.0f, 0.0f);
+      if (hitf) nee = xyz(scp->mats[*light_mat].emission_emit) * Bsdf::eval(N, D);
+      bool bounce = true;
+      if (kEmit) {
+        // kMode 3: the mean of nee_loops runs at the camera ray's hit,
+        // nee_loops_deep at later vertices, each added as it ends; another run
+        // starts from the vertex's entry flag and light (the last run's flag
+        // and light stay)
+        const int32_t runs = b > 1 ? pp->nee_loops_deep : pp->nee_loops;
+        if (runs > 1)
+          color = color + (nee * (1.0f / (float)runs)) * att;
+        else
+          color = color + nee * att;
+        if (++nl < runs) {
+          hitf = (ent & 1) != 0;
+          *light_mat = ent >> 1;
+          tries = 0;
+          stage = kTry;
+          bounce = false;
+        }
+      } else {
+        color = color + nee * att;
       }
-      if (rough == 1.0f && scp->emit.T > 0 && pp->emit_area > 0.0f && b < pp->bounces &&
+      if (kEmit && bounce && rough == 1.0f && scp->emit.T > 0 && pp->emit_area > 0.0f && b < pp->bounces &&
           light_sample_bounded(scp->ecull_c, scp->ecull_h, O, pp->emit_area)) {
         // Expected emission of this vertex's bounce ray.  The reference adds
         // Le * att when the bounce (a hemisphere draw at roughness 1, density
@@ -1254,42 +1249,60 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
           lw = q * cy * pp->emit_area / r2;
           ls_prim = __float_as_uint(p0.w);
           D = w;
-          qstage = 4;  // the emitter query below: is it the closest emitter?
-        } else {
-          D = Bsdf::sample(Din, N, seed, rough);  // p^ = 0
+          stage = kLightEmit;  // the emitter query below: is it the closest emitter?
+        } else {  // p^ = 0
           cond = true;
           rejects = 0;
-          qstage = 0;
+          stage = kBounce;
         }
-      } else {
-        D = Bsdf::sample(Din, N, seed, rough);
-        qstage = 0;
-        if (b == pp->bounces) {
-          finish_sample();
-          alive = begin_sample();
-          if (!alive) continue;
+        bounce = false;
+      }
+      if (bounce) stage = kBounce;
+    }
+    if (stage == kBounce) {
+      D = Bsdf::sample(Din, N, seed, rough);
+      stage = b == pp->bounces ? kSampleEnd : kRay;
+    }
+
+    // -- the next samples, the finished pixels and the lanes' next ones
+    while (stage == kSampleEnd || stage == kNext) {
+      if (stage == kSampleEnd) {
+        finish_sample();
+        stage = kNext;
+        if (s == pp->spp) {
+          write_pixel();
+          if (!src.next(job)) {
+            stage = kIdle;
+            break;
+          }
+          begin_pixel();
         }
       }
+      begin_sample();
     }
-    // -- one traversal per iteration: the closest hit of a radiance ray
-    // (qstage 0), the any-hit query of an occlusion ray (qstage 2, 3) or
-    // (kScan) the emitter query of an NEE try or a light sample (qstage 6, 4).
+    if (!__ballot(stage != kIdle)) break;
+
+    // -- one traversal: the closest hit of a radiance ray, the any-hit query of
+    // an occlusion ray or (kScan) the emitter query of an NEE try or a light
+    // sample.
+    if (stage == kIdle || stage == kTry) continue;
     const bool valid = ray_valid(D);
     int32_t k = -1;
     float t = 0.0f;
     if (valid && scp->all.T > 0) {
       const RayT r = make_ray(O, D);
-      const bool any = qstage == 2 || (kEmit && qstage == 3);
+      const bool any = stage == kAny || (kEmit && stage == kLightAny);
       if constexpr (kScan)
-        k = closest_walk<kPathBlock, true>(*scp, qstage >= 4, r, kTmin, any ? tE : kTmax,
-                                           any ? primE : 0xFFFFFFFFu, any, t, my_stk, spill, paused);
+        k = closest_walk<kPathBlock, true>(*scp, stage == kTryEmit || (kEmit && stage == kLightEmit), r, kTmin,
+                                           any ? tE : kTmax, any ? primE : 0xFFFFFFFFu, any, t, my_stk, spill,
+                                           paused);
       else
         k = closest<kCount, kPathBlock>(scp->all, r, kTmin, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu, any, t,
                                         my_stk, spill, tc);
     }
     if (kScan && paused) continue;
 
-    if (qstage == 0) {
+    if (stage == kRay) {
       // radiance: miss (189-194) / closest hit (211-255)
       if (kCount) {
         c_rad++;
@@ -1318,12 +1331,10 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
         if (kEmit && cond && m.emission_emit.w != 0.0f) {
           // a conditioned bounce hit an emitter: draw it again (not a bounce)
           --b;
-          if (++rejects == kMaxRedraws) {
+          if (++rejects == kMaxRedraws)
             finish = true;
-          } else {
-            D = Bsdf::sample(Din, N, seed, rough);
-            continue;
-          }
+          else
+            stage = kBounce;
         } else if (m.emission_emit.w != 0.0f) {
           color = color + xyz(m.emission_emit) * att;
           finish = true;
@@ -1368,7 +1379,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
           } else {
             att = att * xyz(m.diffuse_alpha);
             rough = m.rough_n.x;
-            qstage = 1;
+            stage = kTry;
             tries = 0;
             if (kEmit) {  // the NEE loops of this vertex start from this flag and light
               ent = (*light_mat << 1) | (hitf ? 1 : 0);
@@ -1378,45 +1389,35 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
           }
         }
       }
-      if (finish) {
-        finish_sample();
-        alive = begin_sample();
-      }
-    } else if (kScan && qstage >= 4) {
-      // the closest emitter of an NEE try (6) or a light sample (4)
+      if (finish) stage = kSampleEnd;
+    } else if (kScan && (stage == kTryEmit || (kEmit && stage == kLightEmit))) {
+      // the closest emitter of an NEE try or a light sample
       float4 e0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), e1 = e0;
       if (k >= 0) {
         e0 = scp->all.tris[3 * (size_t)k];
         e1 = scp->all.tris[3 * (size_t)k + 1];
       }
       const uint32_t prim = __float_as_uint(e0.w);
-      if (k >= 0 && (qstage == 6 || (kEmit && prim == ls_prim))) {  // is anything in front of it?
+      if (k >= 0 && (stage == kTryEmit || prim == ls_prim)) {  // is anything in front of it?
         tE = t;
         primE = prim;
         matE = (int32_t)__float_as_uint(e1.w);
-        qstage = qstage == 6 ? 2 : 3;
-      } else if (kEmit && qstage == 4) {  // p^ = 0
-        D = Bsdf::sample(Din, N, seed, rough);
+        stage = stage == kTryEmit ? kAny : kLightAny;
+      } else if (stage == kTryEmit) {
+        no_emitter();
+      } else {  // p^ = 0
         cond = true;
         rejects = 0;
-        qstage = 0;
-      } else if (!hitf) {
-        alive = nee_after(-5);
-      } else {  // stale hit flag: a miss clears it, any other hit keeps it
-        tE = kTmax;
-        primE = 0xFFFFFFFFu;
-        matE = -1;
-        qstage = 2;
+        stage = kBounce;
       }
-    } else if (kEmit && qstage == 3) {
+    } else if (kEmit && stage == kLightAny) {
       // the light sample of a prefix bounce: visible unless blocked before (tE, primE)
       const float ph = k >= 0 ? 0.0f : lw;
       color = color + (xyz(scp->mats[matE].emission_emit) * ph) * att;
       att = att * (1.0f - ph);
-      D = Bsdf::sample(Din, N, seed, rough);
       cond = true;
       rejects = 0;
-      qstage = 0;
+      stage = kBounce;
     } else {
       // occlusion, second query: blocked before (tE, primE)?
       const bool blocked = k >= 0;
@@ -1435,7 +1436,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
         code = -1;
         hitf = false;
       }
-      alive = nee_after(code);
+      nee_after(code);
     }
   }
 
