@@ -135,8 +135,8 @@ lisa_status lisa_update_vertices_noalloc(lisa_ctx* ctx, const float* d_verts, co
 /* Replaces render() -> launchSubframe() -> optixLaunch(w, h, 1)
  * (src/LiSA/src/render.cc:35-58, 133-148).  The float4 accum buffer stays on
  * the device (as OptixParams::accum_buffer); accum_rgba_out (w*h*4 floats)
- * and rgba8_out (w*h*4 bytes, make_color of helpers.h:57-66 done on the host)
- * are optional host copies. */
+ * and rgba8_out (w*h*4 bytes, make_color of helpers.h:57-66: the bytes of
+ * lisa_srgb_quantize) are optional host copies. */
 lisa_status lisa_render(lisa_ctx* ctx, const lisa_render_params* p,
                         float* accum_rgba_out, uint8_t* rgba8_out);
 

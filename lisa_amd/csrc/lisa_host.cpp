@@ -70,6 +70,27 @@ inline uint8_t quant8(float x) {
 
 }  // namespace
 
+const lisa::SrgbSteps& lisa::srgb_steps() {
+  static const SrgbSteps steps = [] {
+    SrgbSteps s;
+    for (int v = 1; v <= 255; ++v) {  // bisection over the bits of [0, 1]
+      uint32_t lo = 0, hi = 0x3F800000u;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) / 2;
+        float c;
+        std::memcpy(&c, &mid, 4);
+        if (quant8(to_srgb(c)) >= v)
+          hi = mid;
+        else
+          lo = mid + 1;
+      }
+      std::memcpy(&s.at[v - 1], &lo, 4);
+    }
+    return s;
+  }();
+  return steps;
+}
+
 extern "C" {
 
 lisa_status lisa_camera_uvw(const float eye[3], const float look_at[3], float fov, float aspect,

@@ -10,6 +10,13 @@ namespace lisa {
 void set_global_error(const std::string& msg);
 lisa_status global_fail(lisa_status code, const std::string& msg);
 const char* global_error();
+// lisa_srgb_quantize's byte steps: at[v - 1] is the smallest float in [0, 1] whose
+// byte is at least v, v = 1 .. 255 (the byte of a channel never falls as the
+// float grows).
+struct SrgbSteps {
+  float at[255];
+};
+const SrgbSteps& srgb_steps();
 // `steps` Adam steps of the radiance cache on the same device-resident
 // samples (feature rows of feat_stride floats, the first 12 used; targets 3
 // per row, non-finite targets ignored), enqueued back to back; *loss is the
