@@ -3136,6 +3136,71 @@ struct DevBuf {
   }
 };
 
+// A context's scene memory and the scratch of its builds.  hipMalloc and
+// hipFree of a scene's two dozen buffers took longer than building its trees
+// (292k triangles: lisa_set_scene 4.2 ms, of which kernels and copies 1.5), and a
+// program that loads or moves scenes on one context asks for the same sizes
+// again: blocks go back to a list and are handed out to requests of at least
+// half their size.  A block is only handed to work on the context's stream (or
+// behind a copy that waits for it), so one that is given back while the stream
+// still uses it is safe.  The list keeps at most kPoolFree bytes and is
+// released with the context.
+constexpr size_t kPoolFree = size_t{1} << 30;
+struct DevPool {
+  struct Block {
+    void* p;
+    size_t n;
+  };
+  std::vector<Block> idle, used;
+  hipError_t take(void** p, size_t want) {
+    want = (std::max<size_t>(want, 1) + 255) / 256 * 256;
+    size_t best = idle.size();
+    for (size_t i = 0; i < idle.size(); ++i)
+      if (idle[i].n >= want && idle[i].n <= 2 * want + 65536 && (best == idle.size() || idle[i].n < idle[best].n))
+        best = i;
+    if (best < idle.size()) {
+      used.push_back(idle[best]);
+      idle.erase(idle.begin() + (long)best);
+      *p = used.back().p;
+      return hipSuccess;
+    }
+    hipError_t e = hipMalloc(p, want);
+    if (e != hipSuccess && !idle.empty()) {
+      (void)hipGetLastError();
+      trim(0);
+      e = hipMalloc(p, want);
+    }
+    if (e == hipSuccess) used.push_back(Block{*p, want});
+    return e;
+  }
+  void give(void* p) {
+    if (!p) return;
+    for (size_t i = used.size(); i-- > 0;)
+      if (used[i].p == p) {
+        idle.push_back(used[i]);
+        used.erase(used.begin() + (long)i);
+        return;
+      }
+  }
+  void trim(size_t keep) {  // the largest idle blocks first
+    size_t sum = 0;
+    for (const Block& b : idle) sum += b.n;
+    while (sum > keep) {
+      size_t big = 0;
+      for (size_t i = 1; i < idle.size(); ++i)
+        if (idle[i].n > idle[big].n) big = i;
+      sum -= idle[big].n;
+      (void)hipFree(idle[big].p);
+      idle.erase(idle.begin() + (long)big);
+    }
+  }
+  void release() {
+    trim(0);
+    for (const Block& b : used) (void)hipFree(b.p);
+    used.clear();
+  }
+};
+
 // Device memory of lisa_update_vertices_noalloc (the refit for callers that
 // cannot allocate): the two union tables of the level refit, 2 float4 per
 // triangle each, for scenes of at most kNoAllocMaxTris triangles (64 MB per
@@ -3273,6 +3338,7 @@ struct lisa_ctx {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::string err;
   int32_t T = 0, M = 0;
+  DevPool pool;
   DevBvh all, emit;  // over every triangle / over the emitting triangles
   float4* d_nrm = nullptr;
   DevMat* d_mats = nullptr;
@@ -3370,29 +3436,21 @@ lisa_status fail(lisa_ctx* ctx, lisa_status code, const std::string& msg) {
       return fail((ctx), LISA_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-void free_bvh(DevBvh& b) {
-  (void)hipFree(b.nodes);
-  (void)hipFree(b.wide);
-  (void)hipFree(b.tris);
-  (void)hipFree(b.morton);
-  (void)hipFree(b.prim);
-  (void)hipFree(b.parent);
-  (void)hipFree(b.leaf_parent);
-  (void)hipFree(b.range);
-  (void)hipFree(b.walk);
-  (void)hipFree(b.agg);
-  (void)hipFree(b.lists);
-  (void)hipFree(b.counts);
+void free_bvh(lisa_ctx* c, DevBvh& b) {
+  for (void* p : {(void*)b.nodes, (void*)b.wide, (void*)b.tris, (void*)b.morton, (void*)b.prim, (void*)b.parent,
+                  (void*)b.leaf_parent, (void*)b.range, (void*)b.walk, (void*)b.agg, (void*)b.lists,
+                  (void*)b.counts})
+    c->pool.give(p);
   b = DevBvh();
 }
 
 void free_scene(lisa_ctx* c) {
   c->gen++;
   c->j_seq = false;
-  free_bvh(c->all);
-  free_bvh(c->emit);
-  (void)hipFree(c->d_nrm);
-  (void)hipFree(c->d_mats);
+  free_bvh(c, c->all);
+  free_bvh(c, c->emit);
+  c->pool.give(c->d_nrm);
+  c->pool.give(c->d_mats);
   c->d_nrm = nullptr;
   c->d_mats = nullptr;
   c->T = c->M = 0;
@@ -3414,16 +3472,21 @@ SceneView view(const lisa_ctx* c) {
                    (uint32_t)agg_capacity(c->all.T)};
 }
 
-// Device scratch freed at scope exit.
+// Device scratch, given back to the context's pool at scope exit.
 struct Scratch {
+  DevPool& pool;
   std::vector<void*> ptrs;
+  explicit Scratch(lisa_ctx* ctx) : pool(ctx->pool) {}
   ~Scratch() {
-    for (void* p : ptrs) (void)hipFree(p);
+    for (void* p : ptrs) pool.give(p);
+    pool.trim(kPoolFree);
   }
   template <typename T>
   hipError_t alloc(T** p, size_t count) {
-    const hipError_t e = hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(count, 1) * sizeof(T));
-    if (e == hipSuccess) ptrs.push_back(*p);
+    void* q = nullptr;
+    const hipError_t e = pool.take(&q, std::max<size_t>(count, 1) * sizeof(T));
+    *p = static_cast<T*>(q);
+    if (e == hipSuccess) ptrs.push_back(q);
     return e;
   }
 };
@@ -3479,8 +3542,7 @@ PathArgs make_args(const lisa_render_params* p) {
 
 // Every child box of b (T >= 2) from its triangles: the leaf level, then one
 // k_rf_level pass per level of the union table (scratch: two tables of T
-// entries, 32 bytes each).  Enqueued on ctx->stream; waits before returning
-// (the scratch is freed).
+// entries, 32 bytes each).  Enqueued on ctx->stream.
 // The same passes on caller-provided tables (2 * T float4 each); no allocation, no wait.
 lisa_status refit_levels_on(lisa_ctx* ctx, DevBvh& b, float4* ta, float4* tb) {
   hipStream_t st = ctx->stream;
@@ -3496,14 +3558,11 @@ lisa_status refit_levels_on(lisa_ctx* ctx, DevBvh& b, float4* ta, float4* tb) {
   return LISA_OK;
 }
 lisa_status refit_levels(lisa_ctx* ctx, DevBvh& b) {
-  Scratch S;
+  Scratch S(ctx);
   float4 *ta = nullptr, *tb = nullptr;
   HIP_TRY(ctx, S.alloc(&ta, 2 * (size_t)b.T));
   HIP_TRY(ctx, S.alloc(&tb, 2 * (size_t)b.T));
-  lisa_status rc = refit_levels_on(ctx, b, ta, tb);
-  if (rc != LISA_OK) return rc;
-  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // the tables are freed on return
-  return LISA_OK;
+  return refit_levels_on(ctx, b, ta, tb);
 }
 
 // The 4-wide form of b from its nodes (when b has one), on stream st.
@@ -3554,14 +3613,14 @@ lisa_status prepare_walk(lisa_ctx* ctx, uint32_t* place) {
   DevBvh &all = ctx->all, &emit = ctx->emit;
   const size_t nodes = agg_capacity(all.T) + agg_capacity(emit.T);
   if (all.T == 0 || nodes > kWalkMaxNodes) return LISA_OK;
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&all.walk), 128 * nodes));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&all.walk), 128 * nodes));
   all.bytes += 128 * nodes;
   for (DevBvh* b : {&all, &emit}) {
     if (b->T == 0) continue;
     const size_t cap = agg_capacity(b->T), chunks = ((size_t)b->T + kAggChunk - 1) / kAggChunk;
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b->agg), 64 * cap));
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b->lists), 64 * chunks * kAggOut));
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b->counts), 8 * chunks));
+    HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b->agg), 64 * cap));
+    HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b->lists), 64 * chunks * kAggOut));
+    HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b->counts), 8 * chunks));
     b->bytes += 64 * cap + 64 * chunks * kAggOut + 8 * chunks;
     HIP_TRY(ctx, hipMemsetAsync(b->agg, 0xFF, 64 * cap, st));  // refs kEmpty: indexes that k_agg leaves out
   }
@@ -3585,21 +3644,21 @@ lisa_status build_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
   b.T = n;
   b.nI = n > 1 ? n - 1 : 1;
   const size_t nodes_b = 64 * (size_t)b.nI, tris_b = 48 * ((size_t)std::max(n, 1) + 1);
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.nodes), nodes_b));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b.nodes), nodes_b));
   if (wide) {
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.wide), 2 * nodes_b));
+    HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b.wide), 2 * nodes_b));
     b.bytes += 2 * nodes_b;
   }
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.tris), tris_b));
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.morton), 4 * (size_t)std::max(n, 1)));
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.prim), 4 * (size_t)std::max(n, 1)));
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.parent), 4 * (size_t)std::max(n, 1)));
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.leaf_parent), 4 * (size_t)std::max(n, 1)));
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&b.range), 8 * (size_t)std::max(n, 1)));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b.tris), tris_b));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b.morton), 4 * (size_t)std::max(n, 1)));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b.prim), 4 * (size_t)std::max(n, 1)));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b.parent), 4 * (size_t)std::max(n, 1)));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b.leaf_parent), 4 * (size_t)std::max(n, 1)));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b.range), 8 * (size_t)std::max(n, 1)));
   b.bytes += nodes_b + tris_b + 16 * (size_t)std::max(n, 1);
   HIP_TRY(ctx, hipMemsetAsync(b.nodes, 0, nodes_b, st));
   if (n == 0) return LISA_OK;
-  Scratch S;
+  Scratch S(ctx);
   float *d_part = nullptr, *d_bounds = nullptr;
   int32_t *d_parent = b.parent, *d_leafp = b.leaf_parent;
   uint32_t *d_k2 = nullptr, *d_v2 = nullptr, *d_hist = nullptr, *d_tot = nullptr;
@@ -3639,8 +3698,6 @@ lisa_status build_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
   lisa_status rw = wide_nodes(ctx, b, st);
   if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipGetLastError());
-  // scratch is freed on return: wait for the kernels that use it
-  HIP_TRY(ctx, hipStreamSynchronize(st));
   return LISA_OK;
 }
 
@@ -3658,7 +3715,6 @@ lisa_status refit_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
   }
   lisa_status rw = wide_nodes(ctx, b, st);
   if (rw != LISA_OK) return rw;
-  HIP_TRY(ctx, hipStreamSynchronize(st));
   HIP_TRY(ctx, hipGetLastError());
   return LISA_OK;
 }
@@ -3968,7 +4024,7 @@ lisa_status lisa_update_vertices(lisa_ctx* ctx, const float* verts, const float*
   if (!verts) return fail(ctx, LISA_ERR_INVALID_ARG, "verts is NULL");
   HIP_TRY(ctx, hipSetDevice(ctx->device));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  Scratch S;
+  Scratch S(ctx);
   float *d_v = nullptr, *d_n = nullptr;
   HIP_TRY(ctx, S.alloc(&d_v, 9 * (size_t)T));
   HIP_TRY(ctx, hipMemcpy(d_v, verts, 36 * (size_t)T, hipMemcpyHostToDevice));
@@ -4103,6 +4159,7 @@ void lisa_destroy(lisa_ctx* c) {
   c->c_rgba8.release();
   c->pg.release();
   free_scene(c);
+  c->pool.release();
   (void)hipFree(c->d_accum);
   (void)hipFree(c->d_counters);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -4142,11 +4199,11 @@ lisa_status lisa_set_scene(lisa_ctx* ctx, const float* verts, const float* norma
   std::vector<uint32_t> emit_ids;
   for (int32_t k = 0; k < T; ++k)
     if (mats[mat_idx[k]].emit) emit_ids.push_back((uint32_t)k);
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->d_mats), sizeof(DevMat) * hm.size()));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&ctx->d_mats), sizeof(DevMat) * hm.size()));
   HIP_TRY(ctx, hipMemcpy(ctx->d_mats, hm.data(), sizeof(DevMat) * hm.size(), hipMemcpyHostToDevice));
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->d_nrm), 48 * (size_t)std::max(T, 1)));
+  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&ctx->d_nrm), 48 * (size_t)std::max(T, 1)));
   ctx->scene_bytes = sizeof(DevMat) * hm.size() + 48 * (size_t)std::max(T, 1);
-  Scratch S;
+  Scratch S(ctx);
   float *d_v = nullptr, *d_n = nullptr;
   int32_t* d_mat = nullptr;
   uint32_t* d_gid = nullptr;
@@ -4364,7 +4421,7 @@ lisa_status lisa_trace_subset(lisa_ctx* ctx, const lisa_render_params* p, const 
       return fail(ctx, LISA_ERR_INVALID_ARG, "pixel id out of range");
   HIP_TRY(ctx, hipSetDevice(ctx->device));
   const size_t ns = (size_t)n_pixels * p->spp;
-  Scratch S;
+  Scratch S(ctx);
   int32_t* d_px = nullptr;
   float4* d_acc = nullptr;
   float* d_rgb = nullptr;
@@ -4422,7 +4479,7 @@ lisa_status lisa_trace_rays(lisa_ctx* ctx, const float* O, const float* D, int32
     return fail(ctx, LISA_ERR_INVALID_ARG, "bad ray arrays");
   if (n == 0) return LISA_OK;
   HIP_TRY(ctx, hipSetDevice(ctx->device));
-  Scratch S;
+  Scratch S(ctx);
   float *d_o = nullptr, *d_d = nullptr, *d_t = nullptr;
   int32_t* d_p = nullptr;
   HIP_TRY(ctx, S.alloc(&d_o, 3 * (size_t)n));
