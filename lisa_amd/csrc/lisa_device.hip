@@ -251,7 +251,9 @@ __device__ __forceinline__ bool line_culled(float4 c, float4 H, F3 O, F3 d) {
 // integers k - 2^23 (hemisphere_raw's times 2^23, exact), a multiply-add, a sign
 // extension and a conversion each.  The products of a test are fused (one
 // rounding each instead of two, within the margin), its three axes run without
-// branches.  (vx, vy, vz): the box's centre from the vertex; H: its half extents.
+// branches.  A draw of zero needs no exception (unlike in line_culled, whose
+// results the counters record): the separating axes hold for any direction, and a
+// line that passes the box by the margin meets no emitter.  (vx, vy, vz): the box's centre from the vertex; H: its half extents.
 __device__ __forceinline__ bool try_culled(float vx, float vy, float vz, float4 H, uint32_t& t) {
   auto draw = [&]() {
     t = lcg24(t);
@@ -263,7 +265,7 @@ __device__ __forceinline__ bool try_culled(float vx, float vy, float vz, float4 
               pz = __builtin_fmaf(vx, y, -(vy * x));
   const float qx = __builtin_fmaf(H.y, az, H.z * ay), qy = __builtin_fmaf(H.z, ax, H.x * az),
               qz = __builtin_fmaf(H.x, ay, H.y * ax);
-  return ((fabsf(px) > qx) | (fabsf(py) > qy) | (fabsf(pz) > qz)) & (fminf(fminf(ax, ay), az) != 0.0f);
+  return (fabsf(px) > qx) | (fabsf(py) > qy) | (fabsf(pz) > qz);
 }
 
 // kTryJump[j]: 3 j steps of the LCG (j tries) as one, s -> x s + y mod 2^24.
@@ -295,7 +297,8 @@ static_assert(kNeeTries <= 31, "a half wave makes a vertex's tries at once");
 // 15 vertices: each half wave then makes all tries of one vertex at once, from
 // the LCG states 3 j steps on, and the first that is not culled is a bit scan of
 // the ballot.  A pass costs about two tries and serves two vertices (C2 at 32 spp
-// 29.1 -> 25.4 ms, Cornell box of 1k triangles 256^2, 16 spp 4.26 -> 3.66).  With more than kNeeSerial vertices every lane
+// 29.1 -> 25.4 ms, Cornell box of 1k triangles 256^2, 16 spp 4.26 -> 3.66; without
+// the vertex's try count in the pass 22.8 -> 22.4).  With more than kNeeSerial vertices every lane
 // makes its own tries in turn (`shared` false: always, where the lanes' scenes
 // may differ).
 constexpr int kNeeSerial = 30;  // 16 measured 5 % slower on C2; 64 (never in turn) the same
@@ -320,8 +323,7 @@ __device__ __forceinline__ bool nee_scan(bool scan, float4 c, float4 H, F3 O, ui
   if (m == 0) return false;
   const int lane = (int)__lane_id(), j = lane & 31;
   const uint2 jump = kTryJumps.j[j];
-  const uint32_t pack = (t & 0xFFFFFFu) | ((uint32_t)tries << 24);
-  int32_t adv = 0;
+  int32_t adv = 32;  // no candidate
   while (m) {
     const int i0 = __ffsll((unsigned long long)m) - 1;
     m &= m - 1;
@@ -329,17 +331,16 @@ __device__ __forceinline__ bool nee_scan(bool scan, float4 c, float4 H, F3 O, ui
     m &= m - 1;
     const int src = lane < 32 ? i0 : i1;
     const float sx = __shfl(vx, src), sy = __shfl(vy, src), sz = __shfl(vz, src);
-    const uint32_t w = __shfl(pack, src);
-    uint32_t u = __umul24(w, jump.x) + jump.y;
-    const bool left = !try_culled(sx, sy, sz, H, u) && j + (int)(w >> 24) < kNeeTries;
-    const uint64_t b = __ballot(left);
-    if (lane == i0 || lane == i1) {
-      const uint32_t h = lane == i0 ? (uint32_t)b : (uint32_t)(b >> 32);
-      found = h != 0;
-      adv = found ? __ffs((int)h) - 1 : kNeeTries - tries;
-    }
+    uint32_t u = __umul24(__shfl(t, src), jump.x) + jump.y;
+    // a try past the vertex's last one may be a candidate too: dropped below
+    const uint64_t b = __ballot(!try_culled(sx, sy, sz, H, u));
+    const uint32_t b0 = (uint32_t)b, b1 = (uint32_t)(b >> 32);
+    adv = lane == i1 ? (b1 ? __builtin_ctz(b1) : 32) : adv;
+    adv = lane == i0 ? (b0 ? __builtin_ctz(b0) : 32) : adv;  // (an odd one out: both halves are its)
   }
   if (scan) {
+    found = adv < kNeeTries - tries;
+    adv = min(adv, kNeeTries - tries);
     tries += adv;
     const uint2 g = kTryJumps.j[adv];
     seed = (__umul24(t, g.x) + g.y) ^ 0x800000u;
@@ -369,6 +370,13 @@ __device__ __forceinline__ bool light_sample_bounded(float4 c, float4 H, F3 O, f
   const float dz = fmaxf(fabsf(O.z - c.z) - H.z, 0.0f);
   const float d2 = dx * dx + dy * dy + dz * dz;
   return 0.9f * A <= d2;
+}
+
+// The next float above a finite x (nextafterf(x, INFINITY)) in four operations:
+// closest_walk's last check of every hit was 3 % of C2 with nextafterf, 2 % so.
+__device__ __forceinline__ float float_up(float x) {
+  const int32_t b = (int32_t)__float_as_uint(x + 0.0f);  // -0 as +0
+  return __uint_as_float((uint32_t)(b + ((b >> 31) | 1)));
 }
 
 // Triangle bounds widened outward by one ulp: an origin exactly on a face
@@ -750,7 +758,14 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
     // box.  The hit stands if its own box passes; otherwise closest() answers.
     if (best_k >= 0) {
       float b[6], tn;
-      leaf_box(bv.tris, best_k, b);
+      const float4 a = bv.tris[3 * (size_t)best_k], c = bv.tris[3 * (size_t)best_k + 1],
+                   e = bv.tris[3 * (size_t)best_k + 2];
+      b[0] = -float_up(-fminf(fminf(a.x, c.x), e.x));  // leaf_box of finite vertices
+      b[1] = -float_up(-fminf(fminf(a.y, c.y), e.y));
+      b[2] = -float_up(-fminf(fminf(a.z, c.z), e.z));
+      b[3] = float_up(fmaxf(fmaxf(a.x, c.x), e.x));
+      b[4] = float_up(fmaxf(fmaxf(a.y, c.y), e.y));
+      b[5] = float_up(fmaxf(fmaxf(a.z, c.z), e.z));
       done = done && slab(b[0], b[1], b[2], b[3], b[4], b[5], r, tmin, tlim * kWiden, tn);
     }
   }
