@@ -9,8 +9,8 @@ traversal-bound 5.2M-triangle displaced icosphere (1920x1080, 64 spp,
     python bench.py [--steps K] [--warmup W] [--spp S] [--no-cpu] [--workload W]
 
 Prints one JSON line.  `value` is rays traced (radiance + occlusion, exact
-counts from the counting kernel, which is bit-identical in work to the
-timed one) per second of wall time over the K timed steps.  `roofline` uses
+counts from the counting kernel, which traces the same rays as the timed
+one) per second of wall time over the K timed steps.  `roofline` uses
 the average kernel duration from HIP events recorded on the context's own
 stream; `cpu_baseline` times the CPU oracle on a seeded pixel subset of the
 same workload on this host's cores.  The default run also times the other
@@ -31,6 +31,8 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Mrays/s; time to RMSE≤1e-2 vs 16k-spp ref, cache vs plain, 1 MI355X"
 HBM_PEAK_GBS = 8000.0
+# one 64-lane VALU instruction per SIMD every 4 cycles: 1,024 SIMDs at 2.4 GHz
+VALU_PEAK_TINST = round(256 * 4 * 16 * 2.4e-3, 2)
 # Algorithmic bytes: one 64-byte node line per BVH node visit, one 48-byte
 # triangle record per triangle test, 96 bytes (vertices + normals) per
 # shaded radiance hit, one float4 accum store per pixel.
@@ -108,10 +110,11 @@ def parse():
     return ap.parse_args()
 
 
-def profile_record(workload, spp, bvh):
+def profile_record(workload, spp):
     """The plain megakernel's rocprofv3 figures recorded in
-    profiles/k_path_<workload>_pmc.json for the same spp and tree walk
-    ("binary" or "4-wide"; a record without the key is of the binary walk), or {}:
+    profiles/k_path_<workload>_pmc.json for the same spp, or {}:
+    valu_lane_insts (SQ_THREAD_CYCLES_VALU of one launch: active lanes summed
+    over the VALU instructions),
     hbm_bytes_per_launch (two --pmc runs, FETCH_SIZE and WRITE_SIZE, scaled
     by the copy-kernel calibration) and valu_lane_utilization
     (SQ_THREAD_CYCLES_VALU / (64 x SQ_ACTIVE_INST_VALU))."""
@@ -119,7 +122,7 @@ def profile_record(workload, spp, bvh):
     try:
         with open(path) as fh:
             rec = json.load(fh)
-        return rec if int(rec["spp"]) == spp and rec.get("bvh", "binary") == bvh else {}
+        return rec if int(rec["spp"]) == spp and rec["bvh"] == "agglomerated 4-wide" else {}
     except (OSError, KeyError, ValueError):
         return {}
 
@@ -127,9 +130,17 @@ def profile_record(workload, spp, bvh):
 def bench_plain(a, workload, steps, warmup, cpu=True):
     """One plain-megakernel workload: exact ray counts from the counting
     instantiation, `steps` timed renders after `warmup`, the kernel's
-    roofline (algorithmic bytes over the HIP-event kernel time; DRAM traffic
-    from the committed rocprof counters) and, with `cpu`, the CPU oracle on a
-    seeded pixel subset.  Returns (result dict, ctx triangle count)."""
+    roofline (the committed rocprof counters over the HIP-event kernel time)
+    and, with `cpu`, the CPU oracle on a seeded pixel subset.  Returns the
+    result dict.
+
+    The tiled megakernel is bound by VALU issue, so that is its roofline:
+    lane-instructions per second against 64 per SIMD every 4 cycles (the rate
+    of min, max, compare and select; fma, add and moves of two waves can
+    overlap).  Bytes of the counted walk would not do: the counting build walks the Morton
+    tree, which the oracle reproduces, and the timed build the agglomerated
+    one, which visits a fraction of its nodes.  The wavefront form does walk
+    the Morton tree and keeps the byte roofline."""
     from lisa_amd import capi, scenes
 
     factory, def_spp, def_cpu_px = WORKLOADS[workload]
@@ -142,9 +153,8 @@ def bench_plain(a, workload, steps, warmup, cpu=True):
     ctx = capi.Context(0)
     ctx.set_scene(sc["verts"], sc["normals"], sc["mat_idx"], sc["materials"])
     bvh_ms = ctx.stats()["bvh_build_ms"]
-    wide = ctx.stats()["wide_tree"]  # scenes of >= 2^20 triangles: the 4-wide walk
-    print(f"[bench] scene {sc['name']}: {ctx.T} triangles, LBVH build {bvh_ms:.2f} ms"
-          + (" (with its 4-wide form)" if wide else ""), file=sys.stderr, flush=True)
+    print(f"[bench] scene {sc['name']}: {ctx.T} triangles, BVH build {bvh_ms:.2f} ms",
+          file=sys.stderr, flush=True)
 
     # exact work per step (counting instantiation of the same kernel)
     p = capi.render_params(W, H, spp, B, cam["eye"], U, V, Wv, flags=capi.FLAG_COUNT)
@@ -168,31 +178,31 @@ def bench_plain(a, workload, steps, warmup, cpu=True):
     wall = time.perf_counter() - t0
     avg_kernel_ms = sum(kernel_ms) / len(kernel_ms)
 
-    alg_bytes = (S_NODE * counts["node_visits"] + S_TRI * counts["tri_tests"]
-                 + S_SHADE * counts["radiance_hits"] + S_PIXEL * W * H)
-    achieved = alg_bytes / (avg_kernel_ms * 1e-3) / 1e9
-    rec = {} if (a.persistent or a.wavefront) else profile_record(workload, spp,
-                                                                  "4-wide" if wide else "binary")
-    traffic = rec.get("hbm_bytes_per_launch")
-    resident = workload in ("cornell", "cornell65k")
-    roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                "traffic": traffic,
-                "dram_frac": (None if traffic is None else
-                              round(traffic / (avg_kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)),
-                # fraction of a wave's 64 lanes active per VALU instruction
-                "lane_utilization": rec.get("valu_lane_utilization"),
-                "limiter": ("instruction issue under divergence; the scene is L2 / Infinity "
-                            "Cache resident, so `frac` counts bytes served mostly from cache"
-                            if resident else
-                            "instruction issue under divergence, with the scene's nodes and "
-                            "triangles streamed from HBM"),
-                "kernel": ("k_path_pq<0>" if a.persistent else
-                           "k_wf_trace + k_wf_shade rounds" if a.wavefront else
-                           "k_path<false,false,false,true> (4-wide walk)" if wide else
-                           "k_path<false,false,false>"),
-                "alg_bytes_per_launch": alg_bytes,
-                "avg_kernel_ms": round(avg_kernel_ms, 3)}
+    seconds = avg_kernel_ms * 1e-3
+    rec = {} if (a.persistent or a.wavefront) else profile_record(workload, spp)
+    traffic, insts = rec.get("hbm_bytes_per_launch"), rec.get("valu_lane_insts")
+    if a.wavefront:
+        alg_bytes = (S_NODE * counts["node_visits"] + S_TRI * counts["tri_tests"]
+                     + S_SHADE * counts["radiance_hits"] + S_PIXEL * W * H)
+        achieved = alg_bytes / seconds / 1e9
+        roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+                    "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+                    "kernel": "k_wf_trace + k_wf_shade rounds", "alg_bytes_per_launch": alg_bytes}
+    else:
+        achieved = None if insts is None else insts / seconds / 1e12
+        roofline = {"bound": "valu_issue",
+                    "achieved": None if achieved is None else round(achieved, 2),
+                    "peak": VALU_PEAK_TINST, "unit": "T lane-instructions/s",
+                    "frac": None if achieved is None else round(achieved / VALU_PEAK_TINST, 4),
+                    # fraction of a wave's 64 lanes active per VALU instruction
+                    "lane_utilization": rec.get("valu_lane_utilization"),
+                    "limiter": "VALU issue under divergence: the lanes of a wave end their "
+                               "walks and their stages at different points",
+                    "kernel": "k_path_pq<0>" if a.persistent else "k_path<false,false,false>"}
+    roofline.update(traffic=traffic,
+                    dram_frac=(None if traffic is None else
+                               round(traffic / seconds / 1e9 / HBM_PEAK_GBS, 4)),
+                    avg_kernel_ms=round(avg_kernel_ms, 3))
 
     cpu_res = None
     if cpu:
@@ -232,7 +242,7 @@ def bench_plain(a, workload, steps, warmup, cpu=True):
                                   + (" (persistent launch)" if a.persistent else ""),
                       "width": W, "height": H,
                       "spp": spp, "bounces": B, "triangles": ctx.T,
-                      "bvh": "binary + 4-wide form" if wide else "binary",
+                      "bvh": "agglomerated 4-wide",
                       "parallelism": "single GPU"},
            "samples_per_s": round(W * H * spp * steps / wall, 1),
            "rays_per_step": rays, "bvh_build_ms": round(bvh_ms, 3),
