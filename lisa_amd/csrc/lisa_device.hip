@@ -619,12 +619,19 @@ __device__ __forceinline__ int32_t closest_wide(const BvhView& bv, const RayT& r
 // construction; 20 entries are passed by 1e-5 of a batch scene's walks, 28 by
 // none seen), as does a scene without a walk tree.
 //
-// Bound by instruction issue of the wave's longest walk.  Visits per ray and
+// Bound by VALU issue: min, max, compare, select and shift take 4.2 to 5 cycles
+// of a SIMD, fma, add and moves 2.4 to 2.9 (two waves' overlap), and k_path on C2
+// fills 103 % of the slots at 4 cycles, with 51 % of the lanes active.  Five loads
+// per node instead of seven (planes as 16-bit floats around the node's centre,
+// 18 VALU instructions more) took 24.4 ms against 22.2 (C2 at 32 spp) and 28.7
+// against 28.6 (icosphere of 1.3M triangles, 1080p, 16 spp); sorting only the
+// nearest out (three exchanges) 22.2 and 28.6.  Visits per ray and
 // per wave of 64 (the longest): Cornell box of 65k triangles 23.4 / 60.5 in
 // the binary Morton tree, 11.4 / 29.7 in its 4-wide form, 4.2 / 17.0 here;
 // icosphere of 328k 21.0 / 63.6, 11.1 / 32.7, 5.4 / 23.2.  k_path at 32 spp,
 // 1024^2: C2 67.5 -> 44.5 ms; icosphere of 1.3M triangles, 1080p, 16 spp:
-// 85.6 -> 53.8 ms (before: its 4-wide Morton walk).
+// 85.6 -> 53.8 ms (before: its 4-wide Morton walk); with all that follows, here
+// and in the path loop, 22.0 and 28.5 ms.
 //
 // Pausing (kPause): once no more than half of the lanes that entered are left
 // walking, each of these puts its walk on its stack and leaves with
