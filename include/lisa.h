@@ -86,8 +86,8 @@ typedef struct lisa_stats {
   int32_t num_nodes;  /* internal BVH nodes (64 B each) */
   int32_t num_emitters; /* triangles whose material emits (the NEE light BVH) */
   uint64_t device_bytes; /* device memory held by the context */
-  int32_t wide_tree;  /* 1: the scene's Morton tree also has its 4-wide form, which
-                         lisa_trace_rays walks (lisa_set_wide_threshold) */
+  int32_t wide_tree;  /* 1: the scene's Morton tree also has its 4-wide form
+                         (lisa_set_wide_threshold) */
   int32_t reserved;
 } lisa_stats;
 
@@ -177,9 +177,10 @@ lisa_status lisa_get_stats(const lisa_ctx* ctx, lisa_stats* out);
 /* Scenes set from now on with at least min_triangles triangles (default
  * 2^20) also get the 4-wide form of their Morton tree (128 bytes per inner
  * node: each node's children, inner children replaced by their own two), and
- * lisa_trace_rays takes its hits from it: fewer, wider visits, which pay where
- * the tree streams from HBM.  (The path kernels that count nothing walk an
- * agglomerated 4-wide tree that every scene has.)  The hits are the same
+ * lisa_trace_rays takes its hits from a 4-wide walk: of the agglomerated tree
+ * that the path kernels walk, or of that form in a scene without one (a
+ * coordinate that is not finite, more than about 31 million triangles): fewer,
+ * wider visits, which pay where the tree streams from HBM.  The hits are the same
  * (closest hit, equal t to the lower triangle id); node-visit counters
  * (LISA_FLAG_COUNT) stay those of the binary tree.  0 gives every scene the
  * wide form.  No counterpart in the reference (OptiX chooses its acceleration

@@ -341,7 +341,7 @@ class Context:
 
     def set_wide_threshold(self, min_triangles):
         """Scenes set from now on with at least min_triangles triangles get the 4-wide
-        form of the Morton tree, which trace_rays walks (lisa_set_wide_threshold)."""
+        form of the Morton tree, and trace_rays a 4-wide walk (lisa_set_wide_threshold)."""
         self._ck(lib().lisa_set_wide_threshold(self.h, int(min_triangles)))
 
     def stats(self):

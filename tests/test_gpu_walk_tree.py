@@ -1,7 +1,7 @@
 """GPU: the agglomerated 4-wide tree that the path kernels walk.
 
-Bar: hit ids and t of lisa_trace_rays (which walks it below the 4-wide
-threshold) equal the oracle's brute-force loop bit for bit, and a render equals
+Bar: hit ids and t of lisa_trace_rays (which walks it from
+the wide threshold on) equal the oracle's brute-force loop bit for bit, and a render equals
 the counting build's, which walks the Morton tree, bit for bit -- at triangle
 counts around the clustering's workgroup sizes, with equal boxes, NaN and
 infinite vertices, rays along axes and from far away, and after both kinds of
@@ -47,8 +47,9 @@ def test_triangle_counts(capi, oracle_mod, T):
     o = oracle_mod.Scene(v, n, m, MATS)
     O, D = random_rays(1024, seed=T)
     with capi.Context(0) as ctx:
+        ctx.set_wide_threshold(0)
         ctx.set_scene(v, n, m, MATS)
-        assert not ctx.stats()["wide_tree"]
+        assert ctx.stats()["wide_tree"]
         gp, gt = ctx.trace_rays(O, D)
         rp, rt, _ = o.closest_hit(O, D, brute=True)
         assert np.array_equal(gp, rp) and _same(gt, rt)
@@ -69,6 +70,7 @@ def test_equal_boxes_and_slivers(capi, oracle_mod):
     o = oracle_mod.Scene(v, n, m, MATS)
     O, D = random_rays(2048, seed=3)
     with capi.Context(0) as ctx:
+        ctx.set_wide_threshold(0)
         ctx.set_scene(v, n, m, MATS)
         gp, gt = ctx.trace_rays(O, D)
         rp, rt, _ = o.closest_hit(O, D, brute=True)
@@ -85,6 +87,7 @@ def test_non_finite_vertices(capi, oracle_mod, bad):
     o = oracle_mod.Scene(v, n, m, MATS)
     O, D = random_rays(1024, seed=9)
     with capi.Context(0) as ctx:
+        ctx.set_wide_threshold(0)
         ctx.set_scene(v, n, m, MATS)
         gp, gt = ctx.trace_rays(O, D)
         rp, rt, _ = o.closest_hit(O, D, threads=8)
@@ -109,6 +112,7 @@ def test_axis_rays_and_far_origins(capi, oracle_mod, scale, shift):
     D[2560:3072] *= 1e-3
     O = (O.astype(np.float64) * scale + shift).astype(np.float32)
     with capi.Context(0) as ctx:
+        ctx.set_wide_threshold(0)
         ctx.set_scene(v, sc["normals"], sc["mat_idx"], sc["materials"])
         gp, gt = ctx.trace_rays(O, D)
         rp, rt, _ = o.closest_hit(O, D, brute=True)
@@ -122,6 +126,7 @@ def test_renders_equal_the_morton_walk(capi, name):
           "icosphere": lambda: scenes.displaced_icosphere(level=5, width=64, height=40, bounces=12),
           "batch": lambda: scenes.batch_scene(2)}[name]()
     with capi.Context(0) as ctx:
+        ctx.set_wide_threshold(0)
         ctx.set_scene(sc["verts"], sc["normals"], sc["mat_idx"], sc["materials"])
         U, V, Wv = camera(sc, capi)
         for flags in (0, capi.FLAG_FP64_ACCUM):
@@ -138,6 +143,7 @@ def test_follows_vertex_updates(capi, oracle_mod, T):
     w, _, _ = _soup(T, T + 2)
     O, D = random_rays(1024, seed=T)
     with capi.Context(0) as ctx:
+        ctx.set_wide_threshold(0)
         ctx.set_scene(v, n, m, MATS)
         for verts, device in ((w, False), (v, True)):
             if device:
@@ -179,6 +185,7 @@ def test_hits_at_the_edge_of_the_leaf_box(capi, oracle_mod):
     O, D = O.astype(np.float32), D.astype(np.float32)
     o = oracle_mod.Scene(v, n, m, MATS)
     with capi.Context(0) as ctx:
+        ctx.set_wide_threshold(0)
         ctx.set_scene(v, n, m, MATS)
         gp, gt = ctx.trace_rays(O, D)
         rp, rt, _ = o.closest_hit(O, D, threads=16)
