@@ -37,7 +37,7 @@ def _run(cmd):
 
 def build(verbose_resources=False, defines=(), out_dir=OUT, cli=True):
     """Compile liblisa.so (and the CLI) into out_dir; `defines` are extra
-    -D tuning macros (LISA_STACK_LDS, LISA_WALK_STACK, LISA_PATH_MIN_BLOCKS,
+    -D tuning macros (LISA_STACK_LDS, LISA_WALK_STACK, LISA_WALK_MAX_NODES, LISA_PATH_MIN_BLOCKS,
     LISA_MODE_WAVES, LISA_EMIT_WAVES, LISA_TILE_WAVES; LISA_PATH_BLOCK must stay 64: a workgroup is one wave)."""
     os.makedirs(out_dir, exist_ok=True)
     dev_o = os.path.join(out_dir, "lisa_device.o")
@@ -74,6 +74,16 @@ def build_small_stack():
     return build(defines=("LISA_STACK_LDS=2", "LISA_WALK_STACK=8"), out_dir=SMALL_STACK, cli=False)
 
 
+# Variant in which no scene gets the agglomerated walk tree, as scenes past
+# 2^25 walk nodes do not: every query is answered by the Morton trees.
+NO_WALK = os.path.join(OUT, "nowalk")
+
+
+def build_no_walk():
+    return build(defines=("LISA_WALK_MAX_NODES=0",), out_dir=NO_WALK, cli=False)
+
+
 if __name__ == "__main__":
     build(verbose_resources="-v" in sys.argv)
     build_small_stack()
+    build_no_walk()

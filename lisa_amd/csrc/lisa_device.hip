@@ -3338,8 +3338,14 @@ hipError_t wf_pending(hipStream_t st, const WfState& ws, uint32_t* pending) {
 // visits pay; below it the binary walk is the faster one.
 constexpr int64_t kWideMinTris = 1 << 20;
 // closest_walk addresses a node by a 32-bit byte offset: 2^25 nodes of 128
-// bytes, scenes of up to 31 million triangles; larger ones keep the Morton tree.
-constexpr size_t kWalkMaxNodes = size_t{1} << 25;
+// bytes, the scene's and its emitters' together (agg_capacity): scenes of up to
+// 31.4 million triangles with few emitters, of 15.7 million that all emit.
+// Larger ones keep the Morton tree.
+#ifndef LISA_WALK_MAX_NODES
+#define LISA_WALK_MAX_NODES (1 << 25)
+#endif
+constexpr size_t kWalkMaxNodes = LISA_WALK_MAX_NODES;
+static_assert(kWalkMaxNodes <= size_t{1} << 25, "32-bit byte offsets of the walk nodes");
 
 // lisa_render_progressive: n launches of the plain megakernel, one per
 // subframe, chained in one instantiated hipGraph; before each launch the
@@ -3639,9 +3645,21 @@ lisa_status build_walk(lisa_ctx* ctx) {
   return LISA_OK;
 }
 
-// Memory of the walk trees, and the emitters' places among the scene's
-// triangles (enqueued; `place` is T words of scratch).
-lisa_status prepare_walk(lisa_ctx* ctx, uint32_t* place) {
+// The emitters' places among the scene's triangles (enqueued; `place` is T words
+// of scratch): what a walk of the emitters' Morton tree, and their walk tree,
+// name a hit by -- also in a scene that gets no walk tree.
+lisa_status link_emitters(lisa_ctx* ctx, uint32_t* place) {
+  hipStream_t st = ctx->stream;
+  DevBvh &all = ctx->all, &emit = ctx->emit;
+  if (emit.T == 0) return LISA_OK;
+  k_place<<<grid_for(all.T, kBuildBlock), kBuildBlock, 0, st>>>(all.prim, all.T, place);
+  k_link<<<grid_for(emit.T, kBuildBlock), kBuildBlock, 0, st>>>(emit.prim, emit.T, place, emit.tris);
+  HIP_TRY(ctx, hipGetLastError());
+  return LISA_OK;
+}
+
+// Memory of the walk trees, in scenes that get them.
+lisa_status prepare_walk(lisa_ctx* ctx) {
   hipStream_t st = ctx->stream;
   DevBvh &all = ctx->all, &emit = ctx->emit;
   const size_t nodes = agg_capacity(all.T) + agg_capacity(emit.T);
@@ -3658,11 +3676,6 @@ lisa_status prepare_walk(lisa_ctx* ctx, uint32_t* place) {
     HIP_TRY(ctx, hipMemsetAsync(b->agg, 0xFF, 64 * cap, st));  // refs kEmpty: indexes that k_agg leaves out
   }
   HIP_TRY(ctx, hipMemsetAsync(all.tris + 3 * (size_t)all.T, 0, 48, st));  // the dummy triangle of empty slots
-  if (emit.T > 0) {
-    k_place<<<grid_for(all.T, kBuildBlock), kBuildBlock, 0, st>>>(all.prim, all.T, place);
-    k_link<<<grid_for(emit.T, kBuildBlock), kBuildBlock, 0, st>>>(emit.prim, emit.T, place, emit.tris);
-  }
-  HIP_TRY(ctx, hipGetLastError());
   return LISA_OK;
 }
 
@@ -4260,7 +4273,8 @@ lisa_status lisa_set_scene(lisa_ctx* ctx, const float* verts, const float* norma
     rc = build_bvh(ctx, ctx->emit, d_v, d_n, d_mat, d_gid, (int32_t)emit_ids.size(), nullptr);
   uint32_t* d_place = nullptr;
   if (rc == LISA_OK) HIP_TRY(ctx, S.alloc(&d_place, (size_t)T));
-  if (rc == LISA_OK) rc = prepare_walk(ctx, d_place);
+  if (rc == LISA_OK) rc = link_emitters(ctx, d_place);
+  if (rc == LISA_OK) rc = prepare_walk(ctx);
   if (rc == LISA_OK) rc = build_walk(ctx);
   if (rc != LISA_OK) return rc;
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
