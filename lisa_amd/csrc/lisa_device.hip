@@ -590,6 +590,23 @@ __device__ __forceinline__ int32_t closest_wide(const BvhView& bv, const RayT& r
   return best_k;
 }
 
+// The query of closest_walk() by the Morton trees of the scene or of its
+// emitters, kWide: by the scene's 4-wide form where it has one.  The index of an
+// emitter's hit is its triangle's place in `all`.
+template <int kStride, bool kWide>
+__device__ __forceinline__ int32_t closest_morton(const SceneView& sc, bool emitters, const RayT& r, float tmin,
+                                                  float tlim, uint32_t lim_prim, bool any, float& t_out,
+                                                  uint32_t* stk, volatile uint32_t* spill) {
+  if (kWide && !emitters && sc.all.wide)
+    return closest_wide<kStride>(sc.all, r, tmin, tlim, lim_prim, any, t_out, stk);
+  const BvhView bv{emitters ? sc.emit.nodes : sc.all.nodes, emitters ? sc.emit.tris : sc.all.tris,
+                   emitters ? sc.emit.T : sc.all.T, nullptr, nullptr, 0.0f};
+  TravCount tc;
+  int32_t k = closest<false, kStride>(bv, r, tmin, tlim, lim_prim, any, t_out, stk, spill, tc);
+  if (emitters && k >= 0) k = (int32_t)__float_as_uint(sc.emit.tris[3 * (size_t)k + 2].w);
+  return k;
+}
+
 // The same query over the walk tree (k_agg, k_walk_nodes): the scene's
 // triangles under an agglomerated 4-wide tree.  The accepted triangle is
 // closest()'s: the acceptance rule does not depend on the order of the tests,
@@ -776,14 +793,8 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
       done = done && slab(b[0], b[1], b[2], b[3], b[4], b[5], r, tmin, tlim * kWiden, tn);
     }
   }
-  if (!done) {
-    const BvhView slow{emitters ? sc.emit.nodes : sc.all.nodes, emitters ? sc.emit.tris : sc.all.tris,
-                       emitters ? sc.emit.T : sc.all.T, nullptr, nullptr, 0.0f};
-    TravCount tc;
-    best_k = closest<false, kStride>(slow, r, tmin, tlim, lim_prim, any, t_out, stk, spill, tc);
-    if (emitters && best_k >= 0)  // the triangle's place in `all`
-      best_k = (int32_t)__float_as_uint(sc.emit.tris[3 * (size_t)best_k + 2].w);
-  }
+  if (!done)
+    best_k = closest_morton<kStride, false>(sc, emitters, r, tmin, tlim, lim_prim, any, t_out, stk, spill);
   return best_k;
 }
 
@@ -953,9 +964,17 @@ enum Stage : int32_t {
 // suffix radiance (final - so far) / throughput of each vertex becomes a
 // training row at the sample's row slots.  Without accum_prev the launch writes its own mean (no
 // running mean over subframes; the subframe then only picks the RNG stream).
-template <bool kRecord, bool kCount, class Src, int kMode = 0, bool kF64 = false, class Bsdf = LISA_BSDF>
+//
+// kMorton: for scenes without a walk tree.  The Morton trees answer there, whose
+// walks do not pause, so that an NEE try's emitter query stays in the loop of the
+// tries, as in the counting builds: left to the round's walk, each try waits for
+// the other lanes' longest (an infinite vertex, so that no try is culled, 960x540,
+// 4 spp: Cornell box of 65k triangles 152 -> 36 ms, icosphere of 1.3M 743 -> 183).
+template <bool kRecord, bool kCount, class Src, int kMode = 0, bool kF64 = false, bool kMorton = false,
+          class Bsdf = LISA_BSDF>
 __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
-  constexpr bool kScan = !kCount && !kRecord;  // culled NEE tries by nee_scan, none seen one by one
+  // culled NEE tries by nee_scan, none seen one by one
+  constexpr bool kScan = !kCount && !kRecord && !kMorton;
   Job job{0, 0, 0};
   const bool work = src.next(job);
   if (!__ballot(work)) return;
@@ -997,7 +1016,6 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
 
   constexpr bool kQuery = kMode == 1 || kMode == 3;  // ends at the cache query
   constexpr bool kEmit = kMode == 3;                 // prefix emission in expectation
-  static_assert(kScan || !kEmit, "kMode 3 leaves the draws of a try to the NEE loop");
   uint32_t t_used = 0;  // kMode 2: vertex slots recorded in this sample
   // kMode 3: the current radiance ray is a bounce drawn on
   // the condition that it hits no emitter (redrawn when it does); lw is the
@@ -1227,6 +1245,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
           *light_mat = ent >> 1;
           tries = 0;
           stage = kTry;
+          if (!kScan) D = hemisphere_raw(seed);
           bounce = false;
         }
       } else {
@@ -1308,8 +1327,8 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     if (!__ballot(stage != kIdle)) break;
 
     // -- one traversal: the closest hit of a radiance ray, the any-hit query of
-    // an occlusion ray or (kScan) the emitter query of an NEE try or a light
-    // sample.
+    // an occlusion ray or the emitter query of an NEE try (kScan) or a light
+    // sample (kMode 3).
     if (stage == kIdle || stage == kTry) continue;
     const bool valid = ray_valid(D);
     int32_t k = -1;
@@ -1317,10 +1336,13 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
     if (valid && scp->all.T > 0) {
       const RayT r = make_ray(O, D);
       const bool any = stage == kAny || (kEmit && stage == kLightAny);
+      const bool emitters = stage == kTryEmit || (kEmit && stage == kLightEmit);
       if constexpr (kScan)
-        k = closest_walk<kPathBlock, true>(*scp, stage == kTryEmit || (kEmit && stage == kLightEmit), r, kTmin,
-                                           any ? tE : kTmax, any ? primE : 0xFFFFFFFFu, any, t, my_stk, spill,
-                                           paused);
+        k = closest_walk<kPathBlock, true>(*scp, emitters, r, kTmin, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu,
+                                           any, t, my_stk, spill, paused);
+      else if constexpr (kMorton)
+        k = closest_morton<kPathBlock, true>(*scp, emitters, r, kTmin, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu,
+                                             any, t, my_stk, spill);
       else
         k = closest<kCount, kPathBlock>(scp->all, r, kTmin, any ? tE : kTmax, any ? primE : 0xFFFFFFFFu, any, t,
                                         my_stk, spill, tc);
@@ -1415,7 +1437,7 @@ __device__ __forceinline__ void path_lane(Src& src, uint32_t* my_stk) {
         }
       }
       if (finish) stage = kSampleEnd;
-    } else if (kScan && (stage == kTryEmit || (kEmit && stage == kLightEmit))) {
+    } else if ((kScan && stage == kTryEmit) || (kEmit && stage == kLightEmit)) {
       // the closest emitter of an NEE try or a light sample
       float4 e0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), e1 = e0;
       if (k >= 0) {
@@ -1506,21 +1528,21 @@ struct OnePixel {
   }
 };
 
-template <bool kRecord, bool kCount, bool kF64 = false>
+template <bool kRecord, bool kCount, bool kF64 = false, bool kMorton = false>
 __global__ __launch_bounds__(kPathBlock, (kRecord || kCount) ? 4 : LISA_PATH_MIN_BLOCKS) void k_path(SceneView sc, PathArgs p) {
   __shared__ uint32_t stk[kLaneLds * kPathBlock];
   OnePixel src{sc, p, false};
-  path_lane<kRecord, kCount, OnePixel, 0, kF64>(src, stk + threadIdx.x);
+  path_lane<kRecord, kCount, OnePixel, 0, kF64, kMorton>(src, stk + threadIdx.x);
 }
 
 // Path loop in a cache mode (1: cached render of the full image in tiles,
 // 2: training paths on a pixel list).
-template <int kMode>
+template <int kMode, bool kMorton = false>
 __global__ __launch_bounds__(kPathBlock, kMode == 3 ? LISA_EMIT_WAVES : LISA_MODE_WAVES) void k_path_mode(
     SceneView sc, PathArgs p) {
   __shared__ uint32_t stk[kLaneLds * kPathBlock];
   OnePixel src{sc, p, false};
-  path_lane<false, false, OnePixel, kMode>(src, stk + threadIdx.x);
+  path_lane<false, false, OnePixel, kMode, false, kMorton>(src, stk + threadIdx.x);
 }
 
 // One scene's pixels from a device counter, for persistent launches: the
@@ -1573,12 +1595,12 @@ struct PixelQueue {
 // Persistent form of the path loop (kMode as in k_path_mode, 0 = plain):
 // `total` work indices (pixels of the list, or 64 per 8x8 tile) handed out
 // by `counter`, which must be zero at launch.
-template <int kMode>
+template <int kMode, bool kMorton = false>
 __global__ __launch_bounds__(kPathBlock, kMode == 3 ? LISA_MODE_WAVES : 1) void k_path_pq(
     SceneView sc, PathArgs p, uint32_t* counter, uint32_t total, uint32_t chunk) {
   __shared__ uint32_t stk[kLaneLds * kPathBlock];
   PixelQueue src{sc, p, counter, total, chunk, 0u, 0u};
-  path_lane<false, false, PixelQueue, kMode>(src, stk + threadIdx.x);
+  path_lane<false, false, PixelQueue, kMode, false, kMorton>(src, stk + threadIdx.x);
 }
 
 // frame[item] += throughput * max(network output, 0) / spp for every query.
@@ -1728,6 +1750,7 @@ struct QueueSrc {
   }
 };
 
+template <bool kMorton>
 __global__ __launch_bounds__(kPathBlock) void k_path_queue(const BatchScene* scenes, int32_t n,
                                                            uint32_t* counter, uint32_t total,
                                                            uint32_t chunk) {
@@ -1740,7 +1763,7 @@ __global__ __launch_bounds__(kPathBlock) void k_path_queue(const BatchScene* sce
   src.chunk = chunk;
   src.cur = src.end = 0;
   src.bs = scenes;
-  path_lane<false, false>(src, stk + threadIdx.x);
+  path_lane<false, false, QueueSrc, 0, false, kMorton>(src, stk + threadIdx.x);
 }
 
 // The wave-tile form of the batched launch: each wave takes one 8x8 tile of
@@ -1767,6 +1790,7 @@ struct TileSrc {
   }
 };
 
+template <bool kMorton>
 __global__ __launch_bounds__(kPathBlock, LISA_TILE_WAVES) void k_path_tiles(const BatchScene* scenes, int32_t n,
                                                            uint32_t* counter, uint32_t total) {
   __shared__ uint32_t stk[kLaneLds * kPathBlock];
@@ -1786,7 +1810,7 @@ __global__ __launch_bounds__(kPathBlock, LISA_TILE_WAVES) void k_path_tiles(cons
     }
     lo = __builtin_amdgcn_readfirstlane(lo);
     TileSrc src{scenes + lo, t - scenes[lo].first / 64u, false};
-    path_lane<false, false, TileSrc>(src, stk + threadIdx.x);
+    path_lane<false, false, TileSrc, 0, false, kMorton>(src, stk + threadIdx.x);
   }
 }
 
@@ -3443,6 +3467,7 @@ struct lisa_batch {
   std::vector<size_t> accum_px;
   std::vector<uint64_t> gens;  // each context's generation when the batch was made
   uint32_t total = 0;
+  bool morton = false;  // a scene has no walk tree: every scene by its Morton trees
   hipStream_t stream = nullptr;
   BatchScene* d_scenes = nullptr;
   uint32_t* d_counter = nullptr;
@@ -3510,6 +3535,10 @@ SceneView view(const lisa_ctx* c) {
                    make_float4(c->ecull_h[0], c->ecull_h[1], c->ecull_h[2], 0.0f),
                    (uint32_t)agg_capacity(c->all.T)};
 }
+
+// Whether the scene has no walk tree, so that the path kernels walk its Morton
+// trees (kMorton).
+bool no_walk(const lisa_ctx* c) { return c->all.T > 0 && !view(c).all.walk; }
 
 // Device scratch, given back to the context's pool at scope exit.
 struct Scratch {
@@ -3765,6 +3794,13 @@ lisa_status refit_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
   return LISA_OK;
 }
 
+// The plain path kernel of the context's scene.
+using PathKernel = void (*)(SceneView, PathArgs);
+PathKernel plain_path(const lisa_ctx* ctx, bool f64) {
+  if (no_walk(ctx)) return f64 ? k_path<false, false, true, true> : k_path<false, false, false, true>;
+  return f64 ? k_path<false, false, true> : k_path<false, false>;
+}
+
 }  // namespace
 
 // Persistent launch of the path loop in mode kMode over `a`'s pixel list or
@@ -3785,7 +3821,8 @@ lisa_status launch_persistent(lisa_ctx* ctx, PathArgs a, int slot) {
     total = a.tiles_x * ((a.height + 7) / 8) * 64u;
   }
   const unsigned blocks = (unsigned)(ctx->cus * kPersistentBlocksPerCu);
-  k_path_pq<kMode><<<blocks, kPathBlock, 0, st>>>(view(ctx), a, counter, total, 1u);
+  const auto path = no_walk(ctx) ? k_path_pq<kMode, true> : k_path_pq<kMode>;
+  path<<<blocks, kPathBlock, 0, st>>>(view(ctx), a, counter, total, 1u);
   HIP_TRY(ctx, hipGetLastError());
   return LISA_OK;
 }
@@ -3972,7 +4009,8 @@ lisa_status trace_train_rows(lisa_ctx* ctx, PathArgs a, const int32_t* d_pix, si
   a.t_row = ctx->c_trow.p;
   a.t_n = ctx->c_tn.p;
   a.t_depth = depth;
-  k_path_mode<2><<<grid_for((int64_t)n, kPathBlock), kPathBlock, 0, st>>>(view(ctx), a);
+  const auto path = no_walk(ctx) ? k_path_mode<2, true> : k_path_mode<2>;
+  path<<<grid_for((int64_t)n, kPathBlock), kPathBlock, 0, st>>>(view(ctx), a);
   HIP_TRY(ctx, hipGetLastError());
   lisa_status rc = scan_counts(ctx, ctx->c_tn.p, paths, ctx->c_tscan, ctx->c_qcount.p + 1, st);
   if (rc != LISA_OK) return rc;
@@ -4026,10 +4064,10 @@ lisa_status trace_queries_launch(lisa_ctx* ctx, PathArgs& a, const int32_t* d_pi
       a.tiles_x = (a.width + kTileW - 1) / kTileW;
       blocks = a.tiles_x * ((a.height + kTileH - 1) / kTileH);
     }
-    if (a.emit_expect)
-      k_path_mode<3><<<blocks, kPathBlock, 0, st>>>(view(ctx), a);
-    else
-      k_path_mode<1><<<blocks, kPathBlock, 0, st>>>(view(ctx), a);
+    const bool morton = no_walk(ctx);
+    const auto path = a.emit_expect ? (morton ? k_path_mode<3, true> : k_path_mode<3>)
+                                    : (morton ? k_path_mode<1, true> : k_path_mode<1>);
+    path<<<blocks, kPathBlock, 0, st>>>(view(ctx), a);
     HIP_TRY(ctx, hipGetLastError());
   }
   return LISA_OK;
@@ -4333,10 +4371,8 @@ lisa_status lisa_render(lisa_ctx* ctx, const lisa_render_params* p, float* accum
     k_path<false, true, true><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
   else if (count)
     k_path<false, true><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
-  else if (a.fp64)
-    k_path<false, false, true><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
   else
-    k_path<false, false><<<grid, kPathBlock, 0, st>>>(view(ctx), a);
+    plain_path(ctx, a.fp64)<<<grid, kPathBlock, 0, st>>>(view(ctx), a);
   HIP_TRY(ctx, hipGetLastError());
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
   if (rgba8_out) {
@@ -4395,8 +4431,7 @@ lisa_status lisa_render_progressive(lisa_ctx* ctx, const lisa_render_params* p, 
   a.counters = ctx->d_counters;
   a.sum64 = f64 ? ctx->c_sum64.p : nullptr;
   SceneView sv = view(ctx);
-  void* const fn = f64 ? reinterpret_cast<void*>(&k_path<false, false, true>)
-                       : reinterpret_cast<void*>(&k_path<false, false>);
+  void* const fn = reinterpret_cast<void*>(plain_path(ctx, f64));
   auto node_params = [&](PathArgs& pa, void** args) {
     hipKernelNodeParams kp;
     std::memset(&kp, 0, sizeof(kp));
@@ -4671,6 +4706,7 @@ lisa_status lisa_batch_create(lisa_batch** out, lisa_ctx* const* ctxs,
   }
   b->device = dev;
   b->total = (uint32_t)total;
+  b->morton = std::any_of(ctxs, ctxs + n, [](const lisa_ctx* c) { return no_walk(c); });
   b->stream = ctxs[0]->stream;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, dev) == hipSuccess) b->cus = prop.multiProcessorCount;
@@ -4747,11 +4783,14 @@ static hipError_t enqueue_batch(lisa_batch* b) {
     return e != hipSuccess ? e : enqueue_batch_rounds(b);
   }
   k_queue_reset<<<1, 1, 0, b->stream>>>(b->d_counter);
-  if (b->cfg.form == 1)
-    k_path_tiles<<<b->cfg.grid_blocks, kPathBlock, 0, b->stream>>>(b->d_scenes, b->n, b->d_counter, b->total);
-  else
-    k_path_queue<<<b->cfg.grid_blocks, kPathBlock, 0, b->stream>>>(b->d_scenes, b->n, b->d_counter, b->total,
-                                                                   (uint32_t)b->cfg.chunk);
+  if (b->cfg.form == 1) {
+    const auto tiles = b->morton ? k_path_tiles<true> : k_path_tiles<false>;
+    tiles<<<b->cfg.grid_blocks, kPathBlock, 0, b->stream>>>(b->d_scenes, b->n, b->d_counter, b->total);
+  } else {
+    const auto queue = b->morton ? k_path_queue<true> : k_path_queue<false>;
+    queue<<<b->cfg.grid_blocks, kPathBlock, 0, b->stream>>>(b->d_scenes, b->n, b->d_counter, b->total,
+                                                            (uint32_t)b->cfg.chunk);
+  }
   return hipGetLastError();
 }
 
@@ -5031,7 +5070,7 @@ lisa_status lisa_render_cached(lisa_ctx* ctx, lisa_cache* cache, const lisa_rend
       if (rc != LISA_OK) return rc;
     } else {
       const unsigned tiles = ((p->width + kTileW - 1) / kTileW) * ((p->height + kTileH - 1) / kTileH);
-      k_path<false, false><<<tiles, kPathBlock, 0, st>>>(view(ctx), a);
+      plain_path(ctx, false)<<<tiles, kPathBlock, 0, st>>>(view(ctx), a);
       HIP_TRY(ctx, hipGetLastError());
     }
     HIP_TRY(ctx, hipStreamSynchronize(st));

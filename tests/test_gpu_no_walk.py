@@ -59,3 +59,27 @@ def test_hits_without_a_walk_tree(capi, oracle_mod, no_walk):
         rp, rt, _ = oracle_mod.Scene(v, n, m, mats).closest_hit(O, D, brute=True)
         for wide in (False, True):
             assert _same(no_walk[f"{wide} {name} prim"], rp) and _same(no_walk[f"{wide} {name} t"], rt)
+
+
+def test_an_infinite_vertex_costs_no_rounds(capi):
+    """A scene that loses its walk tree to an infinite vertex, and with it the cull of
+    NEE tries: the render takes no longer than the counting one, which walks the
+    same trees (left to the round's walk, each try's emitter query made it take four
+    times as long)."""
+    from lisa_amd import scenes
+    from tests.scene_util import camera
+    sc = scenes.cornell_65k()
+    v = np.array(sc["verts"], np.float32)
+    v[1000, 4] = np.inf
+    with capi.Context(0) as ctx:
+        ctx.set_scene(v, sc["normals"], sc["mat_idx"], sc["materials"])
+        U, V, W = camera(sc, capi)
+        ms, img = {}, {}
+        for flags in (0, capi.FLAG_COUNT):
+            p = capi.render_params(320, 320, 4, 7, sc["camera"]["eye"], U, V, W, flags=flags)
+            for _ in range(3):
+                img[flags], _ = ctx.render(p)
+                ms[flags] = min(ms.get(flags, 1e9), ctx.stats()["render_ms"])
+        print(ms, flush=True)
+        assert _same(img[0], img[capi.FLAG_COUNT])
+        assert ms[0] < 1.5 * ms[capi.FLAG_COUNT]
