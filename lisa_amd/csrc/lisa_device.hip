@@ -827,9 +827,13 @@ __global__ __launch_bounds__(kRayBlock) void k_trace_rays(SceneView sc, const fl
     // counts stay the binary walk's, which alone serves the smaller scenes: a
     // second walk there made the kernel of 10^5 rays 0.166 ms instead of 0.120
     // (65k triangles), of 2*10^6 0.989 instead of 0.877.
-    if (sc.all.wide && sc.all.walk)
+    // A limit below zero, or a direction so short that t passes 2^60 scenes, is no
+    // path's: closest_walk's box test does not cover them, and the binary walk's hit
+    // stands.
+    const bool four = tmin >= 0.0f && fabsf(r.Sz) <= 0x1p60f;
+    if (sc.all.wide && sc.all.walk && four)
       k = closest_walk<kRayBlock>(sc, false, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x, spill, paused);
-    else if (sc.all.wide)
+    else if (sc.all.wide && !sc.all.walk)
       k = closest_wide<kRayBlock>(sc.all, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x);
     if (k >= 0) prim = (int32_t)__float_as_uint(sc.all.tris[3 * (size_t)k].w);
   }
