@@ -39,6 +39,8 @@ constexpr uint32_t kLeaf = 0x80000000u;
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 // 1 + 2*gamma(3) (Ize, "Robust BVH Ray Traversal", JCGT 2013).
 constexpr float kRobust = 0x1.000006p+0f;
+// Share of a coordinate by which closest_walk's box planes stand further out.
+constexpr float kBoxMargin = 0x1p-20f;
 // Boxes are culled against the best hit distance widened by 2^-16, so a
 // triangle whose hit lies on its box boundary (axis-aligned or coplanar
 // geometry, where the slab entry can round a few ulp above the triangle's t)
@@ -615,13 +617,21 @@ __device__ __forceinline__ int32_t closest_morton(const SceneView& sc, bool emit
 //
 // Box tests: t = l / D - O / D as one fused multiply-add per plane with the
 // near and far planes picked by the sign of D (the node's float4s are loaded
-// in that order).  Its error is below 5u (|O| + span) / |D| (u = 2^-24), so
-// the near planes are moved by e = 2^-20 (|O| + span) / |D| towards the
-// origin and the far planes away from it, which covers that error and the
-// slack of slab()'s own rounding and kRobust (12u of t).  An axis whose
-// arithmetic overflows gives NaN and is left out of the test.  A direction
-// component of zero takes 1 / D = 2^100: a plane on the wrong side of the
-// origin is then at t < -2^60 or > 2^60.
+// in that order).  With slab()'s rounded 1 / D, both stand at t = (l - O) / D but for
+// rounding: slab() is within 2u |t| (u = 2^-24), kRobust adds 6u |t|, the multiply-add
+// is within u |t| + 2u |O / D|, and |t| is at most |l / D| + |O / D|.  So the planes are
+// stored kBoxMargin |l| = 16u |l| further out (k_walk_nodes), and e = 16u |O / D| moves
+// the near ones towards the origin and the far ones away from it.
+// Nothing depends on the scene's size: with a margin of its span, one far triangle
+// made every box near a ray pass (Cornell box of 65k triangles, an emitting quad at
+// 10^5, 512^2, 4 spp: 224 ms against 5.3; without the quad 1.33 either way; C2 22.1
+// either way.  The relative part as a factor of the far t, four products a node,
+// made a batch scene 3 % slower).  An axis whose arithmetic overflows gives NaN and is
+// left out of the test.  A direction component of zero (or below 2^-100) takes 1 / D =
+// 2^100 and adds 2^40 (|O| + span) to e: a far plane at the origin is then past every
+// t of the other axes (their 1 / D are below 2^30: path directions have length one,
+// lisa_trace_rays sees to its own), and a near plane 2^-60 (|O| + span) behind the
+// origin's rounding is too.
 //
 // An iteration visits an inner node and then tests a triangle if the lane
 // holds one, so the wave runs one copy of the triangle test per iteration
@@ -670,11 +680,13 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
     const F3 inv = mk(fabsf(r.inv.x) <= big ? r.inv.x : copysignf(big, r.inv.x),
                       fabsf(r.inv.y) <= big ? r.inv.y : copysignf(big, r.inv.y),
                       fabsf(r.inv.z) <= big ? r.inv.z : copysignf(big, r.inv.z));
+    auto margin = [&](float o, float u, float inv0) {
+      return __builtin_fmaf(fabsf(u), kBoxMargin, fabsf(inv0) <= big ? 0x1p-126f : (fabsf(o) + bv.span) * 0x1p40f);
+    };
     const float ux = r.O.x * inv.x, uy = r.O.y * inv.y, uz = r.O.z * inv.z;
-    const float ex = (fabsf(r.O.x) + bv.span) * fabsf(inv.x) * 0x1p-20f;
-    const float ey = (fabsf(r.O.y) + bv.span) * fabsf(inv.y) * 0x1p-20f;
-    const float ez = (fabsf(r.O.z) + bv.span) * fabsf(inv.z) * 0x1p-20f;
-    const F3 on = mk(-ux - ex, -uy - ey, -uz - ez), of = mk(ex - ux, ey - uy, ez - uz);
+    const float ex = margin(r.O.x, ux, r.inv.x), ey = margin(r.O.y, uy, r.inv.y), ez = margin(r.O.z, uz, r.inv.z);
+    const F3 on = mk(-ux - ex, -uy - ey, -uz - ez);
+    const F3 of = mk(ex - ux, ey - uy, ez - uz);
     // byte offsets of the near planes in a node: lo at 0, hi at 16
     const uint32_t sx = inv.x < 0.0f ? 16u : 0u, sy = inv.y < 0.0f ? 16u : 0u, sz = inv.z < 0.0f ? 16u : 0u;
     const char* __restrict__ base = bv.walk;
@@ -827,10 +839,9 @@ __global__ __launch_bounds__(kRayBlock) void k_trace_rays(SceneView sc, const fl
     // counts stay the binary walk's, which alone serves the smaller scenes: a
     // second walk there made the kernel of 10^5 rays 0.166 ms instead of 0.120
     // (65k triangles), of 2*10^6 0.989 instead of 0.877.
-    // A limit below zero, or a direction so short that t passes 2^60 scenes, is no
-    // path's: closest_walk's box test does not cover them, and the binary walk's hit
-    // stands.
-    const bool four = tmin >= 0.0f && fabsf(r.Sz) <= 0x1p60f;
+    // A limit below zero, or a direction shorter than 2^-30, is no path's: closest_walk's
+    // box test does not cover them, and the binary walk's hit stands.
+    const bool four = tmin >= 0.0f && fabsf(r.Sz) <= 0x1p30f;
     if (sc.all.wide && sc.all.walk && four)
       k = closest_walk<kRayBlock>(sc, false, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x, spill, paused);
     else if (sc.all.wide && !sc.all.walk)
@@ -3142,9 +3153,13 @@ __global__ __launch_bounds__(kBuildBlock) void k_walk_nodes(const float4* __rest
       ref[s] = kLeaf | __float_as_uint(links[3 * (size_t)(ref[s] & ~kLeaf) + 2].w);
   }
   float4* w = walk + 8 * ((size_t)first + n);
+  // the planes kBoxMargin further out (closest_walk); an empty slot's stay infinite
+  auto out = [](float v, float m) { return fabsf(v) < INFINITY ? __builtin_fmaf(fabsf(v), m, v) : v; };
   for (int a = 0; a < 3; ++a) {
-    w[2 * a] = make_float4(lo[0][a], lo[1][a], lo[2][a], lo[3][a]);
-    w[2 * a + 1] = make_float4(hi[0][a], hi[1][a], hi[2][a], hi[3][a]);
+    w[2 * a] = make_float4(out(lo[0][a], -kBoxMargin), out(lo[1][a], -kBoxMargin), out(lo[2][a], -kBoxMargin),
+                           out(lo[3][a], -kBoxMargin));
+    w[2 * a + 1] = make_float4(out(hi[0][a], kBoxMargin), out(hi[1][a], kBoxMargin), out(hi[2][a], kBoxMargin),
+                               out(hi[3][a], kBoxMargin));
   }
   w[6] = make_float4(__uint_as_float(ref[0]), __uint_as_float(ref[1]), __uint_as_float(ref[2]),
                      __uint_as_float(ref[3]));

@@ -47,7 +47,26 @@ def test_hits_with_a_far_quad(capi, oracle_mod, d):
         assert np.array_equal(gp, rp) and _same(gt, rt)
 
 
-@pytest.mark.parametrize("scale,tmin", [(1e-25, 1e-4), (1e-33, 1e-4), (1e-36, 1.0), (1e30, 1e-34), (1.0, -1.0),
+def test_a_far_quad_costs_no_boxes(capi):
+    """A margin of the scene's span made every box near a ray pass (26 times the
+    time of the counting render)."""
+    sc = cornell(256, 128, 256, 256, 2, 5)
+    v, n, m, mats = _far_quad(sc, 1e5)
+    U, V, W = camera(sc, capi)
+    with capi.Context(0) as ctx:
+        ctx.set_scene(v, n, m, mats)
+        ms, img = {}, {}
+        for flags in (0, capi.FLAG_COUNT):
+            p = capi.render_params(256, 256, 2, 5, sc["camera"]["eye"], U, V, W, flags=flags)
+            for _ in range(3):
+                img[flags], _ = ctx.render(p)
+                ms[flags] = min(ms.get(flags, 1e9), ctx.stats()["render_ms"])
+        print(ms, flush=True)
+        assert _same(img[0], img[capi.FLAG_COUNT])
+        assert ms[0] < 1.5 * ms[capi.FLAG_COUNT]
+
+
+@pytest.mark.parametrize("scale,tmin", [(1e-9, 1e-4), (1e-25, 1e-4), (1e-33, 1e-4), (1e-36, 1.0), (1e30, 1e-34), (1.0, -1.0),
                                         (1.0, 0.0)])
 def test_directions_and_limits_no_path_makes(capi, oracle_mod, scale, tmin):
     sc = cornell(32, 16, 16, 16, 1, 1)
