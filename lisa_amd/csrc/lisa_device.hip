@@ -731,17 +731,25 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
   bool done = false;
   int32_t best_k = -1;
   if (bv.walk) {
-    const float big = 0x1p100f;
-    const F3 inv = mk(fabsf(r.inv.x) <= big ? r.inv.x : copysignf(big, r.inv.x),
-                      fabsf(r.inv.y) <= big ? r.inv.y : copysignf(big, r.inv.y),
-                      fabsf(r.inv.z) <= big ? r.inv.z : copysignf(big, r.inv.z));
-    auto margin = [&](float o, float u, float inv0) {
-      return __builtin_fmaf(fabsf(u), kBoxMargin, fabsf(inv0) <= big ? 0x1p-126f : (fabsf(o) + bv.span) * 0x1p40f);
-    };
+    F3 inv = r.inv;
     const float ux = r.O.x * inv.x, uy = r.O.y * inv.y, uz = r.O.z * inv.z;
-    const float ex = margin(r.O.x, ux, r.inv.x), ey = margin(r.O.y, uy, r.inv.y), ez = margin(r.O.z, uz, r.inv.z);
-    const F3 on = mk(-ux - ex, -uy - ey, -uz - ez);
-    const F3 of = mk(ex - ux, ey - uy, ez - uz);
+    F3 on = mk(__builtin_fmaf(fabsf(ux), -kBoxMargin, -ux), __builtin_fmaf(fabsf(uy), -kBoxMargin, -uy),
+               __builtin_fmaf(fabsf(uz), -kBoxMargin, -uz));
+    F3 of = mk(__builtin_fmaf(fabsf(ux), kBoxMargin, -ux), __builtin_fmaf(fabsf(uy), kBoxMargin, -uy),
+               __builtin_fmaf(fabsf(uz), kBoxMargin, -uz));
+    constexpr float big = 0x1p100f;
+    if (fmaxf(fmaxf(fabsf(inv.x), fabsf(inv.y)), fabsf(inv.z)) > big) {
+      auto clamp = [&](float o, float& v, float& n, float& f) {
+        if (fabsf(v) <= big) return;
+        v = copysignf(big, v);
+        const float u = o * v, e = __builtin_fmaf(fabsf(u), kBoxMargin, (fabsf(o) + bv.span) * 0x1p40f);
+        n = -u - e;
+        f = e - u;
+      };
+      clamp(r.O.x, inv.x, on.x, of.x);
+      clamp(r.O.y, inv.y, on.y, of.y);
+      clamp(r.O.z, inv.z, on.z, of.z);
+    }
     // byte offsets of the near planes in a node: lo at 0, hi at 16
     const uint32_t sx = inv.x < 0.0f ? 16u : 0u, sy = inv.y < 0.0f ? 16u : 0u, sz = inv.z < 0.0f ? 16u : 0u;
     const char* __restrict__ base = bv.walk;
@@ -894,9 +902,10 @@ __global__ __launch_bounds__(kRayBlock) void k_trace_rays(SceneView sc, const fl
     // counts stay the binary walk's, which alone serves the smaller scenes: a
     // second walk there made the kernel of 10^5 rays 0.166 ms instead of 0.120
     // (65k triangles), of 2*10^6 0.989 instead of 0.877.
-    // A limit below zero, or a direction shorter than 2^-30, is no path's: closest_walk's
-    // box test does not cover them, and the binary walk's hit stands.
-    const bool four = tmin >= 0.0f && fabsf(r.Sz) <= 0x1p30f;
+    // A limit below zero, or a direction shorter than 2^-30 or longer than 2^30, is no
+    // path's: closest_walk's box test does not cover them, and the binary walk's hit
+    // stands.
+    const bool four = tmin >= 0.0f && fabsf(r.Sz) <= 0x1p30f && fabsf(r.Sz) >= 0x1p-30f;
     if (sc.all.wide && sc.all.walk && four)
       k = closest_walk<kRayBlock>(sc, false, r, tmin, tmax, 0xFFFFFFFFu, false, t, stk + threadIdx.x, spill, paused);
     else if (sc.all.wide && !sc.all.walk)
