@@ -81,7 +81,7 @@ typedef struct lisa_render_params {
 
 typedef struct lisa_stats {
   float render_ms;    /* last render/trace kernel time (HIP events on the context stream) */
-  float bvh_build_ms; /* last lisa_set_scene device build time */
+  float bvh_build_ms; /* device time of the last lisa_set_scene's build or vertex update's refit */
   int32_t num_tris;
   int32_t num_nodes;  /* internal BVH nodes (64 B each) */
   int32_t num_emitters; /* triangles whose material emits (the NEE light BVH) */
@@ -114,10 +114,12 @@ lisa_status lisa_set_scene(lisa_ctx* ctx, const float* verts, const float* norma
  * for the T triangles of the current scene: triangle records are rewritten
  * in the build's Morton order and both LBVHs are refit bottom-up, keeping
  * topology and Morton codes (animated / re-posed geometry; cheaper than a
- * rebuild, box quality degrades with large motion); a 4-wide form of the
- * tree is rebuilt from the refitted one, and the tree that renders walk is
- * clustered anew from the moved triangles.  No counterpart in the
- * reference, whose GAS is built once (optix_wrapper.cc:104-106). */
+ * rebuild, box quality degrades with large motion).  The tree that renders
+ * walk is clustered anew from the moved triangles by the first call that walks
+ * it (its time is in that call, render_ms included): a caller that goes on to
+ * move vertices, or to lisa_trace_rays in a smaller scene, does not pay for it.
+ * No counterpart in the reference, whose GAS is built once
+ * (optix_wrapper.cc:104-106). */
 lisa_status lisa_update_vertices(lisa_ctx* ctx, const float* verts, const float* normals);
 
 /* lisa_update_vertices for callers that cannot allocate device memory (code

@@ -3502,6 +3502,7 @@ struct lisa_ctx {
   uint64_t scene_bytes = 0, accum_bytes = 0;
   float bmin[3] = {0, 0, 0}, bmax[3] = {1, 1, 1};  // scene box (cache features)
   float span = 0.0f;                               // its largest |coordinate|
+  bool walk_stale = false, wide_stale = false;     // the triangles moved since (ready_trees)
   float ecull_c[3] = {0, 0, 0}, ecull_h[3] = {INFINITY, INFINITY, INFINITY};  // never culls
   int32_t n_cull = 0;  // nee_scan's boxes, in c_ecdf; below 0: the cull box alone
   // radiance-cache frame scratch (lisa_render_cached), grown on demand
@@ -3732,14 +3733,6 @@ lisa_status refit_levels(lisa_ctx* ctx, DevBvh& b) {
   return refit_levels_on(ctx, b, ta, tb);
 }
 
-// The 4-wide form of b from its nodes (when b has one), on stream st.
-lisa_status wide_nodes(lisa_ctx* ctx, DevBvh& b, hipStream_t st) {
-  if (!b.wide || b.T == 0) return LISA_OK;
-  k_wide<<<grid_for(b.nI, kBuildBlock), kBuildBlock, 0, st>>>(b.nodes, b.nI, b.wide);
-  HIP_TRY(ctx, hipGetLastError());
-  return LISA_OK;
-}
-
 // The walk trees of the scene and of its emitters (their triangle records are
 // in place and linked), enqueued on the context's stream: no allocation, no wait.
 lisa_status build_walk(lisa_ctx* ctx) {
@@ -3783,6 +3776,35 @@ lisa_status link_emitters(lisa_ctx* ctx, uint32_t* place) {
   k_place<<<grid_for(all.T, kBuildBlock), kBuildBlock, 0, st>>>(all.prim, all.T, place);
   k_link<<<grid_for(emit.T, kBuildBlock), kBuildBlock, 0, st>>>(emit.prim, emit.T, place, emit.tris);
   HIP_TRY(ctx, hipGetLastError());
+  return LISA_OK;
+}
+
+// Brings the tree that the scene's walks take up to date with its triangles, on the
+// context's stream: the walk trees, or in a scene without them the 4-wide form of
+// the Morton tree, if it has one.  Every call that launches such walks makes it
+// first.  lisa_set_scene makes the walk trees itself; a vertex update leaves the one
+// or the other to the first call that walks it, and whoever only moves vertices or
+// traces rays through the binary tree pays for neither.  (Cornell box of 65k
+// triangles, on the host's clock: lisa_update_vertices_noalloc 0.32 -> 0.14 ms, with a
+// 256^2 frame of 1 spp after each 0.75 -> 0.76; the 4-wide form of 5.2M triangles,
+// which nothing read while there was a walk tree, was 671 MB of writes in each load
+// and update: lisa_set_scene 22.0 -> 21.3 ms, lisa_update_vertices 10.7 -> 8.9.)
+// *built (optional): whether something was enqueued, for callers whose kernels run on
+// another stream.
+lisa_status ready_trees(lisa_ctx* ctx, bool* built = nullptr) {
+  DevBvh& all = ctx->all;
+  const bool walk = view(ctx).all.walk != nullptr;
+  bool& stale = walk ? ctx->walk_stale : ctx->wide_stale;
+  if (built) *built = stale;
+  if (!stale) return LISA_OK;
+  if (walk) {
+    lisa_status rc = build_walk(ctx);
+    if (rc != LISA_OK) return rc;
+  } else if (all.wide && all.T > 0) {
+    k_wide<<<grid_for(all.nI, kBuildBlock), kBuildBlock, 0, ctx->stream>>>(all.nodes, all.nI, all.wide);
+    HIP_TRY(ctx, hipGetLastError());
+  }
+  stale = false;
   return LISA_OK;
 }
 
@@ -3869,8 +3891,6 @@ lisa_status build_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
     lisa_status rc = refit_levels(ctx, b);
     if (rc != LISA_OK) return rc;
   }
-  lisa_status rw = wide_nodes(ctx, b, st);
-  if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipGetLastError());
   return LISA_OK;
 }
@@ -3887,8 +3907,6 @@ lisa_status refit_bvh(lisa_ctx* ctx, DevBvh& b, const float* d_v, const float* d
     lisa_status rc = refit_levels(ctx, b);
     if (rc != LISA_OK) return rc;
   }
-  lisa_status rw = wide_nodes(ctx, b, st);
-  if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipGetLastError());
   return LISA_OK;
 }
@@ -4299,9 +4317,9 @@ lisa_status lisa_update_vertices(lisa_ctx* ctx, const float* verts, const float*
   }
   hipStream_t st = ctx->stream;
   HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
+  ctx->walk_stale = ctx->wide_stale = true;
   lisa_status rc = refit_bvh(ctx, ctx->all, d_v, d_n, ctx->d_nrm);
   if (rc == LISA_OK) rc = refit_bvh(ctx, ctx->emit, d_v, nullptr, nullptr);
-  if (rc == LISA_OK) rc = build_walk(ctx);
   if (rc != LISA_OK) return rc;
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
   HIP_TRY(ctx, hipStreamSynchronize(st));
@@ -4327,6 +4345,7 @@ lisa_status lisa_update_vertices_noalloc(lisa_ctx* ctx, const float* d_verts, co
   float4* const tb = ptr + 2 * (size_t)kNoAllocMaxTris;
   hipStream_t st = ctx->stream;
   HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
+  ctx->walk_stale = ctx->wide_stale = true;
   DevBvh* trees[2] = {&ctx->all, &ctx->emit};
   for (DevBvh* b : trees) {
     if (b->T == 0) continue;
@@ -4339,11 +4358,7 @@ lisa_status lisa_update_vertices_noalloc(lisa_ctx* ctx, const float* d_verts, co
       lisa_status rc = refit_levels_on(ctx, *b, ta, tb);
       if (rc != LISA_OK) return rc;
     }
-    lisa_status rw = wide_nodes(ctx, *b, st);
-    if (rw != LISA_OK) return rw;
   }
-  lisa_status rw = build_walk(ctx);
-  if (rw != LISA_OK) return rw;
   HIP_TRY(ctx, hipGetLastError());
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
   HIP_TRY(ctx, hipStreamSynchronize(st));
@@ -4496,6 +4511,8 @@ lisa_status lisa_set_scene(lisa_ctx* ctx, const float* verts, const float* norma
   if (rc == LISA_OK) rc = prepare_walk(ctx);
   if (rc == LISA_OK) rc = build_walk(ctx);
   if (rc != LISA_OK) return rc;
+  ctx->walk_stale = false;
+  ctx->wide_stale = true;  // its first walk makes it
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
   HIP_TRY(ctx, hipStreamSynchronize(st));
   HIP_TRY(ctx, hipEventElapsedTime(&ctx->bvh_ms, ctx->ev0, ctx->ev1));
@@ -4541,6 +4558,10 @@ lisa_status lisa_render(lisa_ctx* ctx, const lisa_render_params* p, float* accum
   if (count)
     HIP_TRY(ctx, hipMemsetAsync(ctx->d_counters, 0, LISA_NCOUNTERS * sizeof(unsigned long long), st));
   HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
+  if (!count) {
+    rc = ready_trees(ctx);
+    if (rc != LISA_OK) return rc;
+  }
   const unsigned grid = a.tiles_x * tiles_y;
   if (p->flags & LISA_FLAG_WAVEFRONT) {
     lisa_status rc2 = render_wavefront(ctx, a);
@@ -4656,7 +4677,11 @@ lisa_status lisa_render_progressive(lisa_ctx* ctx, const lisa_render_params* p, 
     e = hipGraphExecKernelNodeSetParams(g.exec, g.nodes[(size_t)i], &kp);
   }
   if (e == hipSuccess) e = hipEventRecord(ctx->ev0, ctx->stream);
-  if (e == hipSuccess) e = hipGraphLaunch(g.exec, ctx->stream);
+  if (e == hipSuccess) {
+    rc = ready_trees(ctx);
+    if (rc != LISA_OK) return rc;
+    e = hipGraphLaunch(g.exec, ctx->stream);
+  }
   if (e == hipSuccess) e = hipEventRecord(ctx->ev1, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
@@ -4754,6 +4779,10 @@ lisa_status lisa_trace_rays(lisa_ctx* ctx, const float* O, const float* D, int32
   hipStream_t st = ctx->stream;
   HIP_TRY(ctx, hipMemsetAsync(ctx->d_counters, 0, LISA_NCOUNTERS * sizeof(unsigned long long), st));
   HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
+  if (ctx->all.wide) {
+    lisa_status rc = ready_trees(ctx);
+    if (rc != LISA_OK) return rc;
+  }
   k_trace_rays<true><<<grid_for(n, kRayBlock), kRayBlock, 0, st>>>(view(ctx), d_o, d_d, n, tmin, tmax,
                                                                    d_p, d_t, ctx->d_counters);
   HIP_TRY(ctx, hipGetLastError());
@@ -4863,6 +4892,12 @@ lisa_status lisa_batch_create(lisa_batch** out, lisa_ctx* const* ctxs,
     if (c->accum_px != npx && ensure_accum(c, npx) != LISA_OK) {
       lisa::set_global_error("batch scene " + std::to_string(i) + ": " + c->err);
       return LISA_ERR_ALLOC;
+    }
+    // the batch's launches are on another context's stream
+    bool built = false;
+    if (ready_trees(c, &built) != LISA_OK || (built && hipStreamSynchronize(c->stream) != hipSuccess)) {
+      lisa::set_global_error("batch scene " + std::to_string(i) + ": " + c->err);
+      return LISA_ERR_HIP;
     }
     PathArgs a = make_args(&params[i]);
     a.tiles_x = (params[i].width + 7) / 8;
@@ -5187,6 +5222,10 @@ lisa_status lisa_render_cached(lisa_ctx* ctx, lisa_cache* cache, const lisa_rend
   PathArgs base = cache_args(ctx, p);
   float loss = 0.0f;
   HIP_TRY(ctx, ctx->c_frame.ensure(npx));
+  bool built = false;
+  rc = ready_trees(ctx, &built);
+  if (rc != LISA_OK) return rc;
+  if (built) HIP_TRY(ctx, hipStreamSynchronize(st));  // the training paths may run on a second stream
   // The frame's prefix paths do not read the network, so without a fallback
   // decision (which waits for this frame's loss) they run on the context's
   // stream while the training steps run on the cache's.
@@ -5397,6 +5436,8 @@ lisa_status lisa_cache_trace_queries(lisa_ctx* ctx, const lisa_render_params* p,
   rc = upload_pixels(ctx, p, pixels, n);
   if (rc != LISA_OK) return rc;
   HIP_TRY(ctx, ctx->c_frame.ensure((size_t)n));
+  rc = ready_trees(ctx);
+  if (rc != LISA_OK) return rc;
   PathArgs a = cache_args(ctx, p);
   a.emit_expect = pre.emit_expect;
   a.nee_loops = pre.nee_loops;
@@ -5428,6 +5469,7 @@ lisa_status lisa_cache_trace_rows(lisa_ctx* ctx, const lisa_render_params* p, co
     return fail(ctx, LISA_ERR_INVALID_ARG, "n * spp * row slots per sample >= 2^31");
   HIP_TRY(ctx, hipSetDevice(ctx->device));
   rc = upload_pixels(ctx, p, pixels, n);
+  if (rc == LISA_OK) rc = ready_trees(ctx);
   if (rc != LISA_OK) return rc;
   PathArgs a = cache_args(ctx, p);
   uint32_t rows = 0;
