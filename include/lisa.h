@@ -85,7 +85,9 @@ typedef struct lisa_stats {
   int32_t num_tris;
   int32_t num_nodes;  /* internal BVH nodes (64 B each) */
   int32_t num_emitters; /* triangles whose material emits (the NEE light BVH) */
-  uint64_t device_bytes; /* device memory held by the context */
+  uint64_t device_bytes; /* device memory of the scene and the accum buffer; not the work buffers of FP64,
+                            byte, cached and wavefront frames, nor the freed scene memory kept for the
+                            next scene (at most 1 GiB, given back when an allocation fails) */
   int32_t wide_tree;  /* 1: the scene's Morton tree also has its 4-wide form
                          (lisa_set_wide_threshold) */
   int32_t reserved;

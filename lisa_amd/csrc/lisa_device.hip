@@ -30,6 +30,7 @@
 #include "lisa.h"
 #include "lisa_internal.h"
 #include "lisa_math.h"
+#include "lisa_pool.h"
 
 using namespace lisa;
 
@@ -3260,92 +3261,6 @@ struct DevBvh {
   uint64_t bytes = 0;
 };
 
-// Device buffer that only grows: reallocated when a call needs more.
-template <typename T>
-struct DevBuf {
-  T* p = nullptr;
-  size_t cap = 0;
-  hipError_t ensure(size_t want) {
-    if (p && want <= cap) return hipSuccess;
-    (void)hipFree(p);
-    p = nullptr;
-    cap = 0;
-    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&p), std::max<size_t>(want, 1) * sizeof(T));
-    if (e == hipSuccess) cap = want;
-    return e;
-  }
-  void release() {
-    (void)hipFree(p);
-    p = nullptr;
-    cap = 0;
-  }
-};
-
-// A context's scene memory and the scratch of its builds.  hipMalloc and
-// hipFree of a scene's two dozen buffers took longer than building its trees
-// (292k triangles: lisa_set_scene 4.2 ms, of which kernels and copies 1.5), and a
-// program that loads or moves scenes on one context asks for the same sizes
-// again: blocks go back to a list and are handed out to requests of at least
-// half their size.  A block is only handed to work on the context's stream (or
-// behind a copy that waits for it), so one that is given back while the stream
-// still uses it is safe.  The list keeps at most kPoolFree bytes and is
-// released with the context.
-constexpr size_t kPoolFree = size_t{1} << 30;
-struct DevPool {
-  struct Block {
-    void* p;
-    size_t n;
-  };
-  std::vector<Block> idle, used;
-  hipError_t take(void** p, size_t want) {
-    want = (std::max<size_t>(want, 1) + 255) / 256 * 256;
-    size_t best = idle.size();
-    for (size_t i = 0; i < idle.size(); ++i)
-      if (idle[i].n >= want && idle[i].n <= 2 * want + 65536 && (best == idle.size() || idle[i].n < idle[best].n))
-        best = i;
-    if (best < idle.size()) {
-      used.push_back(idle[best]);
-      idle.erase(idle.begin() + (long)best);
-      *p = used.back().p;
-      return hipSuccess;
-    }
-    hipError_t e = hipMalloc(p, want);
-    if (e != hipSuccess && !idle.empty()) {
-      (void)hipGetLastError();
-      trim(0);
-      e = hipMalloc(p, want);
-    }
-    if (e == hipSuccess) used.push_back(Block{*p, want});
-    return e;
-  }
-  void give(void* p) {
-    if (!p) return;
-    for (size_t i = used.size(); i-- > 0;)
-      if (used[i].p == p) {
-        idle.push_back(used[i]);
-        used.erase(used.begin() + (long)i);
-        return;
-      }
-  }
-  void trim(size_t keep) {  // the largest idle blocks first
-    size_t sum = 0;
-    for (const Block& b : idle) sum += b.n;
-    while (sum > keep) {
-      size_t big = 0;
-      for (size_t i = 1; i < idle.size(); ++i)
-        if (idle[i].n > idle[big].n) big = i;
-      sum -= idle[big].n;
-      (void)hipFree(idle[big].p);
-      idle.erase(idle.begin() + (long)big);
-    }
-  }
-  void release() {
-    trim(0);
-    for (const Block& b : used) (void)hipFree(b.p);
-    used.clear();
-  }
-};
-
 // Device memory of lisa_update_vertices_noalloc (the refit for callers that
 // cannot allocate): the two union tables of the level refit, 2 float4 per
 // triangle each, for scenes of at most kNoAllocMaxTris triangles (64 MB per
@@ -3367,14 +3282,14 @@ struct WfBuffers {
   BatchScene* d_scenes = nullptr;
   int32_t scene_cap = 0;
   WfState ws{};
-  hipError_t ensure(uint32_t slots) {
+  hipError_t ensure(uint32_t slots, DevPool* const* pools, size_t n) {
     const size_t P = ((size_t)slots + 63) / 64 * 64;
     const size_t want = P * (7 * 16 + 16 + 8 + 4 + 4) + 256;
     if (!mem || want > bytes) {
       (void)hipFree(mem);
       mem = nullptr;
       bytes = 0;
-      const hipError_t e = hipMalloc(&mem, want);
+      const hipError_t e = dev_alloc(&mem, want, pools, n);
       if (e != hipSuccess) return e;
       bytes = want;
     }
@@ -3396,12 +3311,13 @@ struct WfBuffers {
     ws.slots = slots;
     return hipSuccess;
   }
-  hipError_t ensure_scenes(int32_t n) {
+  hipError_t ensure_scenes(int32_t n, DevPool* const* pools, size_t n_pools) {
     if (d_scenes && n <= scene_cap) return hipSuccess;
     (void)hipFree(d_scenes);
     d_scenes = nullptr;
     scene_cap = 0;
-    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&d_scenes), sizeof(BatchScene) * (size_t)n);
+    const hipError_t e = dev_alloc(reinterpret_cast<void**>(&d_scenes), sizeof(BatchScene) * (size_t)n, pools,
+                                   n_pools);
     if (e == hipSuccess) scene_cap = n;
     return e;
   }
@@ -3553,6 +3469,7 @@ struct lisa_ctx {
 struct lisa_batch {
   int32_t device = 0, n = 0, cus = 256;
   std::vector<lisa_ctx*> ctxs;
+  std::vector<DevPool*> pools;  // the contexts', which make room for the batch's buffers
   std::vector<lisa_render_params> params;
   std::vector<size_t> accum_px;
   std::vector<uint64_t> gens;  // each context's generation when the batch was made
@@ -3641,22 +3558,8 @@ int scene_kind(const lisa_ctx* c) {
 }
 
 // Device scratch, given back to the context's pool at scope exit.
-struct Scratch {
-  DevPool& pool;
-  std::vector<void*> ptrs;
-  explicit Scratch(lisa_ctx* ctx) : pool(ctx->pool) {}
-  ~Scratch() {
-    for (void* p : ptrs) pool.give(p);
-    pool.trim(kPoolFree);
-  }
-  template <typename T>
-  hipError_t alloc(T** p, size_t count) {
-    void* q = nullptr;
-    const hipError_t e = pool.take(&q, std::max<size_t>(count, 1) * sizeof(T));
-    *p = static_cast<T*>(q);
-    if (e == hipSuccess) ptrs.push_back(q);
-    return e;
-  }
+struct Scratch : PoolScratch {
+  explicit Scratch(lisa_ctx* ctx) : PoolScratch(ctx->pool) {}
 };
 
 inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
@@ -3670,7 +3573,8 @@ lisa_status ensure_accum(lisa_ctx* ctx, size_t npx) {
   ctx->gen++;
   ctx->j_seq = false;
   ctx->sum64_valid = false;
-  HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->d_accum), npx * sizeof(float4)));
+  DevPool* const pool = &ctx->pool;
+  HIP_TRY(ctx, dev_alloc(reinterpret_cast<void**>(&ctx->d_accum), npx * sizeof(float4), &pool, 1));
   ctx->accum_px = npx;
   ctx->accum_bytes = npx * sizeof(float4);
   return LISA_OK;
@@ -3808,21 +3712,30 @@ lisa_status ready_trees(lisa_ctx* ctx, bool* built = nullptr) {
   return LISA_OK;
 }
 
-// Memory of the walk trees, in scenes that get them.
+// Memory of the walk trees, in scenes that get them: all of it or none.  Where it is
+// not to be had, the scene keeps the Morton trees, as one past the node limit does.
 lisa_status prepare_walk(lisa_ctx* ctx) {
   hipStream_t st = ctx->stream;
   DevBvh &all = ctx->all, &emit = ctx->emit;
   const size_t nodes = agg_capacity(all.T) + agg_capacity(emit.T);
   if (all.T == 0 || nodes > kWalkMaxNodes) return LISA_OK;
-  HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&all.walk), 128 * nodes));
+  auto chunks = [](const DevBvh& b) { return ((size_t)b.T + kAggChunk - 1) / kAggChunk; };
+  PoolWant wants[7] = {{reinterpret_cast<void**>(&all.walk), 128 * nodes}};
+  size_t n = 1;
+  for (DevBvh* b : {&all, &emit}) {
+    if (b->T == 0) continue;
+    wants[n++] = {reinterpret_cast<void**>(&b->agg), 64 * agg_capacity(b->T)};
+    wants[n++] = {reinterpret_cast<void**>(&b->lists), 64 * chunks(*b) * kAggOut};
+    wants[n++] = {reinterpret_cast<void**>(&b->counts), 8 * chunks(*b)};
+  }
+  const hipError_t e = ctx->pool.take_all(wants, n);
+  if (e == hipErrorOutOfMemory) return LISA_OK;
+  HIP_TRY(ctx, e);
   all.bytes += 128 * nodes;
   for (DevBvh* b : {&all, &emit}) {
     if (b->T == 0) continue;
-    const size_t cap = agg_capacity(b->T), chunks = ((size_t)b->T + kAggChunk - 1) / kAggChunk;
-    HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b->agg), 64 * cap));
-    HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b->lists), 64 * chunks * kAggOut));
-    HIP_TRY(ctx, ctx->pool.take(reinterpret_cast<void**>(&b->counts), 8 * chunks));
-    b->bytes += 64 * cap + 64 * chunks * kAggOut + 8 * chunks;
+    const size_t cap = agg_capacity(b->T);
+    b->bytes += 64 * cap + 64 * chunks(*b) * kAggOut + 8 * chunks(*b);
     HIP_TRY(ctx, hipMemsetAsync(b->agg, 0xFF, 64 * cap, st));  // refs kEmpty: indexes that k_agg leaves out
   }
   HIP_TRY(ctx, hipMemsetAsync(all.tris + 3 * (size_t)all.T, 0, 48, st));  // the dummy triangle of empty slots
@@ -3940,7 +3853,7 @@ constexpr int kPersistentBlocksPerCu = 20;
 template <int kMode>
 lisa_status launch_persistent(lisa_ctx* ctx, PathArgs a, int slot) {
   hipStream_t st = ctx->stream;
-  HIP_TRY(ctx, ctx->c_qcount.ensure(64));
+  HIP_TRY(ctx, ctx->c_qcount.ensure(64, ctx->pool));
   uint32_t* counter = ctx->c_qcount.p + slot;
   HIP_TRY(ctx, hipMemsetAsync(counter, 0, 4, st));
   uint32_t total;
@@ -3966,8 +3879,9 @@ lisa_status render_wavefront(lisa_ctx* ctx, PathArgs a) {
   a.tiles_x = (a.width + 7) / 8;
   const uint32_t total = a.tiles_x * ((a.height + 7) / 8) * 64u;
   const uint32_t slots = std::min<uint32_t>(total, (uint32_t)ctx->cus * kWfWavesPerCu * kWfBlock * 2u);
-  HIP_TRY(ctx, ctx->wf.ensure(slots));
-  HIP_TRY(ctx, ctx->wf.ensure_scenes(1));
+  DevPool* const pool = &ctx->pool;
+  HIP_TRY(ctx, ctx->wf.ensure(slots, &pool, 1));
+  HIP_TRY(ctx, ctx->wf.ensure_scenes(1, &pool, 1));
   BatchScene hs;
   hs.sc = view(ctx);
   hs.p = a;
@@ -4132,7 +4046,7 @@ lisa_status read_scene_box(lisa_ctx* ctx, bool may_alloc = true) {
   // light sampling of LISA_CACHE_EMISSION: area prefix sums of the emitters
   const int32_t TE = ctx->emit.T, n_chunks = (TE + kCdfChunk - 1) / kCdfChunk;
   if (may_alloc)
-    HIP_TRY(ctx, ctx->c_ecdf.ensure(ecdf_words(TE)));
+    HIP_TRY(ctx, ctx->c_ecdf.ensure(ecdf_words(TE), ctx->pool));
   else if (ctx->c_ecdf.cap < ecdf_words(TE))  // sized by lisa_set_scene for these emitters
     return fail(ctx, LISA_ERR_ALLOC, "emitter prefix-sum buffer smaller than the scene's emitters");
   float* chunk_tot = ctx->c_ecdf.p + TE;
@@ -4177,7 +4091,7 @@ PathArgs cache_args(const lisa_ctx* ctx, const lisa_render_params* p) {
 lisa_status scan_counts(lisa_ctx* ctx, const uint8_t* cnt, size_t n, DevBuf<uint32_t>& offs,
                         uint32_t* d_total, hipStream_t st) {
   const size_t nb = (n + kScanItems - 1) / kScanItems;
-  HIP_TRY(ctx, offs.ensure(nb));
+  HIP_TRY(ctx, offs.ensure(nb, ctx->pool));
   if (nb > 0) k_scan_chunks<<<(unsigned)nb, 256, 0, st>>>(cnt, n, offs.p);
   k_scan_top<<<1, 256, 0, st>>>(offs.p, (uint32_t)nb, d_total);
   HIP_TRY(ctx, hipGetLastError());
@@ -4194,13 +4108,13 @@ lisa_status trace_train_rows(lisa_ctx* ctx, PathArgs a, const int32_t* d_pix, si
   // vertex slots per path: one hit per sample at a fixed depth, else up to one per bounce
   const size_t slots = depth > 0 ? 1 : a.bounces;
   const size_t paths = n * a.spp;
-  HIP_TRY(ctx, ctx->c_trec.ensure(n * slots * 18));
-  HIP_TRY(ctx, ctx->c_trow.ensure(paths * slots * 15));
-  HIP_TRY(ctx, ctx->c_tn.ensure(paths));
-  HIP_TRY(ctx, ctx->c_tfeat.ensure(cap * 12));
-  HIP_TRY(ctx, ctx->c_ttgt.ensure(cap * 3));
-  HIP_TRY(ctx, ctx->c_tacc.ensure(n));
-  HIP_TRY(ctx, ctx->c_qcount.ensure(64));
+  HIP_TRY(ctx, ctx->c_trec.ensure(n * slots * 18, ctx->pool));
+  HIP_TRY(ctx, ctx->c_trow.ensure(paths * slots * 15, ctx->pool));
+  HIP_TRY(ctx, ctx->c_tn.ensure(paths, ctx->pool));
+  HIP_TRY(ctx, ctx->c_tfeat.ensure(cap * 12, ctx->pool));
+  HIP_TRY(ctx, ctx->c_ttgt.ensure(cap * 3, ctx->pool));
+  HIP_TRY(ctx, ctx->c_tacc.ensure(n, ctx->pool));
+  HIP_TRY(ctx, ctx->c_qcount.ensure(64, ctx->pool));
   HIP_TRY(ctx, hipMemsetAsync(ctx->c_tn.p, 0, paths, st));
   a.pixels = d_pix;
   a.n_items = (int32_t)n;
@@ -4236,13 +4150,13 @@ lisa_status trace_queries_launch(lisa_ctx* ctx, PathArgs& a, const int32_t* d_pi
                                  float4* frame, bool persistent, bool full = false) {
   hipStream_t st = ctx->stream;
   const size_t slots = full ? 0 : n * a.spp;
-  HIP_TRY(ctx, ctx->c_qrec.ensure(slots * 4));
-  HIP_TRY(ctx, ctx->c_qhas.ensure(slots));
-  HIP_TRY(ctx, ctx->c_qfeat.ensure(slots * 12));
-  HIP_TRY(ctx, ctx->c_qatt.ensure(slots * 3));
-  HIP_TRY(ctx, ctx->c_qout.ensure(slots * 3));
-  HIP_TRY(ctx, ctx->c_qitem.ensure(slots));
-  HIP_TRY(ctx, ctx->c_qcount.ensure(64));
+  HIP_TRY(ctx, ctx->c_qrec.ensure(slots * 4, ctx->pool));
+  HIP_TRY(ctx, ctx->c_qhas.ensure(slots, ctx->pool));
+  HIP_TRY(ctx, ctx->c_qfeat.ensure(slots * 12, ctx->pool));
+  HIP_TRY(ctx, ctx->c_qatt.ensure(slots * 3, ctx->pool));
+  HIP_TRY(ctx, ctx->c_qout.ensure(slots * 3, ctx->pool));
+  HIP_TRY(ctx, ctx->c_qitem.ensure(slots, ctx->pool));
+  HIP_TRY(ctx, ctx->c_qcount.ensure(64, ctx->pool));
   if (slots > 0) HIP_TRY(ctx, hipMemsetAsync(ctx->c_qhas.p, 0, slots, st));
   a.pixels = d_pix;
   a.n_items = (int32_t)n;
@@ -4536,13 +4450,14 @@ lisa_status lisa_render(lisa_ctx* ctx, const lisa_render_params* p, float* accum
     rc = ensure_accum(ctx, npx);
     if (rc != LISA_OK) return rc;
   }
+  if (rgba8_out) HIP_TRY(ctx, ctx->c_rgba8.ensure(npx, ctx->pool));
   ctx->j_seq = false;  // the buffer now holds a plain render
   const bool f64 = (p->flags & LISA_FLAG_FP64_ACCUM) != 0;
   if (f64) {
     if (p->subframe > 0 && !ctx->sum64_valid)
       return fail(ctx, LISA_ERR_INVALID_ARG,
                   "FP64 subframe > 0 needs the FP64 sums of subframe 0 (or lisa_accum64_load)");
-    HIP_TRY(ctx, ctx->c_sum64.ensure(npx));
+    HIP_TRY(ctx, ctx->c_sum64.ensure(npx, ctx->pool));
   }
   ctx->sum64_valid = false;  // set again when an FP64 render succeeds
   PathArgs a = make_args(p);
@@ -4578,7 +4493,6 @@ lisa_status lisa_render(lisa_ctx* ctx, const lisa_render_params* p, float* accum
   HIP_TRY(ctx, hipGetLastError());
   HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
   if (rgba8_out) {
-    HIP_TRY(ctx, ctx->c_rgba8.ensure(npx));
     k_srgb<<<grid_for((int64_t)npx, 256), 256, 0, st>>>(ctx->d_accum, (int64_t)npx, lisa::srgb_steps(),
                                                        ctx->c_rgba8.p);
     HIP_TRY(ctx, hipGetLastError());
@@ -4621,7 +4535,7 @@ lisa_status lisa_render_progressive(lisa_ctx* ctx, const lisa_render_params* p, 
     if (p->subframe > 0 && !ctx->sum64_valid)
       return fail(ctx, LISA_ERR_INVALID_ARG,
                   "FP64 subframe > 0 needs the FP64 sums of subframe 0 (or lisa_accum64_load)");
-    HIP_TRY(ctx, ctx->c_sum64.ensure(npx));
+    HIP_TRY(ctx, ctx->c_sum64.ensure(npx, ctx->pool));
   }
   ctx->sum64_valid = false;  // set again when an FP64 run succeeds
   PathArgs a = make_args(p);
@@ -4855,7 +4769,7 @@ lisa_status lisa_accum64_load(lisa_ctx* ctx, const double* sums, int64_t n_pixel
     if (rc != LISA_OK) return rc;
   }
   ctx->j_seq = false;
-  HIP_TRY(ctx, ctx->c_sum64.ensure(npx));
+  HIP_TRY(ctx, ctx->c_sum64.ensure(npx, ctx->pool));
   HIP_TRY(ctx, hipMemcpyAsync(ctx->c_sum64.p, sums, npx * sizeof(double4), hipMemcpyHostToDevice, ctx->stream));
   k_mean64<<<grid_for((int64_t)npx, 256), 256, 0, ctx->stream>>>(ctx->c_sum64.p, (int64_t)npx, ctx->d_accum);
   HIP_TRY(ctx, hipGetLastError());
@@ -4913,6 +4827,7 @@ lisa_status lisa_batch_create(lisa_batch** out, lisa_ctx* const* ctxs,
   if (total >= (1ull << 32) - (1ull << 20)) return fail(nullptr, LISA_ERR_INVALID_ARG, "batch too large");
   lisa_batch* b = new lisa_batch;
   b->ctxs.assign(ctxs, ctxs + n);
+  for (lisa_ctx* c : b->ctxs) b->pools.push_back(&c->pool);
   b->params.assign(params, params + n);
   b->accum_px.resize(n);
   b->gens.resize(n);
@@ -4929,8 +4844,8 @@ lisa_status lisa_batch_create(lisa_batch** out, lisa_ctx* const* ctxs,
   b->cfg.grid_blocks = b->cus * 16;
   b->cfg.chunk = 1;
   hipError_t e;
-  if ((e = hipMalloc(reinterpret_cast<void**>(&b->d_scenes), sizeof(BatchScene) * n)) != hipSuccess ||
-      (e = hipMalloc(reinterpret_cast<void**>(&b->d_counter), 256)) != hipSuccess ||
+  if ((e = dev_alloc(reinterpret_cast<void**>(&b->d_scenes), sizeof(BatchScene) * n, b->pools.data(), b->pools.size())) != hipSuccess ||
+      (e = dev_alloc(reinterpret_cast<void**>(&b->d_counter), 256, b->pools.data(), b->pools.size())) != hipSuccess ||
       (e = hipMemcpy(b->d_scenes, hs.data(), sizeof(BatchScene) * n, hipMemcpyHostToDevice)) != hipSuccess ||
       (e = hipEventCreate(&b->ev0)) != hipSuccess || (e = hipEventCreate(&b->ev1)) != hipSuccess) {
     lisa_batch_destroy(b);
@@ -5021,7 +4936,7 @@ lisa_status lisa_batch_render(lisa_batch* b, float* elapsed_ms) {
   if (hipSetDevice(b->device) != hipSuccess) return fail(nullptr, LISA_ERR_HIP, "hipSetDevice");
   hipError_t e;
   if (!b->exec && b->cfg.graph) {  // capture reset + persistent launch once, replay afterwards
-    if (b->cfg.form == 2 && (e = b->wf.ensure(wf_batch_slots(b))) != hipSuccess)
+    if (b->cfg.form == 2 && (e = b->wf.ensure(wf_batch_slots(b), b->pools.data(), b->pools.size())) != hipSuccess)
       return fail(nullptr, LISA_ERR_ALLOC, std::string("wavefront buffers: ") + hipGetErrorString(e));
     e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
@@ -5060,7 +4975,7 @@ lisa_status lisa_batch_render(lisa_batch* b, float* elapsed_ms) {
       b->cfg.graph = 0;
     }
   }
-  if (b->cfg.form == 2 && (e = b->wf.ensure(wf_batch_slots(b))) != hipSuccess)
+  if (b->cfg.form == 2 && (e = b->wf.ensure(wf_batch_slots(b), b->pools.data(), b->pools.size())) != hipSuccess)
     return fail(nullptr, LISA_ERR_ALLOC, std::string("wavefront buffers: ") + hipGetErrorString(e));
   for (int32_t i = 0; i < b->n; ++i) {  // each accum buffer will hold a plain render
     b->ctxs[i]->j_seq = false;
@@ -5212,8 +5127,8 @@ lisa_status lisa_render_cached(lisa_ctx* ctx, lisa_cache* cache, const lisa_rend
       ctx->j_pix[i] = (int32_t)(z % npx);
     }
     if (nj > 0) {
-      HIP_TRY(ctx, ctx->c_jpix.ensure(nj));
-      HIP_TRY(ctx, ctx->c_jout.ensure(nj));
+      HIP_TRY(ctx, ctx->c_jpix.ensure(nj, ctx->pool));
+      HIP_TRY(ctx, ctx->c_jout.ensure(nj, ctx->pool));
       HIP_TRY(ctx, hipMemcpy(ctx->c_jpix.p, ctx->j_pix.data(), 4 * nj, hipMemcpyHostToDevice));
     }
   }
@@ -5221,7 +5136,7 @@ lisa_status lisa_render_cached(lisa_ctx* ctx, lisa_cache* cache, const lisa_rend
   const bool taken_over = ctx->j_from >= 0 && (int64_t)p->subframe >= ctx->j_from;
   PathArgs base = cache_args(ctx, p);
   float loss = 0.0f;
-  HIP_TRY(ctx, ctx->c_frame.ensure(npx));
+  HIP_TRY(ctx, ctx->c_frame.ensure(npx, ctx->pool));
   bool built = false;
   rc = ready_trees(ctx, &built);
   if (rc != LISA_OK) return rc;
@@ -5253,7 +5168,7 @@ lisa_status lisa_render_cached(lisa_ctx* ctx, lisa_cache* cache, const lisa_rend
     }
     const size_t nt = cp->train_paths;
     const size_t cap = cp->train_max > 0 ? cp->train_max : nt * cp->train_bounces;
-    HIP_TRY(ctx, ctx->c_tpix.ensure(nt));
+    HIP_TRY(ctx, ctx->c_tpix.ensure(nt, ctx->pool));
     k_train_pixels<<<grid_for((int64_t)nt, 256), 256, 0, ts>>>(
         ctx->c_tpix.p, (uint32_t)nt, cp->seed * 0x9E3779B97F4A7C15ull + p->subframe + 1, (uint32_t)npx);
     HIP_TRY(ctx, hipGetLastError());
@@ -5349,8 +5264,8 @@ lisa_status lisa_render_cached(lisa_ctx* ctx, lisa_cache* cache, const lisa_rend
     jp.subframe = p->subframe ^ 0x20000000u;
     jp.flags = 0;
     const size_t ns = (size_t)nj * p->spp;
-    HIP_TRY(ctx, ctx->c_jacc.ensure((size_t)nj));
-    HIP_TRY(ctx, ctx->c_jrgb.ensure(3 * ns));
+    HIP_TRY(ctx, ctx->c_jacc.ensure((size_t)nj, ctx->pool));
+    HIP_TRY(ctx, ctx->c_jrgb.ensure(3 * ns, ctx->pool));
     PathArgs ja = make_args(&jp);  // the plain loop on the judge pixels, per-sample radiance kept
     ja.pixels = ctx->c_jpix.p;
     ja.n_items = nj;
@@ -5412,7 +5327,7 @@ lisa_status upload_pixels(lisa_ctx* ctx, const lisa_render_params* p, const int3
   const int64_t npx = (int64_t)p->width * p->height;
   for (int32_t i = 0; i < n; ++i)
     if (pixels[i] < 0 || pixels[i] >= npx) return fail(ctx, LISA_ERR_INVALID_ARG, "pixel id out of range");
-  HIP_TRY(ctx, ctx->c_tpix.ensure((size_t)n));
+  HIP_TRY(ctx, ctx->c_tpix.ensure((size_t)n, ctx->pool));
   HIP_TRY(ctx, hipMemcpy(ctx->c_tpix.p, pixels, 4 * (size_t)n, hipMemcpyHostToDevice));
   return LISA_OK;
 }
@@ -5435,7 +5350,7 @@ lisa_status lisa_cache_trace_queries(lisa_ctx* ctx, const lisa_render_params* p,
   HIP_TRY(ctx, hipSetDevice(ctx->device));
   rc = upload_pixels(ctx, p, pixels, n);
   if (rc != LISA_OK) return rc;
-  HIP_TRY(ctx, ctx->c_frame.ensure((size_t)n));
+  HIP_TRY(ctx, ctx->c_frame.ensure((size_t)n, ctx->pool));
   rc = ready_trees(ctx);
   if (rc != LISA_OK) return rc;
   PathArgs a = cache_args(ctx, p);
