@@ -3531,9 +3531,15 @@ void free_scene(lisa_ctx* c) {
 
 constexpr int32_t kCdfChunk = 64;  // emitters per chunk of the area prefix sums (k_emit_chunks)
 // Words of c_ecdf for TE emitters: the prefix sums, the chunks' bases, then from
-// cull_head() on two words of results (k_emit_add, k_emit_bases) and the cull boxes.
-inline size_t cull_head(int32_t TE) { return ((size_t)TE + (TE + kCdfChunk - 1) / kCdfChunk + 3) / 4 * 4; }
-inline size_t ecdf_words(int32_t TE) { return cull_head(TE) + 4 + 8 * kCullBoxes; }
+// scene_head() on what read_scene_box() reads back, and the cull boxes.
+struct SceneHead {
+  float area;       // of the emitters (k_emit_add)
+  int32_t n_cull;   // their cull boxes, below 0: none (k_emit_bases)
+  int32_t pad[2];
+  float4 root[8];   // the root nodes of the scene's and the emitters' Morton trees
+};
+inline size_t scene_head(int32_t TE) { return ((size_t)TE + (TE + kCdfChunk - 1) / kCdfChunk + 3) / 4 * 4; }
+inline size_t ecdf_words(int32_t TE) { return scene_head(TE) + sizeof(SceneHead) / 4 + 8 * kCullBoxes; }
 
 SceneView view(const lisa_ctx* c) {
   // boxes that reach infinity leave closest_walk's margin infinite: such a
@@ -3548,7 +3554,8 @@ SceneView view(const lisa_ctx* c) {
                    make_float4(c->ecull_h[0], c->ecull_h[1], c->ecull_h[2], 0.0f),
                    (uint32_t)agg_capacity(c->all.T),
                    c->n_cull,
-                   c->n_cull > 0 ? reinterpret_cast<const float4*>(c->c_ecdf.p + cull_head(c->emit.T) + 4) : nullptr};
+                   c->n_cull > 0 ? reinterpret_cast<const float4*>(c->c_ecdf.p + scene_head(c->emit.T) + sizeof(SceneHead) / 4)
+                                 : nullptr};
 }
 
 // The path kernels' instance for the context's scene.
@@ -3926,13 +3933,13 @@ __global__ __launch_bounds__(256) void k_emit_chunks(const float4* __restrict__ 
 }
 // nee_scan's boxes over the emitters: the children of their Morton tree's root, the
 // largest inner box replaced by its own two children until there are kCullBoxes.
-// head[1] takes their count, or -1 where they do not have less than half of the root's
+// head->n_cull is their count, or -1 where they do not have less than half of the root's
 // area and one box does (a quad's two triangles have the quad's box each, a dense
 // field of emitters fills the boxes).  With 8 boxes nine lamps on the ceiling took
 // 4.8 ms and sixteen lights 7.5, against 2.7 and 3.3 with 16 and 3.6 and 7.9 with one;
 // shares of a quarter and a tenth leave scenes to one box that gain.  One work-item:
 // thirty node reads, the half of them in turn.
-__device__ void cull_boxes(const float4* __restrict__ nodes, float* head, float4* out) {
+__device__ void cull_boxes(const float4* __restrict__ nodes, SceneHead* head, float4* out) {
   __shared__ float lo[kCullBoxes][3], hi[kCullBoxes][3];
   __shared__ uint32_t ref[kCullBoxes];
   auto area = [](const float* l, const float* h) {
@@ -3977,13 +3984,17 @@ __device__ void cull_boxes(const float4* __restrict__ nodes, float* head, float4
     out[2 * k + 1] = make_float4(0.5f * (hi[k][0] - lo[k][0]) + far, 0.5f * (hi[k][1] - lo[k][1]) + far,
                                  0.5f * (hi[k][2] - lo[k][2]) + far, 0.0f);
   }
-  head[1] = __int_as_float(sum < 0.5f * whole ? m : -1);
+  head->n_cull = sum < 0.5f * whole ? m : -1;
 }
-// Workgroup 0: the chunks' bases; workgroup 1: the cull boxes.
-__global__ void k_emit_bases(float* chunk_tot, int32_t n_chunks, const float4* __restrict__ nodes, float* head,
-                             float4* cull) {
+// Workgroup 0: the chunks' bases; workgroup 1: the cull boxes and the root nodes.
+__global__ void k_emit_bases(float* chunk_tot, int32_t n_chunks, const float4* __restrict__ all,
+                             const float4* __restrict__ emit, SceneHead* head) {
   if (blockIdx.x == 1) {
-    cull_boxes(nodes, head, cull);
+    for (int k = 0; k < 4; ++k) {
+      head->root[k] = all[k];
+      head->root[4 + k] = emit[k];
+    }
+    cull_boxes(emit, head, reinterpret_cast<float4*>(head + 1));
     return;
   }
   float base = 0.0f;
@@ -3993,14 +4004,13 @@ __global__ void k_emit_bases(float* chunk_tot, int32_t n_chunks, const float4* _
     base = base + t;
   }
 }
-// head[0]: the emitters' area.
 __global__ __launch_bounds__(256) void k_emit_add(float* cdf, int32_t T, const float* __restrict__ base,
-                                                  float* head) {
+                                                  SceneHead* head) {
   const int32_t k = (int32_t)(blockIdx.x * 256 + threadIdx.x);
   if (k >= T) return;
   const float c = base[k / kCdfChunk] + cdf[k];
   cdf[k] = c;
-  if (k == T - 1) head[0] = c;
+  if (k == T - 1) head->area = c;
 }
 
 // Union of the child boxes of a root node (its 16 words).
@@ -4031,18 +4041,20 @@ lisa_status read_scene_box(lisa_ctx* ctx, bool may_alloc = true) {
   }
   ctx->n_cull = ctx->emit.T > 0 ? -1 : 0;
   if (T <= 0) return LISA_OK;
-  float rb[16];
-  HIP_TRY(ctx, hipMemcpy(rb, ctx->all.nodes, 64, hipMemcpyDeviceToHost));
-  root_box(rb, ctx->bmin, ctx->bmax);
-  float S = 0.0f;
-  for (int a = 0; a < 3; ++a) S = std::max(S, std::max(std::fabs(ctx->bmin[a]), std::fabs(ctx->bmax[a])));
-  ctx->span = S;
+  auto scene_box = [&](const float4* root) {
+    root_box(reinterpret_cast<const float*>(root), ctx->bmin, ctx->bmax);
+    float S = 0.0f;
+    for (int a = 0; a < 3; ++a) S = std::max(S, std::max(std::fabs(ctx->bmin[a]), std::fabs(ctx->bmax[a])));
+    ctx->span = S;
+    return S;
+  };
   ctx->emit_area = 0.0f;  // no light samples unless the emitters below have area
-  if (ctx->emit.T <= 0) return LISA_OK;
-  const float m2 = S * 0x1p-11f;
-  float lo[3], hi[3];
-  HIP_TRY(ctx, hipMemcpy(rb, ctx->emit.nodes, 64, hipMemcpyDeviceToHost));
-  root_box(rb, lo, hi);
+  SceneHead res;
+  if (ctx->emit.T <= 0) {
+    HIP_TRY(ctx, hipMemcpy(res.root, ctx->all.nodes, 64, hipMemcpyDeviceToHost));
+    scene_box(res.root);
+    return LISA_OK;
+  }
   // light sampling of LISA_CACHE_EMISSION: area prefix sums of the emitters
   const int32_t TE = ctx->emit.T, n_chunks = (TE + kCdfChunk - 1) / kCdfChunk;
   if (may_alloc)
@@ -4050,17 +4062,19 @@ lisa_status read_scene_box(lisa_ctx* ctx, bool may_alloc = true) {
   else if (ctx->c_ecdf.cap < ecdf_words(TE))  // sized by lisa_set_scene for these emitters
     return fail(ctx, LISA_ERR_ALLOC, "emitter prefix-sum buffer smaller than the scene's emitters");
   float* chunk_tot = ctx->c_ecdf.p + TE;
+  SceneHead* head = reinterpret_cast<SceneHead*>(ctx->c_ecdf.p + scene_head(TE));
   k_emit_chunks<<<grid_for(n_chunks, 256), 256, 0, ctx->stream>>>(ctx->emit.tris, TE, ctx->c_ecdf.p, chunk_tot);
-  float* head = ctx->c_ecdf.p + cull_head(TE);
-  k_emit_bases<<<2, 1, 0, ctx->stream>>>(chunk_tot, n_chunks, ctx->emit.nodes, head,
-                                         reinterpret_cast<float4*>(head + 4));
+  k_emit_bases<<<2, 1, 0, ctx->stream>>>(chunk_tot, n_chunks, ctx->all.nodes, ctx->emit.nodes, head);
   k_emit_add<<<grid_for(TE, 256), 256, 0, ctx->stream>>>(ctx->c_ecdf.p, TE, chunk_tot, head);
   HIP_TRY(ctx, hipGetLastError());
-  float res[2];
-  HIP_TRY(ctx, hipMemcpyAsync(res, head, sizeof(res), hipMemcpyDeviceToHost, ctx->stream));
+  // one copy back: the two root nodes in copies of their own were 24 us of an update
+  HIP_TRY(ctx, hipMemcpyAsync(&res, head, sizeof(res), hipMemcpyDeviceToHost, ctx->stream));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  ctx->emit_area = res[0];
-  std::memcpy(&ctx->n_cull, &res[1], 4);
+  const float m2 = scene_box(res.root) * 0x1p-11f;
+  float lo[3], hi[3];
+  root_box(reinterpret_cast<const float*>(res.root + 4), lo, hi);
+  ctx->emit_area = res.area;
+  ctx->n_cull = res.n_cull;
   for (int a = 0; a < 3; ++a) {
     ctx->ecull_c[a] = 0.5f * (lo[a] + hi[a]);
     ctx->ecull_h[a] = 0.5f * (hi[a] - lo[a]) + m2;
@@ -4474,8 +4488,11 @@ lisa_status lisa_render(lisa_ctx* ctx, const lisa_render_params* p, float* accum
     HIP_TRY(ctx, hipMemsetAsync(ctx->d_counters, 0, LISA_NCOUNTERS * sizeof(unsigned long long), st));
   HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
   if (!count) {
-    rc = ready_trees(ctx);
+    bool built = false;
+    rc = ready_trees(ctx, &built);
     if (rc != LISA_OK) return rc;
+    // the image's copy took 30 us longer behind this many launches than this wait does
+    if (built) HIP_TRY(ctx, hipStreamSynchronize(st));
   }
   const unsigned grid = a.tiles_x * tiles_y;
   if (p->flags & LISA_FLAG_WAVEFRONT) {
