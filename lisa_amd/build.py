@@ -63,10 +63,10 @@ def build(verbose_resources=False, defines=(), out_dir=OUT, cli=True):
 
 
 # Variant of the library with a 2-entry LDS traversal stack: every deeper
-# entry goes to the per-lane private overflow array, and a walk of the
-# agglomerated tree past 8 entries is left to the Morton tree, so a parity test
-# run against it exercises both paths (the default 20-entry stack never
-# overflows on the benchmark scenes).
+# entry of a Morton walk goes to the per-lane private overflow array, and the
+# paused walks of the agglomerated tree move blocks there at 8 entries instead
+# of 26, so a parity test run against it exercises both paths (the benchmark
+# scenes' Morton walks need at most 18 entries).
 SMALL_STACK = os.path.join(OUT, "stack2")
 
 

@@ -93,6 +93,9 @@ constexpr int kStackMax = 64;
 #define LISA_WALK_STACK LISA_STACK_LDS
 #endif
 constexpr int kWalkStack = LISA_WALK_STACK;
+// A walk of the path loop that fills them moves its oldest kWalkBlock entries to
+// private memory, up to kWalkBlocks times.
+constexpr int kWalkBlock = (kWalkStack - 2) / 2, kWalkBlocks = (kStackMax - kStackLds) / kWalkBlock;
 constexpr int kStackRows = kStackLds > kWalkStack ? kStackLds : kWalkStack;  // LDS words per lane of a walk
 // LDS words per lane of a path kernel: the traversal stack, then the pixel's
 // running sum of sample radiance (3 floats, touched once per sample) and the
@@ -110,7 +113,7 @@ constexpr int kTileW = kPathBlock >= 128 ? 16 : 8;
 constexpr int kTileH = kPathBlock / kTileW;
 constexpr int kRayBlock = 256;
 static_assert(kStackLds >= 1 && kStackLds <= kStackMax, "LDS stack depth");
-static_assert(kWalkStack >= 4, "walk stack depth");
+static_assert(kWalkStack >= 8, "walk stack depth: a full stack is a block, an entry and a paused walk");
 static_assert(kPathBlock == 64 || kPathBlock == 128 || kPathBlock == 256, "path block size");
 
 struct DevMat {
@@ -696,11 +699,17 @@ __device__ __forceinline__ int32_t closest_morton(const SceneView& sc, bool emit
 // the compiler from threading the jumps of lanes that hold an inner node after
 // an inner node, or a triangle after a triangle, into loops of their own, where
 // the rest of the wave would wait for them (C2 at 32 spp 45.9 ms against
-// 37.3).  The stack is LDS only and ends
-// in a sentinel; a walk that would pass kWalkStack entries leaves the query to
-// closest() over the Morton tree (the tree's depth is not bounded by its
-// construction; 20 entries are passed by 1e-5 of a batch scene's walks, 28 by
-// none seen), as does a scene without a walk tree.
+// 37.3).  The stack is LDS only and ends in a sentinel.  A walk that would pass
+// kWalkStack entries (the tree's depth is not bounded by its construction: 3e-5 of
+// a batch scene's walks) is paused with its oldest entries moved to private memory,
+// and goes on in the next round, as it does when they are wanted again.  Started over
+// in the Morton tree, a few rays that did so in each sample held up the whole
+// image: batch scene of 560k triangles, 1920x1080, 8 spp, one bounce 6.4 -> 3.6 ms (the
+// binary walk 5.6); a shuffled Cornell box of 65k triangles whose codes a quad at
+// distance 10^4 puts into one cell, 128^2, 1 spp, 111 -> 7 (76).  The move stands behind the
+// loop: in it, it cost every walk (C2 2.5 %).  Walks that do not pause, and a stack that
+// is full all the same, leave the query to closest() over the Morton tree, as does a
+// scene without a walk tree.
 //
 // Bound by VALU issue: min, max, compare, select and shift take 4.2 to 5 cycles
 // of a SIMD, fma, add and moves 2.4 to 2.9 (two waves' overlap), and k_path on C2
@@ -756,7 +765,7 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
     const char* __restrict__ base = bv.walk;
     float best_t = tlim, cull_t = tlim * kWiden;
     uint32_t best_prim = lim_prim, cur = emitters ? sc.emit_root : 0u;
-    int sp = 1;
+    int sp = 2;
     int quorum = 0;
     if (kPause && paused) {
       sp = paused;
@@ -767,7 +776,8 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
       cull_t = best_t * kWiden;
       paused = 0;
     } else {
-      stk[0] = kEmpty;  // popped last: the end of the walk
+      stk[0] = 0;             // blocks in private memory
+      stk[kStride] = kEmpty;  // popped last: the end of the walk, or of what is in LDS
     }
     if (kPause) quorum = __popcll(__ballot(1)) / 2;
     done = true;
@@ -829,6 +839,7 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
         if (!(key[0] < INFINITY)) cur = stk[--sp * kStride];
         if (sp > kWalkStack - 4) {  // room for a node's entries or a paused walk
           done = false;
+          stk[sp * kStride] = cur;
           cur = kEmpty;
         }
       }
@@ -851,6 +862,8 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
         }
       }
     }
+    const bool full = !done;
+    const int n = kPause ? (int)stk[0] : 0;
     t_out = best_t;
     // closest() tests a triangle only when slab() passes its leaf box, and the
     // wider test above may let one more through: a hit whose rounded t is past
@@ -867,6 +880,26 @@ __device__ __forceinline__ int32_t closest_walk(const SceneView& sc, bool emitte
       b[4] = float_up(fmaxf(fmaxf(a.y, c.y), e.y));
       b[5] = float_up(fmaxf(fmaxf(a.z, c.z), e.z));
       done = done && slab(b[0], b[1], b[2], b[3], b[4], b[5], r, tmin, tlim * kWiden, tn);
+    }
+    if (kPause) {
+      // the oldest entries to private memory, or back (stk[0]: blocks there); the count is
+      // read before the box test above, whose loads cover it
+      if (full ? n < kWalkBlocks : n > 0 && !(any && best_k >= 0)) {
+        if (!full) {
+          for (int i = 0; i < kWalkBlock; ++i) stk[(2 + i) * kStride] = spill[(n - 1) * kWalkBlock + i];
+          sp = kWalkBlock + 1;
+        } else {
+          for (int i = 0; i < kWalkBlock; ++i) spill[n * kWalkBlock + i] = stk[(2 + i) * kStride];
+          sp -= kWalkBlock;
+          for (int i = 2; i <= sp; ++i) stk[i * kStride] = stk[(i + kWalkBlock) * kStride];
+        }
+        stk[0] = (uint32_t)(full ? n + 1 : n - 1);
+        stk[(sp + 1) * kStride] = __float_as_uint(best_t);
+        stk[(sp + 2) * kStride] = best_prim;
+        stk[(sp + 3) * kStride] = (uint32_t)best_k;
+        paused = sp;
+        return -1;
+      }
     }
   }
   if (!done)
