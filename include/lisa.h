@@ -182,8 +182,8 @@ lisa_status lisa_get_stats(const lisa_ctx* ctx, lisa_stats* out);
  * 2^20) also get the 4-wide form of their Morton tree (128 bytes per inner
  * node: each node's children, inner children replaced by their own two), and
  * lisa_trace_rays takes its hits from a 4-wide walk: of the agglomerated tree
- * that the path kernels walk, or of that form in a scene without one (an
- * infinite coordinate; more than 2^25 nodes over the scene and its emitters,
+ * that the path kernels walk, or of that form in a scene without one (a
+ * coordinate of 10^37 or more; more than 2^25 nodes over the scene and its emitters,
  * which is about 31 million triangles, or half of that if all emit): fewer,
  * wider visits, which pay where the tree streams from HBM.  The hits are the same
  * (closest hit, equal t to the lower triangle id); node-visit counters
