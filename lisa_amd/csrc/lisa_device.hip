@@ -3593,8 +3593,9 @@ constexpr int32_t kCdfChunk = 64;  // emitters per chunk of the area prefix sums
 // scene_head() on what read_scene_box() reads back, and the cull boxes.
 struct SceneHead {
   float area;       // of the emitters (k_emit_add)
-  int32_t n_cull;   // their cull boxes, below 0: none (k_emit_bases)
-  int32_t pad[2];
+  int32_t n_cull;   // their cull boxes (cull_boxes)
+  int32_t loose;    // whether these do better than one
+  int32_t pad;
   float4 mid;       // walk_mid
   float4 root[8];   // the root nodes of the scene's and the emitters' Morton trees
 };
@@ -3994,10 +3995,10 @@ __global__ __launch_bounds__(256) void k_emit_chunks(const float4* __restrict__ 
   chunk_tot[c] = acc;
 }
 // nee_scan's boxes over the emitters: the children of their Morton tree's root, the
-// largest inner box replaced by its own two children until there are kCullBoxes.
-// head->n_cull is their count, or -1 where they do not have less than half of the root's
-// area and one box does (a quad's two triangles have the quad's box each, a dense
-// field of emitters fills the boxes).  With 8 boxes nine lamps on the ceiling took
+// largest inner box replaced by its own two children until there are kCullBoxes; a box
+// whose children are both nearly as large (a quad's two triangles) stays.
+// head->loose: the boxes have less than half of the root's area, and do better than one
+// box (a dense field of emitters fills them).  With 8 boxes nine lamps on the ceiling took
 // 4.8 ms and sixteen lights 7.5, against 2.7 and 3.3 with 16 and 3.6 and 7.9 with one;
 // shares of a quarter and a tenth leave scenes to one box that gain.  One work-item:
 // thirty node reads, the half of them in turn.
@@ -4031,8 +4032,15 @@ __device__ void cull_boxes(const float4* __restrict__ nodes, F3 mid, SceneHead* 
     }
     if (open < 0) break;
     const float4* np = nodes + 4 * (size_t)ref[open];
-    ref[open] = node_child(np, 0, lo[open], hi[open]);
-    ref[m] = node_child(np, 1, lo[m], hi[m]);
+    float l0[3], h0[3];
+    const uint32_t r0 = node_child(np, 0, l0, h0), r1 = node_child(np, 1, l, h);
+    if (area(l0, h0) >= 0.9f * most && area(l, h) >= 0.9f * most) {
+      ref[open] = kLeaf;  // as one
+      continue;
+    }
+    ref[open] = r0;
+    ref[m] = r1;
+    for (int a = 0; a < 3; ++a) lo[open][a] = l0[a], hi[open][a] = h0[a], lo[m][a] = l[a], hi[m][a] = h[a];
     ++m;
   }
   float sum = 0.0f;
@@ -4051,7 +4059,8 @@ __device__ void cull_boxes(const float4* __restrict__ nodes, F3 mid, SceneHead* 
     out[2 * k + 1] = make_float4(0.5f * (hi[k][0] - lo[k][0]) + far, 0.5f * (hi[k][1] - lo[k][1]) + far,
                                  0.5f * (hi[k][2] - lo[k][2]) + far, 0.0f);
   }
-  head->n_cull = sum < 0.5f * whole ? m : -1;
+  head->n_cull = m;
+  head->loose = sum < 0.5f * whole ? 1 : 0;
 }
 // Workgroup 0: the chunks' bases; workgroup 1: the cull boxes and the root nodes.
 __global__ void k_emit_bases(float* chunk_tot, int32_t n_chunks, const float4* __restrict__ all,
@@ -4148,7 +4157,12 @@ lisa_status read_scene_box(lisa_ctx* ctx, bool may_alloc = true) {
   float lo[3], hi[3];
   root_box(reinterpret_cast<const float*>(res.root + 4), lo, hi);
   ctx->emit_area = res.area;
-  ctx->n_cull = res.n_cull;
+  // The boxes, with their own margins, also where the one box is mostly margin (a small
+  // lamp in a large scene: Cornell box of a hundredth of the scene's size, 512^2, 4 spp,
+  // @L -> @M ms).
+  float half = 0.0f;
+  for (int a = 0; a < 3; ++a) half = std::max(half, 0.5f * (hi[a] - lo[a]));
+  ctx->n_cull = res.loose || Sm * 0x1p-11f > 0.25f * half ? res.n_cull : -1;
   for (int a = 0; a < 3; ++a) {
     ctx->ecull_c[a] = 0.5f * (lo[a] + hi[a]);
     ctx->ecull_h[a] = 0.5f * (hi[a] - lo[a]) + S * 0x1p-11f;
