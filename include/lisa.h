@@ -183,9 +183,10 @@ lisa_status lisa_get_stats(const lisa_ctx* ctx, lisa_stats* out);
  * node: each node's children, inner children replaced by their own two), and
  * lisa_trace_rays takes its hits from a 4-wide walk: of the agglomerated tree
  * that the path kernels walk, or of that form in a scene without one (a
- * coordinate of 10^37 or more; more than 2^25 nodes over the scene and its emitters,
- * which is about 31 million triangles, or half of that if all emit): fewer,
- * wider visits, which pay where the tree streams from HBM.  The hits are the same
+ * coordinate of 10^37 or more; more than 2^25 nodes over the scene and its
+ * emitters, which is about 31 million triangles, or half of that if all emit;
+ * no memory for it), where the path kernels walk it too: fewer, wider visits,
+ * which pay where the tree streams from HBM.  The hits are the same
  * (closest hit, equal t to the lower triangle id); node-visit counters
  * (LISA_FLAG_COUNT) stay those of the binary tree.  0 gives every scene the
  * wide form.  No counterpart in the reference (OptiX chooses its acceleration

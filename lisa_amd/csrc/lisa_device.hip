@@ -293,18 +293,19 @@ __device__ __forceinline__ bool try_culled_by(const float4* __restrict__ box, in
   const float ax = fabsf(x), ay = fabsf(y), az = fabsf(z);
   const float m = fmaxf(fmaxf(fabsf(O.x), fabsf(O.y)), fabsf(O.z)) * kCullMargin;
   const float mx = m * (ay + az), my = m * (az + ax), mz = m * (ax + ay);
-  // the constant address space: scalar loads where the lanes' scene is one
-  using ConstBox = const __attribute__((address_space(4))) float;
-  ConstBox* f = (ConstBox*)(uintptr_t)box;
+  // the constant address space: a scalar load per box where the lanes' scene is one
+  using Box = float __attribute__((ext_vector_type(8)));
+  const __attribute__((address_space(4))) Box* f = (const __attribute__((address_space(4))) Box*)(uintptr_t)box;
   bool hit = false;
-  for (int32_t k = 0; k < n; ++k, f += 8) {
-    const F3 c = mk(f[0], f[1], f[2]), H = mk(f[4], f[5], f[6]);
-    const float wx = c.x - O.x, wy = c.y - O.y, wz = c.z - O.z;
+#pragma unroll 2
+  for (int32_t k = 0; k < n; ++k) {
+    const Box b = f[k];
+    const float wx = b[0] - O.x, wy = b[1] - O.y, wz = b[2] - O.z;
     const float px = __builtin_fmaf(wy, z, -(wz * y)), py = __builtin_fmaf(wz, x, -(wx * z)),
                 pz = __builtin_fmaf(wx, y, -(wy * x));
-    const float qx = __builtin_fmaf(H.y, az, __builtin_fmaf(H.z, ay, mx)),
-                qy = __builtin_fmaf(H.z, ax, __builtin_fmaf(H.x, az, my)),
-                qz = __builtin_fmaf(H.x, ay, __builtin_fmaf(H.y, ax, mz));
+    const float qx = __builtin_fmaf(b[5], az, __builtin_fmaf(b[6], ay, mx)),
+                qy = __builtin_fmaf(b[6], ax, __builtin_fmaf(b[4], az, my)),
+                qz = __builtin_fmaf(b[4], ay, __builtin_fmaf(b[5], ax, mz));
     hit |= !((fabsf(px) > qx) | (fabsf(py) > qy) | (fabsf(pz) > qz));
   }
   return !hit;
@@ -351,8 +352,8 @@ static_assert(kNeeTries <= 31, "a half wave makes a vertex's tries at once");
 // against up to kCullBoxes boxes from the top of the emitters' tree too, and with no
 // emitter against none at all.  Cornell box of 65k triangles,
 // 512^2, 4 spp (the binary walk with the query in the loop of the tries / one box /
-// these): no light 3.6 / 5.3 / 1.2 ms, lights in two corners 5.4 / 10.0 / 1.5, six
-// lights 8.1 / 9.3 / 2.5, eight 8.6 / 8.9 / 3.3, 128 17.8 / 11.6 / 11.9 (one box).
+// these): no light 3.6 / 5.3 / 1.3 ms, lights in two corners 5.4 / 10.0 / 1.4, six
+// lights 8.1 / 9.3 / 2.1, eight 8.6 / 8.9 / 2.4, 128 17.8 / 11.6 / 11.6 (one box).
 constexpr int kNeeDense = 16;  // 8 and 32 measured the same
 constexpr int kNeeSerial = 30;  // 16 measured 5 % slower on C2; 64 (never in turn) the same
 template <bool shared, bool kBoxes>
@@ -3533,7 +3534,7 @@ struct lisa_batch {
   std::vector<size_t> accum_px;
   std::vector<uint64_t> gens;  // each context's generation when the batch was made
   uint32_t total = 0;
-  int kind = kPlain;  // the kernels' instance: the most general that a scene asks for
+  int kind = kPlain;  // the kernels' instance (lisa_batch_create)
   hipStream_t stream = nullptr;
   BatchScene* d_scenes = nullptr;
   uint32_t* d_counter = nullptr;
@@ -3994,73 +3995,95 @@ __global__ __launch_bounds__(256) void k_emit_chunks(const float4* __restrict__ 
   }
   chunk_tot[c] = acc;
 }
-// nee_scan's boxes over the emitters: the children of their Morton tree's root, the
-// largest inner box replaced by its own two children until there are kCullBoxes; a box
-// whose children are both nearly as large (a quad's two triangles) stays.
-// head->loose: the boxes have less than half of the root's area, and do better than one
-// box (a dense field of emitters fills them).  With 8 boxes nine lamps on the ceiling took
-// 4.8 ms and sixteen lights 7.5, against 2.7 and 3.3 with 16 and 3.6 and 7.9 with one;
-// shares of a quarter and a tenth leave scenes to one box that gain.  One work-item:
-// thirty node reads, the half of them in turn.
+// nee_scan's boxes over the emitters, from the top of their Morton tree: its largest
+// inner box is opened until there are kCullBoxes, a box whose children are leaves nearly
+// as large (a quad's two triangles) stays; then a box is taken whole again where its
+// parts do not save kBoxWorth of the root's area for each test that they add (the pieces
+// of a lit sphere: a line that passes its box mostly meets one).  head->loose: tests and
+// areas together are below kLooseShare of the root's area; the kernels with the boxes
+// then gain or are as fast.  Cornell box of 65k triangles, 512^2, 4 spp, one box / boxes:
+// 6 lights 9.4 / 2.1 ms, 12 9.3 / 2.6, 16 7.9 / 3.0, 24 9.8 / 6.7; with 8 boxes nine lamps on
+// the ceiling took 4.8 and sixteen lights 7.5 (16: 2.5 and 3.0).  At shares of a half and of
+// 0.8 batch scenes with a large sun and one lit sphere lose a quarter (22.5 -> 28 ms,
+// 38 -> 52), at 0.8 others gain as much (21 -> 17.6, three lamps in a row 2.0 -> 1.6).  One
+// work-item: thirty node reads, the half of them in turn.
+constexpr float kBoxWorth = 1.0f / 256.0f, kLooseShare = 0.3f;
 __device__ void cull_boxes(const float4* __restrict__ nodes, F3 mid, SceneHead* head, float4* out) {
-  __shared__ float lo[kCullBoxes][3], hi[kCullBoxes][3];
-  __shared__ uint32_t ref[kCullBoxes];
-  auto area = [](const float* l, const float* h) {
+  constexpr int kMax = 2 * kCullBoxes - 1;
+  __shared__ float lo[kMax][3], hi[kMax][3], area[kMax], cost[kMax];
+  __shared__ uint32_t ref[kMax];
+  __shared__ int kid[kMax];  // the first of two, 0: none
+  auto put = [&](int k, uint32_t r, const float* l, const float* h) {
+    ref[k] = r;
+    kid[k] = 0;
+    for (int a = 0; a < 3; ++a) lo[k][a] = l[a], hi[k][a] = h[a];
     const float dx = h[0] - l[0], dy = h[1] - l[1], dz = h[2] - l[2];
-    return dx * dy + dy * dz + dz * dx;
+    area[k] = dx * dy + dy * dz + dz * dx;
   };
-  int m = 0;
-  for (int ch = 0; ch < 2; ++ch) {
-    ref[m] = node_child(nodes, ch, lo[m], hi[m]);
-    if (ref[m] != kEmpty) ++m;
+  float l0[3], h0[3], l1[3], h1[3];
+  // the root: node 0, or the only leaf
+  uint32_t r0 = node_child(nodes, 0, l0, h0), r1 = node_child(nodes, 1, l1, h1);
+  if (r1 == kEmpty) {
+    put(0, kLeaf, l0, h0);
+  } else {
+    float l[3], h[3];
+    for (int a = 0; a < 3; ++a) l[a] = fminf(l0[a], l1[a]), h[a] = fmaxf(h0[a], h1[a]);
+    put(0, 0u, l, h);
   }
-  float l[3], h[3];
-  for (int a = 0; a < 3; ++a) {
-    l[a] = m == 2 ? fminf(lo[0][a], lo[1][a]) : lo[0][a];
-    h[a] = m == 2 ? fmaxf(hi[0][a], hi[1][a]) : hi[0][a];
-  }
-  const float whole = area(l, h);
-  while (m < kCullBoxes) {
+  int m = 1;
+  while (m + 2 <= kMax) {
     int open = -1;
-    float most = -1.0f;
-    for (int k = 0; k < m; ++k) {
-      const float s = area(lo[k], hi[k]);
-      if (!(ref[k] & kLeaf) && (open < 0 || s > most)) {
-        open = k;
-        most = s;
-      }
-    }
+    for (int k = 0; k < m; ++k)
+      if (!kid[k] && !(ref[k] & kLeaf) && (open < 0 || area[k] > area[open])) open = k;
     if (open < 0) break;
     const float4* np = nodes + 4 * (size_t)ref[open];
-    float l0[3], h0[3];
-    const uint32_t r0 = node_child(np, 0, l0, h0), r1 = node_child(np, 1, l, h);
-    if (area(l0, h0) >= 0.9f * most && area(l, h) >= 0.9f * most) {
-      ref[open] = kLeaf;  // as one
+    r0 = node_child(np, 0, l0, h0);
+    r1 = node_child(np, 1, l1, h1);
+    put(m, r0, l0, h0);
+    put(m + 1, r1, l1, h1);
+    if ((r0 & r1 & kLeaf) && area[m] >= 0.9f * area[open] && area[m + 1] >= 0.9f * area[open]) {
+      ref[open] = kLeaf;
       continue;
     }
-    ref[open] = r0;
-    ref[m] = r1;
-    for (int a = 0; a < 3; ++a) lo[open][a] = l0[a], hi[open][a] = h0[a], lo[m][a] = l[a], hi[m][a] = h[a];
-    ++m;
+    kid[open] = m;
+    m += 2;
   }
-  float sum = 0.0f;
+  const float whole = area[0];
+  for (int k = m - 1; k >= 0; --k) {  // children come after their parent
+    const float own = kBoxWorth * whole + area[k];
+    cost[k] = own;
+    if (kid[k]) {
+      const float parts = cost[kid[k]] + cost[kid[k] + 1];
+      if (parts < own)
+        cost[k] = parts;
+      else
+        kid[k] = 0;
+    }
+  }
+  int n = 0;
+  for (int k = 0; k < m; ++k) area[k] = k == 0 ? 1.0f : 0.0f;  // from here on: whether the box is reached
   for (int k = 0; k < m; ++k) {
-    sum += area(lo[k], hi[k]);
+    if (area[k] == 0.0f) continue;
+    if (kid[k]) {
+      area[kid[k]] = area[kid[k] + 1] = 1.0f;
+      continue;
+    }
     const float c[3] = {mid.x, mid.y, mid.z};
+    float far = 0.0f;
     for (int a = 0; a < 3; ++a) {
       lo[k][a] -= c[a];
       hi[k][a] -= c[a];
+      far = fmaxf(far, fmaxf(fabsf(lo[k][a]), fabsf(hi[k][a])));
     }
-    float far = 0.0f;
-    for (int a = 0; a < 3; ++a) far = fmaxf(far, fmaxf(fabsf(lo[k][a]), fabsf(hi[k][a])));
     far *= kCullMargin;
-    out[2 * k] = make_float4(0.5f * (lo[k][0] + hi[k][0]), 0.5f * (lo[k][1] + hi[k][1]),
+    out[2 * n] = make_float4(0.5f * (lo[k][0] + hi[k][0]), 0.5f * (lo[k][1] + hi[k][1]),
                              0.5f * (lo[k][2] + hi[k][2]), 0.0f);
-    out[2 * k + 1] = make_float4(0.5f * (hi[k][0] - lo[k][0]) + far, 0.5f * (hi[k][1] - lo[k][1]) + far,
+    out[2 * n + 1] = make_float4(0.5f * (hi[k][0] - lo[k][0]) + far, 0.5f * (hi[k][1] - lo[k][1]) + far,
                                  0.5f * (hi[k][2] - lo[k][2]) + far, 0.0f);
+    ++n;
   }
-  head->n_cull = m;
-  head->loose = sum < 0.5f * whole ? 1 : 0;
+  head->n_cull = n;
+  head->loose = cost[0] < kLooseShare * whole ? 1 : 0;
 }
 // Workgroup 0: the chunks' bases; workgroup 1: the cull boxes and the root nodes.
 __global__ void k_emit_bases(float* chunk_tot, int32_t n_chunks, const float4* __restrict__ all,
@@ -4943,7 +4966,14 @@ lisa_status lisa_batch_create(lisa_batch** out, lisa_ctx* const* ctxs,
   }
   b->device = dev;
   b->total = (uint32_t)total;
-  for (int32_t i = 0; i < n; ++i) b->kind = std::max(b->kind, scene_kind(ctxs[i]));
+  // one scene without a walk tree takes all to the Morton trees; the emitters' boxes, whose
+  // test the lanes of the queue form make each for themselves, only pay where most of
+  // the samples are from scenes that have them (64 batch scenes, one with: 1215 ms
+  // without, 1420 with)
+  double samples[3] = {};
+  for (int32_t i = 0; i < n; ++i)
+    samples[scene_kind(ctxs[i])] += (double)params[i].width * params[i].height * params[i].spp;
+  b->kind = samples[kMorton] > 0 ? kMorton : (samples[kLoose] > samples[kPlain] ? kLoose : kPlain);
   b->stream = ctxs[0]->stream;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, dev) == hipSuccess) b->cus = prop.multiProcessorCount;

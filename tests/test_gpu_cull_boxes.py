@@ -31,6 +31,10 @@ def _lights(name):
         q = [_quad(rs.uniform(-0.45, 0.45, 3), 0.02, k % 3) for k in range(5)]
         q[2][0, 4] = np.nan
         return q
+    if name == "sun and sphere":  # a batch scene's: the one box serves better, or a box each
+        from lisa_amd import scenes
+        return [_quad((0.0, 0.49, 0.0), 0.3, 1),
+                scenes.displaced_icosphere(2)["verts"].reshape(-1, 9) * np.float32(0.1) + np.float32([0.2, -0.2, 0.1] * 3)]
     if name == "none":
         return []
     return [_quad(rs.uniform(-0.45, 0.45, 3), 0.02, int(rs.integers(3))) for _ in range(int(name))]
@@ -52,7 +56,7 @@ def _same(a, b):
 
 
 # 4, 8 and 9 lights: as many triangles as kCullBoxes and half of it, and one pair more
-@pytest.mark.parametrize("name", ["corners", "touching", "lamps", "far", "slivers", "nan", "none",
+@pytest.mark.parametrize("name", ["corners", "touching", "lamps", "far", "slivers", "nan", "none", "sun and sphere",
                                   "1", "2", "4", "8", "9", "40"])
 def test_image_of_the_counting_build(capi, name):
     sc = _scene(name)
