@@ -31,8 +31,9 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Mrays/s; time to RMSE≤1e-2 vs 16k-spp ref, cache vs plain, 1 MI355X"
 HBM_PEAK_GBS = 8000.0
-# one 64-lane VALU instruction per SIMD every 4 cycles: 1,024 SIMDs at 2.4 GHz
-VALU_PEAK_TINST = round(256 * 4 * 16 * 2.4e-3, 2)
+# the vector rate: 32 lanes per SIMD and cycle, 1,024 SIMDs at 2.4 GHz (157 TFLOP/s
+# of FP32 multiply-adds)
+VALU_PEAK_TINST = round(256 * 4 * 32 * 2.4e-3, 2)
 # Algorithmic bytes: one 64-byte node line per BVH node visit, one 48-byte
 # triangle record per triangle test, 96 bytes (vertices + normals) per
 # shaded radiance hit, one float4 accum store per pixel.
@@ -134,10 +135,10 @@ def bench_plain(a, workload, steps, warmup, cpu=True):
     and, with `cpu`, the CPU oracle on a seeded pixel subset.  Returns the
     result dict.
 
-    The tiled megakernel is bound by VALU issue, so that is its roofline:
-    lane-instructions per second against 64 per SIMD every 4 cycles (the rate
-    of min, max, compare and select; fma, add and moves of two waves can
-    overlap).  Bytes of the counted walk would not do: the counting build walks the Morton
+    The tiled megakernel is nearest to the vector rate, so that is its roofline:
+    active lane-instructions per second against 32 lanes per SIMD and cycle.  (Chains
+    of one instruction reach 2.4 to 2.9 cycles a wave for fma, add, mul and moves, 4.2 to 5
+    for min, max, compare and select.)  Bytes of the counted walk would not do: the counting build walks the Morton
     tree, which the oracle reproduces, and the timed build the agglomerated
     one, which visits a fraction of its nodes.  The wavefront form does walk
     the Morton tree and keeps the byte roofline."""
@@ -196,9 +197,9 @@ def bench_plain(a, workload, steps, warmup, cpu=True):
                     "frac": None if achieved is None else round(achieved / VALU_PEAK_TINST, 4),
                     # fraction of a wave's 64 lanes active per VALU instruction
                     "lane_utilization": rec.get("valu_lane_utilization"),
-                    "limiter": "VALU issue under divergence: the lanes of a wave end their "
-                               "walks and their stages at different points",
-                    "kernel": "k_path_pq<0>" if a.persistent else "k_path<false,false,false>"}
+                    "limiter": "divergence (the lanes of a wave end their walks and their stages "
+                               "at different points), then VALU issue and the texture data path",
+                    "kernel": "k_path_pq<0>" if a.persistent else "k_path<false,false,false,0>"}
     roofline.update(traffic=traffic,
                     dram_frac=(None if traffic is None else
                                round(traffic / seconds / 1e9 / HBM_PEAK_GBS, 4)),
