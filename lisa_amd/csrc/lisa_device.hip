@@ -8,11 +8,14 @@
 //                           (child boxes live in the parent; ref bit 31 = leaf,
 //                           low bits = sorted triangle / node index)
 //   wide   float4[8 * nI]   scenes of >= 2^20 triangles: the 4-wide form (k_wide),
-//                           one 128-byte line per internal node (lisa_trace_rays)
+//                           one 128-byte line per internal node, filled when a walk
+//                           first needs it (scenes without a walk tree)
 //   walk   float4[8 * cap]  the agglomerated 4-wide tree that the path kernels walk
-//                           (k_agg, k_walk_nodes), cap ~ 1.07 T
+//                           (k_agg, k_walk_nodes), cap ~ 1.07 T; its planes are
+//                           relative to walk_mid
 //   tris   float4[3 * T]    48 bytes per triangle in Morton order:
-//                           v0.xyz|prim id, v1.xyz|material id, v2.xyz|0
+//                           v0.xyz|prim id, v1.xyz|material id, v2.xyz|0 (emitters:
+//                           the triangle's place among all of the scene's)
 //   nrm    float4[3 * T]    vertex normals in the same order (shading gather)
 //   mats   DevMat[M]        48 bytes per material
 //   accum  float4[w * h]    OptixParams::accum_buffer (structs.hh:62)
@@ -727,9 +730,10 @@ __device__ __forceinline__ int32_t closest_morton(const SceneView& sc, bool emit
 // is full all the same, leave the query to closest() over the Morton tree, as does a
 // scene without a walk tree.
 //
-// Bound by VALU issue: min, max, compare, select and shift take 4.2 to 5 cycles
-// of a SIMD, fma, add and moves 2.4 to 2.9 (two waves' overlap), and k_path on C2
-// fills 103 % of the slots at 4 cycles, with 51 % of the lanes active.  Five loads
+// Bound by divergence and by two units: 50 % of the lanes are active on C2, a SIMD
+// issues one VALU instruction every 3.9 cycles (in chains of one kind, min, max,
+// compare, select and shift take 4.2 to 5, fma, add and moves 2.4 to 2.9), and the
+// texture data path is busy 91 % of the cycles.  Five loads
 // per node instead of seven (planes as 16-bit floats around the node's centre,
 // 18 VALU instructions more) took 24.4 ms against 22.2 (C2 at 32 spp) and 28.7
 // against 28.6 (icosphere of 1.3M triangles, 1080p, 16 spp); sorting only the

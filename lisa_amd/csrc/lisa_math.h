@@ -153,7 +153,7 @@ struct Lambertian {
   }
   // eval * pdf weight: NdotL * (float)((double)NdotL / M_PI).  The product with
   // the rounded reciprocal rounds to the same float for every 24-bit
-  // significand (checked for all of them) at a tenth of the division's cost.
+  // significand (the tests check all of them) at a tenth of the division's cost.
   __device__ static __forceinline__ float eval(F3 N, F3 L) {
     const float NdotL = clampf(dot(N, L), 0.0f, 1.0f);
     const float p = (float)((double)NdotL * (1.0 / 3.14159265358979323846));
